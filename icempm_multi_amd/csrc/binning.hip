@@ -13,6 +13,7 @@
 // Built with -ffp-contract=off so that x*hinv+0.5 is rounded twice, as on the host.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "kernels.h"
@@ -165,12 +166,13 @@ __global__ void __launch_bounds__(kBlock) k_gather(StepArgs a, BinWork w, const 
     sorted_keys[j] = (col - S.c.halo + S.c.xoff) * S.c.gridY + row;
 }
 
-// Points per tile (TX x TY cells) from cell_start; one thread per tile.
-__global__ void __launch_bounds__(kBlock) k_tile_count(StepArgs a, const int *tile_off, int n_tiles_all, int *tile_n,
-                                                       int *tile_flag)
+// Tile builder: half a wave per tile, a lane per column (tx <= 32).
+constexpr int kTileLanes = 32;
+
+// Place of tile t of the table: its scene and first cell.
+__device__ __forceinline__ const SceneDev &tile_place(const StepArgs &a, const int *tile_off, int t, int &scene,
+                                                      int &col0, int &row0)
 {
-    const int t = blockIdx.x * kBlock + threadIdx.x;
-    if (t >= n_tiles_all) return;
     int lo = 0, hi = a.nscenes - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
@@ -179,69 +181,167 @@ __global__ void __launch_bounds__(kBlock) k_tile_count(StepArgs a, const int *ti
     }
     const SceneDev &S = a.scenes[lo];
     const int local = t - tile_off[lo];
-    const int txi = local / S.n_tiles_y, tyi = local % S.n_tiles_y;
-    const int col0 = txi * a.tx, row0 = tyi * a.ty;
-    int n = 0;
-    for (int c = 0; c < a.tx; c++) {
-        const int col = col0 + c;
-        if (col >= S.c.ncols) break;
-        const long long base = S.cell_off + (long long)col * S.c.gridY;
-        n += a.cell_start[base + min(row0 + a.ty, S.c.gridY)] - a.cell_start[base + row0];
-    }
-    tile_n[t] = n;
-    tile_flag[t] = n > 0 ? 1 : 0;
+    scene = lo;
+    col0 = (local / S.n_tiles_y) * a.tx;
+    row0 = (local % S.n_tiles_y) * a.ty;
+    return S;
 }
 
-__global__ void __launch_bounds__(kBlock) k_tile_emit(StepArgs a, const int *tile_off, int n_tiles_all,
-                                                      const int *tile_n, const int *tile_pos, TileItem *tiles,
-                                                      int *n_tiles)
+__device__ __forceinline__ int half_wave_min(int v)
 {
-    const int t = blockIdx.x * kBlock + threadIdx.x;
-    if (t == n_tiles_all - 1) *n_tiles = tile_pos[t] + (tile_n[t] > 0 ? 1 : 0);
-    if (t >= n_tiles_all || tile_n[t] == 0) return;
-    int lo = 0, hi = a.nscenes - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (tile_off[mid] <= t) lo = mid;
-        else hi = mid - 1;
+#pragma unroll
+    for (int k = kTileLanes / 2; k > 0; k >>= 1) v = min(v, __shfl_xor(v, k, kTileLanes));
+    return v;
+}
+
+// 1 per tile that holds points.
+__global__ void __launch_bounds__(kBlock) k_tile_count(StepArgs a, const int *tile_off, int n_tiles_all,
+                                                       int *tile_flag)
+{
+    const int t = (blockIdx.x * kBlock + threadIdx.x) / kTileLanes, k = threadIdx.x & (kTileLanes - 1);
+    if (t >= n_tiles_all) return;
+    int sc, col0, row0;
+    const SceneDev &S = tile_place(a, tile_off, t, sc, col0, row0);
+    int empty = 1;
+    if (k < a.tx && col0 + k < S.c.ncols) {
+        const int *cs = a.cell_start + S.cell_off + (long long)(col0 + k) * S.c.gridY;
+        empty = cs[min(row0 + a.ty, S.c.gridY)] == cs[row0];
     }
-    const SceneDev &S = a.scenes[lo];
-    const int local = t - tile_off[lo];
-    const int col0 = (local / S.n_tiles_y) * a.tx, row0 = (local % S.n_tiles_y) * a.ty;
+    empty = half_wave_min(empty);
+    if (k == 0) tile_flag[t] = !empty;
+}
+
+// The box of a tile's cells that hold points, and the runs of the box's
+// columns.  Each lane bisects its column: cell_start is nondecreasing, so the
+// first and last occupied rows are found in log2(ty) steps (one thread per
+// tile, column after column, took 12 us for any scene).
+__global__ void __launch_bounds__(kBlock) k_tile_emit(StepArgs a, const int *tile_off, int n_tiles_all,
+                                                      const int *tile_flag, const int *tile_pos, TileItem *tiles,
+                                                      TileRun *runs, int *weight, int tile_cost, int *n_tiles)
+{
+    const int t = (blockIdx.x * kBlock + threadIdx.x) / kTileLanes, k = threadIdx.x & (kTileLanes - 1);
+    if (t >= n_tiles_all) return;
+    const int live = tile_flag[t], pos = tile_pos[t];
+    if (t == n_tiles_all - 1 && k == 0) *n_tiles = pos + live;
+    if (!live) return;
+    int sc, col0, row0;
+    const SceneDev &S = tile_place(a, tile_off, t, sc, col0, row0);
     const int rend = min(row0 + a.ty, S.c.gridY);
-    // bounding box of the cells that hold points; cell_start is nondecreasing,
-    // so the first and last occupied rows of a column are found by bisection
-    int c_lo = a.tx, c_hi = -1, r_lo = a.ty, r_hi = -1;
-    for (int k = 0; k < a.tx; k++) {
-        const int col = col0 + k;
-        if (col >= S.c.ncols) break;
-        const int *cs = a.cell_start + S.cell_off + (long long)col * S.c.gridY;
-        const int s0 = cs[row0], s1 = cs[rend];
-        if (s1 == s0) continue;
-        c_lo = min(c_lo, k);
-        c_hi = k;
-        int l = row0, h = rend - 1;           // first row r with cs[r + 1] > s0
-        while (l < h) {
-            const int m = (l + h) >> 1;
-            if (cs[m + 1] > s0) h = m;
-            else l = m + 1;
+    int c_lo = kTileLanes, c_hi = 0, r_lo = a.ty, r_hi = 0, s0 = 0, n = 0;   // c_hi, r_hi: negated for the minimum
+    if (k < a.tx && col0 + k < S.c.ncols) {
+        const int *cs = a.cell_start + S.cell_off + (long long)(col0 + k) * S.c.gridY;
+        s0 = cs[row0];
+        const int s1 = cs[rend];
+        n = s1 - s0;
+        if (n > 0) {
+            c_lo = k;
+            c_hi = -k;
+            int l = row0, h = rend - 1;           // first row r with cs[r + 1] > s0
+            int l2 = row0, h2 = rend - 1;         // last row r with cs[r] < s1
+            while (l < h || l2 < h2) {
+                const int m = (l + h) >> 1, m2 = (l2 + h2 + 1) >> 1;
+                const int v = cs[m + 1], v2 = cs[m2];
+                if (l < h) {
+                    if (v > s0) h = m;
+                    else l = m + 1;
+                }
+                if (l2 < h2) {
+                    if (v2 < s1) l2 = m2;
+                    else h2 = m2 - 1;
+                }
+            }
+            r_lo = l - row0;
+            r_hi = -(l2 - row0);
         }
-        r_lo = min(r_lo, l - row0);
-        l = row0;
-        h = rend - 1;                         // last row r with cs[r] < s1
-        while (l < h) {
-            const int m = (l + h + 1) >> 1;
-            if (cs[m] < s1) l = m;
-            else h = m - 1;
-        }
-        r_hi = max(r_hi, l - row0);
     }
-    TileItem it;
-    it.scene = lo;
-    it.col0 = col0 + c_lo;
-    it.row0 = row0 + r_lo;
-    it.dims = (c_hi - c_lo + 1) | ((r_hi - r_lo + 1) << 16);
-    tiles[tile_pos[t]] = it;
+    c_lo = half_wave_min(c_lo);
+    c_hi = -half_wave_min(c_hi);
+    r_lo = half_wave_min(r_lo);
+    r_hi = -half_wave_min(r_hi);
+    int end = n;   // inclusive prefix sum over the columns
+#pragma unroll
+    for (int o = 1; o < kTileLanes; o <<= 1) {
+        const int v = __shfl_up(end, o, kTileLanes);
+        if (k >= o) end += v;
+    }
+    const int total = __shfl(end, kTileLanes - 1, kTileLanes);
+    if (k >= c_lo && k <= c_hi) {
+        TileRun r;
+        r.off = s0 - (end - n);
+        r.end = end;
+        runs[(long long)pos * a.tx + k - c_lo] = r;
+    }
+    if (k == 0) {
+        TileItem it{};
+        it.scene = sc;
+        it.col0 = col0 + c_lo;
+        it.row0 = row0 + r_lo;
+        it.dims = (c_hi - c_lo + 1) | ((r_hi - r_lo + 1) << 16);
+        it.total = total;
+        tiles[pos] = it;
+        weight[pos] = total + tile_cost;
+    }
+}
+
+// Splits the tiles among the workgroups of a tile launch.  The table is cut
+// into `parts` ranges, one per XCD (the workgroups of a range run on one XCD,
+// see xcd_block), of equal count if no workgroup gets two tiles, else of equal
+// summed weight (points, plus tile_cost per tile).  The workgroups of a range
+// take its tiles in turn: those at work at the same time are neighbours, whose
+// window nodes overlap in the XCD's L2 (with neighbours one after the other in
+// one workgroup instead, the launch of the 4M-point sheet was 13% slower at
+// 14x32 cells).  Before, the whole table was taken in turn by all workgroups,
+// and the last, partial round ran on the first XCDs alone: 12.7% slower on 1.2M
+// points of floes (8x32 cells), 26% on the 2.0M-point sheet in the mixed form
+// (14x32).  pre: exclusive prefix sums of the weights.
+__global__ void __launch_bounds__(kBlock) k_tile_split(const TileItem *tiles, const int *weight, const int *pre,
+                                                       const int *n_tiles, TileWork *work, int n_work, int parts)
+{
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n_work) return;
+    const int n = *n_tiles, per = n_work / parts, part = i / per;
+    // first tile of range k: the first whose middle (doubled) reaches k parts of the weight
+    auto start = [&](int k) {
+        if (n <= n_work) return (int)((long long)n * k / parts);
+        const unsigned long long w2 = 2ull * ((long long)pre[n - 1] + weight[n - 1]);
+        int lo = 0, hi = n;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if ((2ull * pre[mid] + weight[mid]) * parts >= w2 * k) hi = mid;
+            else lo = mid + 1;
+        }
+        return lo;
+    };
+    TileWork out{};
+    out.first = start(part) + i % per;
+    out.end = start(part + 1);
+    out.step = per;
+    if (out.first < out.end) out.item = tiles[out.first];
+    work[i] = out;
+}
+
+// Tiles that hold points under each of several shapes (blockIdx.y).
+__global__ void __launch_bounds__(kBlock) k_tile_census(StepArgs a, TileShapes shapes, int *counts)
+{
+    const int tx = shapes.tx[blockIdx.y], ty = shapes.ty[blockIdx.y];
+    int live = 0;
+    for (int sc = 0; sc < a.nscenes; sc++) {
+        const SceneDev &S = a.scenes[sc];
+        const int ntx = (S.c.ncols + tx - 1) / tx, nty = (S.c.gridY + ty - 1) / ty;
+        const long long n = (long long)ntx * nty;
+        for (long long t = (long long)blockIdx.x * kBlock + threadIdx.x; t < n; t += (long long)gridDim.x * kBlock) {
+            const int col0 = (int)(t / nty) * tx, row0 = (int)(t % nty) * ty, rend = min(row0 + ty, S.c.gridY);
+            int points = 0;
+            for (int c = col0; c < min(col0 + tx, S.c.ncols); c++) {
+                const int *cs = a.cell_start + S.cell_off + (long long)c * S.c.gridY;
+                points |= cs[rend] - cs[row0];
+            }
+            live += points != 0;
+        }
+    }
+#pragma unroll
+    for (int k = 32; k > 0; k >>= 1) live += __shfl_xor(live, k);
+    if ((threadIdx.x & 63) == 0 && live) atomicAdd(&counts[blockIdx.y], live);
 }
 
 inline unsigned nblk(long long n, int b) { return (unsigned)((n + b - 1) / b); }
@@ -291,19 +391,44 @@ hipError_t launch_sort(const StepArgs &a, const SceneDev *host_scenes, int nscen
     return hipGetLastError();
 }
 
-hipError_t launch_build_tiles(const StepArgs &a, const SceneDev *host_scenes, int nscenes, const BinWork &w,
-                              TileItem *tiles, int *n_tiles, long long max_tiles, hipStream_t s)
+hipError_t launch_tile_census(const StepArgs &a, const TileShapes &shapes, long long n_cells, int *counts,
+                              hipStream_t s)
 {
-    (void)w;
-    // tile_off, tile_n, tile_flag and tile_pos live in the tail of `tiles`
-    // storage: the caller sized it as max_tiles TileItems followed by
-    // 4*(max_tiles+nscenes+1) + max_tiles/1000 + 64 ints.
-    int *ibase = (int *)(tiles + max_tiles);
-    int *tile_off = ibase;
-    int *tile_n = tile_off + nscenes + 1;
-    int *tile_flag = tile_n + max_tiles;
-    int *tile_pos = tile_flag + max_tiles;
-    int *scan_tmp = tile_pos + max_tiles;
+    const hipError_t e = launch_fill_zero(counts, sizeof(int) * shapes.n, s);
+    if (e != hipSuccess) return e;
+    const unsigned g = (unsigned)std::min<long long>(std::max<long long>(n_cells / (32 * kBlock), 1), 256);
+    hipLaunchKernelGGL(k_tile_census, dim3(g, shapes.n), dim3(kBlock), 0, s, a, shapes, counts);
+    return hipGetLastError();
+}
+
+// The parts of a tile table of at most max_tiles tiles in one allocation: the
+// workgroups' work, the items, their runs, the tile count, and the builder's
+// own ints (scene offsets, flags, positions or weight sums, weights, scan sums).
+size_t tile_table_layout(char *base, long long max_tiles, int tx, int nscenes, int n_work, TileTable &t)
+{
+    size_t at = 0;
+    auto part = [&](size_t bytes) {
+        char *p = base + at;
+        at = (at + bytes + 63) / 64 * 64;
+        return p;
+    };
+    t.max_tiles = max_tiles;
+    t.n_work = n_work;
+    t.work = (TileWork *)part(sizeof(TileWork) * n_work);
+    t.tiles = (TileItem *)part(sizeof(TileItem) * max_tiles);
+    t.runs = (TileRun *)part(sizeof(TileRun) * tx * max_tiles);
+    t.n_tiles = (int *)part(sizeof(int));
+    t.tile_off = (int *)part(sizeof(int) * (nscenes + 1));
+    t.flag = (int *)part(sizeof(int) * max_tiles);
+    t.pos = (int *)part(sizeof(int) * max_tiles);
+    t.weight = (int *)part(sizeof(int) * max_tiles);
+    t.scan_tmp = (int *)part(sizeof(int) * (max_tiles / 1000 + 64));
+    return at;
+}
+
+hipError_t launch_build_tiles(const StepArgs &a, const SceneDev *host_scenes, int nscenes, long long n_points,
+                              const TileTable &t, hipStream_t s)
+{
     long long total = 0;
     std::vector<int> off(nscenes + 1);
     for (int i = 0; i < nscenes; i++) {
@@ -311,15 +436,22 @@ hipError_t launch_build_tiles(const StepArgs &a, const SceneDev *host_scenes, in
         total += (long long)host_scenes[i].n_tiles_x * host_scenes[i].n_tiles_y;
     }
     off[nscenes] = (int)total;
-    if (total > max_tiles || total == 0) return hipErrorInvalidValue;
-    hipError_t e = hipMemcpyAsync(tile_off, off.data(), sizeof(int) * (nscenes + 1), hipMemcpyHostToDevice, s);
+    if (total > t.max_tiles || total == 0 || a.tx > kTileLanes || t.n_work <= 0) return hipErrorInvalidValue;
+    // a tile's staging and flush cost about as much as 250 points (the sums of
+    // the weights stay below 2^31)
+    const int tile_cost = (int)std::max<long long>(0, std::min<long long>(250, (0x7fffffff - n_points) / total - 1));
+    hipError_t e = hipMemcpyAsync(t.tile_off, off.data(), sizeof(int) * (nscenes + 1), hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return e;
-    const unsigned g = nblk(total, kBlock);
-    hipLaunchKernelGGL(k_tile_count, dim3(g), dim3(kBlock), 0, s, a, tile_off, (int)total, tile_n, tile_flag);
+    const unsigned g = nblk(total * kTileLanes, kBlock);
+    hipLaunchKernelGGL(k_tile_count, dim3(g), dim3(kBlock), 0, s, a, t.tile_off, (int)total, t.flag);
     // positions of the non-empty tiles: exclusive scan of the 0/1 flags
-    if ((e = scan_exclusive(tile_flag, tile_pos, total, scan_tmp, s)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_tile_emit, dim3(g), dim3(kBlock), 0, s, a, tile_off, (int)total, tile_n, tile_pos, tiles,
-                       n_tiles);
+    if ((e = scan_exclusive(t.flag, t.pos, total, t.scan_tmp, s)) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_tile_emit, dim3(g), dim3(kBlock), 0, s, a, t.tile_off, (int)total, t.flag, t.pos, t.tiles,
+                       t.runs, t.weight, tile_cost, t.n_tiles);
+    // (weights past the live tiles are not read from the sums)
+    if ((e = scan_exclusive(t.weight, t.pos, total, t.scan_tmp, s)) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_tile_split, dim3(nblk(t.n_work, kBlock)), dim3(kBlock), 0, s, t.tiles, t.weight, t.pos,
+                       t.n_tiles, t.work, t.n_work, t.n_work % 8 ? 1 : 8);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     // the host copy of off[] must stay alive until the copy ran

@@ -124,6 +124,11 @@ private:
     int push_clocks();
     int build_tiles();
     int alloc_bins();
+    int alloc_tiles();
+    long long count_tiles(int tx, int ty) const;
+    size_t table_bytes(int tx, int ty, int n_work) const;
+    int apply_tile_shape(int tx, int ty, int margin);
+    int choose_tile_shape();
     StepArgs args() const;
     // timed: record hipEvents around the launches of every sample-th substep
     int launch_substeps(int nsub, int start_buf, bool fused, bool direct, bool timed, int sample = 1);
@@ -158,32 +163,33 @@ private:
     long long pitch_ = 0;          // elements per SoA line
     long long n_pts_space_ = 0;    // point index space (sum of scene capacities)
     void *grid_mem_ = nullptr;
+    long long grid_buf_bytes_ = 0; // bytes of one of the three grid buffers (all scenes)
     double *ind_force_mem_ = nullptr;
     SceneDev *d_scenes_ = nullptr;
     SceneClock *d_clocks_ = nullptr;
     unsigned *d_err_ = nullptr;
     int *d_tile_queue_ = nullptr;
     int *d_dirty_ = nullptr;   // kGridBuffers * n_segs_ segment flags
-    int *d_defer_ = nullptr;   // deferred-point list: 2 * n_pts_space_ ints and 64 counters
+    int *d_defer_ = nullptr;   // lists of points set aside: 2 * n_pts_space_ ints
     int clock_slot_ = 0;       // slot of d_clocks_ (2 x nscenes) holding the current clock
     // workgroups of a grid update over n runs: a run per wave, persistent beyond 8 per CU
-    int tile_blocks(int mode);      // workgroups of a tile launch: the resident count
-    int resident_[8] = {0, 0, 0, 0, 0, 0, 0, 0};   // per tile mode; reset when the tile shape changes
     int update_blocks(int n_runs) const { return std::max(1, std::min((n_runs + 3) / 4, n_cus_ * 8)); }
     long long n_segs_ = 0;
     NodeChunk *d_chunks_ = nullptr;
     int n_chunks_ = 0;
+    int n_service_ = 0;            // workgroups for the indenter force in a substep launch
 
     // binning
     BinWork bins_{};
     void *bin_mem_ = nullptr;
     bool bins_valid_ = false;      // cell_start/tiles describe the current point order
     void *tile_mem_ = nullptr;
-    TileItem *d_tiles_ = nullptr;
-    int *d_n_tiles_ = nullptr;
-    long long max_tiles_ = 0;
-    int n_live_tiles_ = 0;
+    size_t tile_mem_bytes_ = 0;
+    TileTable tiles_;
+    static constexpr int kMinTile[2] = {4, 8};   // the smallest shape choose_tile_shape() takes
+    static constexpr size_t kTileMemStart = 64u << 20;   // most memory taken for it ahead
     int tx_ = 8, ty_ = 32, margin_ = 1;
+    bool tiles_pinned_ = false;    // the caller (or the autotuner) chose the shape
     int lane_spread_ = 1;
     int dyn_tiles_ = 0;
     std::vector<SceneDev> host_dev_;

@@ -96,6 +96,9 @@ int Engine::hipfail(hipError_t e, const char *what)
         if (_rc != ICEMPM_OK) return _rc;                      \
     } while (0)
 
+#define LAUNCH_PREC(fn, ...) \
+    (precision_ == ICEMPM_PRECISION_MIXED ? mixed::fn(__VA_ARGS__) : fp64::fn(__VA_ARGS__))
+
 long long Engine::total_points() const
 {
     long long n = 0;
@@ -311,7 +314,14 @@ int Engine::build_scene_dev(int i, SceneDev &d) const
 int Engine::push_scenes()
 {
     host_dev_.resize(nscenes());
-    for (int i = 0; i < nscenes(); i++) build_scene_dev(i, host_dev_[i]);
+    int n_ind = 0;
+    for (int i = 0; i < nscenes(); i++) {
+        build_scene_dev(i, host_dev_[i]);
+        n_ind += host_dev_[i].c.ind_rsq > 0;
+    }
+    // service workgroups of the substep launches: one per scene with an
+    // indenter, at most 16 (each takes every n_service-th scene)
+    n_service_ = std::min(n_ind, 16);
     HIPCHK(hipMemcpyAsync(d_scenes_, host_dev_.data(), sizeof(SceneDev) * nscenes(), hipMemcpyHostToDevice, stream_));
     HIPCHK(hipStreamSynchronize(stream_));
     return ICEMPM_OK;
@@ -383,12 +393,11 @@ int Engine::commit()
         for (int i = 0; i < nscenes(); i++) { scenes_[i].pt_off = offs[i]; scenes_[i].n_pts = 0; }
     }
 
-    // deferred-point list of the kTileFromMomenta launches: a point index and
-    // a scene per point of the point space, and two counters (zero)
+    // lists of the points that kTileFromMomenta launches set aside: a link and
+    // a scene per point of the point space
     if (!points_layout_same || !d_defer_) {
         if (d_defer_) { hipFree(d_defer_); d_defer_ = nullptr; }
-        HIPCHK(hipMalloc(&d_defer_, sizeof(int) * (2 * n_pts_space_ + 64)));
-        HIPCHK(hipMemsetAsync(d_defer_ + 2 * n_pts_space_, 0, sizeof(int) * 64, stream_));
+        HIPCHK(hipMalloc(&d_defer_, sizeof(int) * 2 * std::max<long long>(n_pts_space_, 1)));
     }
 
     // grids: [buffer 0 of all scenes][buffer 1 ...][buffer 2 ...], 3 FP64 lines
@@ -412,6 +421,7 @@ int Engine::commit()
     // cell keys, bin counts and cell starts are 32-bit
     if (cells >= (1LL << 31) - 1) return fail(ICEMPM_ERR_CAPACITY, "grid cells of all scenes exceed 2^31");
     const size_t buf_bytes = (size_t)gelems * sizeof(double);
+    grid_buf_bytes_ = (long long)buf_bytes;
     HIPCHK(hipMalloc(&grid_mem_, kGridBuffers * buf_bytes));
     HIPCHK(hipMemsetAsync(grid_mem_, 0, kGridBuffers * buf_bytes, stream_));
     // segment flags (grid_elems is a multiple of the segment size); each scene's
@@ -453,7 +463,9 @@ int Engine::commit()
     for (int i = 0; i < nscenes(); i++) {
         const int nseg = (int)(scenes_[i].grid_elems >> kSegShift);
         const int len = update_run_length(scenes_[i].grid_elems);
-        for (int s0 = 0; s0 < nseg; s0 += len) chunks.push_back({i, s0, std::min(len, nseg - s0), 0});
+        for (int s0 = 0; s0 < nseg; s0 += len)
+            chunks.push_back({i, s0, std::min(len, nseg - s0), (int)(scenes_[i].seg_off + s0),
+                              (char *)scenes_[i].grid[0] - (char *)grid_mem_, scenes_[i].grid_elems});
     }
     if (d_chunks_) hipFree(d_chunks_);
     n_chunks_ = (int)chunks.size();
@@ -488,19 +500,52 @@ int Engine::alloc_bins()
     bins_.scan_tmp = p; p += nscan;
     bins_.scene_count = p;
     HIPCHK(hipMemsetAsync(bin_mem_, 0, sizeof(int) * n_int, stream_));
-    // tile table for the current shape
-    if (tile_mem_) { hipFree(tile_mem_); tile_mem_ = nullptr; }
+    return alloc_tiles();
+}
+
+long long Engine::count_tiles(int tx, int ty) const
+{
     long long mt = 0;
     for (auto &s : scenes_) {
         const long long ncols = s.prms.GridXTotal + 2LL * s.prms.GridHaloSize;
-        mt += ((ncols + tx_ - 1) / tx_) * ((s.prms.GridY + ty_ - 1) / ty_);
+        mt += ((ncols + tx - 1) / tx) * ((s.prms.GridY + ty - 1) / ty);
     }
-    max_tiles_ = mt;
-    const size_t tbytes = sizeof(TileItem) * mt + sizeof(int) * (4 * (mt + nscenes() + 1) + mt / 1000 + 64) + 64;
-    HIPCHK(hipMalloc(&tile_mem_, tbytes));
-    HIPCHK(hipMemsetAsync(tile_mem_, 0, tbytes, stream_));
-    d_tiles_ = (TileItem *)tile_mem_;
-    d_n_tiles_ = (int *)((char *)tile_mem_ + tbytes - 64);
+    return mt;
+}
+
+size_t Engine::table_bytes(int tx, int ty, int n_work) const
+{
+    TileTable t;
+    return tile_table_layout(nullptr, count_tiles(tx, ty), tx, nscenes(), n_work, t);
+}
+
+// The tile table for the current shape.
+int Engine::alloc_tiles()
+{
+    const long long mt = count_tiles(tx_, ty_);
+    // The kernels loop over their workgroup's tiles, and a launch of exactly
+    // the workgroups the GPU holds at once (one generation) is the fastest:
+    // with more, the later generations start behind the first and the launch
+    // ends on a tail of partly busy CUs (4M-point sheet, substep launch: FP64
+    // 139.7 us with 8 workgroups per CU, 133.5 us with 2, its residency; mixed
+    // 106.0 us with 8, 103.6 us with 4, its residency, 133 us with 2).  The
+    // other launches take the substep launch's count: the tiles are split for it.
+    int r = LAUNCH_PREC(tiles_resident_per_cu, args(), kTileChain);
+    if (r <= 0) r = 8;   // the runtime could not tell: several generations
+    const int n_work = (int)std::min<long long>(std::max<long long>(mt, 1), (long long)n_cus_ * r);
+    const size_t tbytes = tile_table_layout(nullptr, mt, tx_, nscenes(), n_work, tiles_);
+    if (tbytes > tile_mem_bytes_) {
+        // room for the smallest shape choose_tile_shape() may take, unless the
+        // grids are huge: no second allocation when it does
+        const size_t bytes =
+            std::max(tbytes, std::min(table_bytes(kMinTile[0], kMinTile[1], n_cus_ * 8), kTileMemStart));
+        if (tile_mem_) { hipFree(tile_mem_); tile_mem_ = nullptr; }
+        tile_mem_bytes_ = 0;
+        HIPCHK(hipMalloc(&tile_mem_, bytes));
+        tile_mem_bytes_ = bytes;
+    }
+    tile_table_layout((char *)tile_mem_, mt, tx_, nscenes(), n_work, tiles_);
+    HIPCHK(launch_fill_zero(tiles_.work, sizeof(TileWork) * n_work, stream_));   // no tiles until the next build
     return ICEMPM_OK;
 }
 
@@ -521,8 +566,11 @@ StepArgs Engine::args() const
     a.pts = pts_[0];
     a.pitch = pitch_;
     a.cell_start = bins_.cell_start;
-    a.tiles = d_tiles_;
-    a.n_tiles = d_n_tiles_;
+    a.tiles = tiles_.tiles;
+    a.tile_runs = tiles_.runs;
+    a.tile_work = tiles_.work;
+    a.grid_buf_bytes = grid_buf_bytes_;
+    a.n_tiles = tiles_.n_tiles;
     a.chunks = d_chunks_;
     a.n_chunks = n_chunks_;
     a.nscenes = nscenes();
@@ -536,14 +584,71 @@ StepArgs Engine::args() const
     a.dyn_tiles = dyn_tiles_;
     a.tile_queue = d_tile_queue_;
     a.dirty = d_dirty_;
-    a.defer_pts = d_defer_;
+    a.n_work = tiles_.n_work;
+    a.n_service = n_service_;
+    a.n_clear = std::max(1, std::min((n_chunks_ + 3) / 4, n_cus_ * 8));
+    a.defer_next = d_defer_;
     a.defer_scene = d_defer_ ? d_defer_ + n_pts_space_ : nullptr;
-    a.defer_count = d_defer_ ? d_defer_ + 2 * n_pts_space_ : nullptr;
     a.dirty_stride = n_segs_;
     return a;
 }
 
 int Engine::set_tile_shape(int tx, int ty, int margin)
+{
+    RC(apply_tile_shape(tx, ty, margin));
+    tiles_pinned_ = true;
+    return ICEMPM_OK;
+}
+
+// The tile shape of a scene set whose caller pinned none, by the tiles its
+// points occupy after the first sort of an upload.  The smallest shape whose
+// tiles all run at once is the fastest where there is one: a launch then lasts
+// as long as one workgroup's chain of one tile, and a small tile's points need
+// one pass (FP64 substep of 25.6k points: 8.3 us with 4x8 cells, 12.4 with
+// 8x16, 15.9 with 8x32; 102k points: 12.4 with 4x16, 13.2 with 8x16, 18.3 with
+// 8x32).  Where none fits, larger tiles repeat fewer window nodes, but a
+// second round that is nearly empty costs more: 16x32 from two rounds on (4.0M
+// points, 2.9 rounds: 126 us, 137 with 8x32), else 8x32 (1.2M points of floes,
+// 1.3 rounds of 16x32: 79 us, 64 with 8x32).  Small shapes whose table over a
+// huge grid would take more memory than is set aside for it are left out.
+int Engine::choose_tile_shape()
+{
+    static const int ladder[][2] = {{kMinTile[0], kMinTile[1]}, {4, 16}, {8, 16}, {8, 32}, {16, 32}};
+    constexpr int n = sizeof(ladder) / sizeof(ladder[0]);
+    TileShapes shapes;
+    shapes.n = n;
+    for (int i = 0; i < n; i++) {
+        shapes.tx[i] = ladder[i][0];
+        shapes.ty[i] = ladder[i][1];
+    }
+    static_assert(n <= TileShapes::kMax, "shapes to count");
+    HIPCHK(launch_tile_census(args(), shapes, bins_.n_cells_total, bins_.scan_tmp, stream_));
+    int counts[n];
+    HIPCHK(hipMemcpyAsync(counts, bins_.scan_tmp, sizeof counts, hipMemcpyDeviceToHost, stream_));
+    HIPCHK(hipStreamSynchronize(stream_));
+    int pick = n - 2;
+    for (int i = 0; i < n; i++) {
+        StepArgs a = args();
+        a.tx = shapes.tx[i];
+        a.ty = shapes.ty[i];
+        a.win_w = a.tx + 2 + 2 * margin_;
+        a.win_h = a.ty + 2 + 2 * margin_;
+        if (i < n - 2 && table_bytes(a.tx, a.ty, n_cus_ * 8) > std::max(tile_mem_bytes_, kTileMemStart)) continue;
+        const int r = LAUNCH_PREC(tiles_resident_per_cu, a, kTileChain);
+        if (r > 0 && counts[i] <= (long long)n_cus_ * r) {
+            pick = i;
+            break;
+        }
+        if (r > 0 && i == n - 1 && counts[i] >= 2LL * n_cus_ * r) pick = i;
+    }
+    if (shapes.tx[pick] == tx_ && shapes.ty[pick] == ty_) return ICEMPM_OK;
+    tx_ = shapes.tx[pick];
+    ty_ = shapes.ty[pick];
+    invalidate_graphs();
+    return alloc_tiles();   // the caller pushes the scenes and builds the tiles
+}
+
+int Engine::apply_tile_shape(int tx, int ty, int margin)
 {
     if (tx < 1 || tx > 32 || ty < 1 || ty > 1024 || margin < 0 || margin > 4)
         return fail(ICEMPM_ERR_ARGUMENT, "tile shape out of range");
@@ -553,25 +658,13 @@ int Engine::set_tile_shape(int tx, int ty, int margin)
     const size_t lds = (size_t)(tx + 2 + 2 * margin) * (ty + 2 + 2 * margin) * per_node;
     if (lds > 64 * 1024) return fail(ICEMPM_ERR_ARGUMENT, "tile window exceeds the LDS budget");
     if (tx == tx_ && ty == ty_ && margin == margin_) return ICEMPM_OK;
-    for (int &r : resident_) r = 0;
     tx_ = tx;
     ty_ = ty;
     margin_ = margin;
     invalidate_graphs();
     if (!committed_) return ICEMPM_OK;
     // the tile table depends on the shape; cell_start does not
-    if (tile_mem_) { hipFree(tile_mem_); tile_mem_ = nullptr; }
-    long long mt = 0;
-    for (auto &s : scenes_) {
-        const long long ncols = s.prms.GridXTotal + 2LL * s.prms.GridHaloSize;
-        mt += ((ncols + tx_ - 1) / tx_) * ((s.prms.GridY + ty_ - 1) / ty_);
-    }
-    max_tiles_ = mt;
-    const size_t tbytes = sizeof(TileItem) * mt + sizeof(int) * (4 * (mt + nscenes() + 1) + mt / 1000 + 64) + 64;
-    HIPCHK(hipMalloc(&tile_mem_, tbytes));
-    HIPCHK(hipMemsetAsync(tile_mem_, 0, tbytes, stream_));
-    d_tiles_ = (TileItem *)tile_mem_;
-    d_n_tiles_ = (int *)((char *)tile_mem_ + tbytes - 64);
+    RC(alloc_tiles());
     RC(push_scenes());
     if (bins_valid_) RC(build_tiles());
     return ICEMPM_OK;
@@ -757,9 +850,6 @@ int Engine::zero_grid(int scene, int buf)
     return ICEMPM_OK;
 }
 
-#define LAUNCH_PREC(fn, ...) \
-    (precision_ == ICEMPM_PRECISION_MIXED ? mixed::fn(__VA_ARGS__) : fp64::fn(__VA_ARGS__))
-
 // The single-phase calls record hipEvents around their launch (the host-driven
 // substep loop reads per-phase times like the reference's record_timings).
 int Engine::reset_grid(int scene)
@@ -771,29 +861,13 @@ int Engine::reset_grid(int scene)
     return rc;
 }
 
-// Workgroups of a tile launch.  The kernels loop over the tile list, and a
-// launch of exactly the workgroups the GPU holds at once (one generation) is
-// the fastest: with more, the later generations start behind the first and the
-// launch ends on a tail of partly busy CUs (4M-point sheet, fused launch: FP64
-// 139.7 us with 8 workgroups per CU, 133.5 us with 2, its residency; mixed
-// 106.0 us with 8, 103.6 us with 4, its residency, 133 us with 2).
-int Engine::tile_blocks(int mode)
-{
-    int &r = resident_[mode & 7];
-    if (r <= 0) {
-        r = LAUNCH_PREC(tiles_resident_per_cu, args(), mode);
-        if (r <= 0) r = 8;   // the runtime could not tell: several generations
-    }
-    return (int)std::min<long long>(std::max<long long>(max_tiles_, 1), (long long)n_cus_ * r);
-}
-
 int Engine::p2g(int scene)
 {
     RC(ensure_committed());
     const StepArgs a = args();
     timed_begin(true);
     if (bins_valid_ && nscenes() == 1) {
-        HIPCHK(LAUNCH_PREC(launch_tiles, a, kTileP2G, 0, 0, 0, 0, tile_blocks(kTileP2G), stream_));
+        HIPCHK(LAUNCH_PREC(launch_tiles, a, kTileP2G, 0, 0, 0, 0, stream_));
     } else {
         HIPCHK(LAUNCH_PREC(launch_p2g_direct, a, scene, scenes_[scene].n_pts, 0, stream_));
     }
@@ -842,7 +916,7 @@ int Engine::g2p(int scene, int recordPQ)
     const StepArgs a = args();
     timed_begin(true);
     if (bins_valid_ && nscenes() == 1) {
-        HIPCHK(LAUNCH_PREC(launch_tiles, a, kTileG2P, 0, 0, 0, recordPQ ? 1 : 0, tile_blocks(kTileG2P), stream_));
+        HIPCHK(LAUNCH_PREC(launch_tiles, a, kTileG2P, 0, 0, 0, recordPQ ? 1 : 0, stream_));
     } else {
         HIPCHK(LAUNCH_PREC(launch_g2p_direct, a, scene, scenes_[scene].n_pts, 0, recordPQ ? 1 : 0, stream_));
     }
@@ -928,14 +1002,13 @@ int Engine::get_grid(int scene, int buf, double *out, long long n_nodes)
 int Engine::build_tiles()
 {
     const StepArgs a = args();
-    HIPCHK(launch_build_tiles(a, host_dev_.data(), nscenes(), bins_, d_tiles_, d_n_tiles_, max_tiles_, stream_));
+    HIPCHK(launch_build_tiles(a, host_dev_.data(), nscenes(), total_points(), tiles_, stream_));
     int nt = 0;
-    HIPCHK(hipMemcpy(&nt, d_n_tiles_, sizeof(int), hipMemcpyDeviceToHost));
-    if (nt < 0 || nt > max_tiles_) {
+    HIPCHK(hipMemcpy(&nt, tiles_.n_tiles, sizeof(int), hipMemcpyDeviceToHost));
+    if (nt < 0 || nt > tiles_.max_tiles) {
         bins_valid_ = false;
         return fail(ICEMPM_ERR_STATE, "build_tiles: tile count out of range");
     }
-    n_live_tiles_ = nt;
     return ICEMPM_OK;
 }
 
@@ -961,6 +1034,7 @@ int Engine::sort()
         scenes_[i].n_pts = m;
     }
     if (counts_changed) invalidate_graphs();
+    if (!tiles_pinned_ && !bins_valid_) RC(choose_tile_shape());
     RC(push_scenes());
     RC(build_tiles());
     bins_valid_ = true;
@@ -1019,7 +1093,7 @@ int Engine::emit_units(int kind, int n, int b, int cs, bool timed_all, int sampl
         switch (kind) {
         case kUnitHead:
             timed_begin(timed);
-            HIPCHK(LAUNCH_PREC(launch_tiles, au, kTileP2G, b, b, b, -1, tile_blocks(kTileP2G), stream_));
+            HIPCHK(LAUNCH_PREC(launch_tiles, au, kTileP2G, b, b, b, -1, stream_));
             timed_end(timed, kClsP2G);
             continue;                  // part of substep 0: no clock or buffer change
         case kUnitChain:
@@ -1027,7 +1101,7 @@ int Engine::emit_units(int kind, int n, int b, int cs, bool timed_all, int sampl
             const int mode = kind == kUnitChain ? kTileChain : kTileTail;
             const int w = kind == kUnitChain ? (b + 1) % kGridBuffers : b, z = (b + 2) % kGridBuffers;
             timed_begin(timed);
-            HIPCHK(LAUNCH_PREC(launch_tiles, au, mode, b, w, z, -1, tile_blocks(mode), stream_));
+            HIPCHK(LAUNCH_PREC(launch_tiles, au, mode, b, w, z, -1, stream_));
             timed_end(timed, kind == kUnitChain ? kClsFused : kClsG2P);
             b = w;
             cs ^= 1;
@@ -1056,13 +1130,13 @@ int Engine::emit_units(int kind, int n, int b, int cs, bool timed_all, int sampl
             continue;
         default:   // kUnitUnfused
             timed_begin(timed);
-            HIPCHK(LAUNCH_PREC(launch_tiles, au, kTileP2G, b, b, b, -1, tile_blocks(kTileP2G), stream_));
+            HIPCHK(LAUNCH_PREC(launch_tiles, au, kTileP2G, b, b, b, -1, stream_));
             timed_end(timed, kClsP2G);
             timed_begin(timed);
             HIPCHK(fp64::launch_update(au, b, 1, 1, nb_upd, stream_));
             timed_end(timed, kClsUpdate);
             timed_begin(timed);
-            HIPCHK(LAUNCH_PREC(launch_tiles, an, kTileG2P, b, b, b, -1, tile_blocks(kTileG2P), stream_));
+            HIPCHK(LAUNCH_PREC(launch_tiles, an, kTileG2P, b, b, b, -1, stream_));
             timed_end(timed, kClsG2P);
             cs ^= 1;
             b ^= 1;
@@ -1101,8 +1175,6 @@ int Engine::chunk_graph(int kind, int n, int b, int cs, int tmode, bool first_ti
         // The capture records the timing events into the graph: it takes them
         // from the pool (emptied first) and keeps them.
         if (tmode) RC(collect_timings());
-        // workgroup counts are runtime queries: make them before the capture
-        for (int m : {(int)kTileG2P, (int)kTileP2G, (int)kTileTail, (int)kTileChain}) tile_blocks(m);
         HIPCHK(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
         capturing_ = true;
         // first_timed with sampling: unit 0 of the chunk is a sampled substep
@@ -1346,7 +1418,7 @@ int Engine::autotune(int n_trials, float *out_ms, int n_out, int *chosen)
         lane_spread_ = cf[2];
         dyn_tiles_ = cf[3];
         ms = -1;
-        if (set_tile_shape(cf[0], cf[1], margin) != ICEMPM_OK) return ICEMPM_OK;
+        if (apply_tile_shape(cf[0], cf[1], margin) != ICEMPM_OK) return ICEMPM_OK;
         RC(step(1, 0));   // warm-up
         std::vector<GraphExec *> none;
         int b = 0, cs = clock_slot_;
@@ -1404,7 +1476,7 @@ int Engine::autotune(int n_trials, float *out_ms, int n_out, int *chosen)
     if (best_i < 0 || rc != ICEMPM_OK) {
         lane_spread_ = ls0;
         dyn_tiles_ = dy0;
-        RC(set_tile_shape(tx0, ty0, margin0));
+        RC(apply_tile_shape(tx0, ty0, margin0));
     } else {
         lane_spread_ = kTileCandidates[best_i][2];
         dyn_tiles_ = kTileCandidates[best_i][3];

@@ -23,8 +23,7 @@ enum TileMode {
 
 namespace fp64 {
 // record_mode: 1/0 = write P, Q or not; -1 = decide from the scene clock.
-hipError_t launch_tiles(const StepArgs &a, int mode, int rbuf, int wbuf, int zbuf, int record_mode, int n_blocks,
-                        hipStream_t s);
+hipError_t launch_tiles(const StepArgs &a, int mode, int rbuf, int wbuf, int zbuf, int record_mode, hipStream_t s);
 hipError_t launch_p2g_direct(const StepArgs &a, int scene, int n_pts, int wbuf, hipStream_t s);
 hipError_t launch_g2p_direct(const StepArgs &a, int scene, int n_pts, int rbuf, int record_pq, hipStream_t s);
 // Grid update of both precision forms: their grids share one layout (3 FP64
@@ -38,8 +37,7 @@ int tiles_resident_per_cu(const StepArgs &a, int mode);
 
 namespace mixed {
 // record_mode: 1/0 = write P, Q or not; -1 = decide from the scene clock.
-hipError_t launch_tiles(const StepArgs &a, int mode, int rbuf, int wbuf, int zbuf, int record_mode, int n_blocks,
-                        hipStream_t s);
+hipError_t launch_tiles(const StepArgs &a, int mode, int rbuf, int wbuf, int zbuf, int record_mode, hipStream_t s);
 hipError_t launch_p2g_direct(const StepArgs &a, int scene, int n_pts, int wbuf, hipStream_t s);
 hipError_t launch_g2p_direct(const StepArgs &a, int scene, int n_pts, int rbuf, int record_pq, hipStream_t s);
 size_t tile_lds_bytes(const StepArgs &a, int mode);
@@ -68,7 +66,28 @@ struct BinWork {
 // elem_bytes: 8 (FP64 SoA) or 4 (mixed SoA).
 hipError_t launch_sort(const StepArgs &a, const SceneDev *host_scenes, int nscenes, BinWork &w, int elem_bytes,
                        void *pts_src, void *pts_dst, hipStream_t s);
-hipError_t launch_build_tiles(const StepArgs &a, const SceneDev *host_scenes, int nscenes, const BinWork &w,
-                              TileItem *tiles, int *n_tiles, long long max_tiles, hipStream_t s);
+// Tile shapes to count the tiles of (launch_tile_census: counts[i] = tiles of
+// shape i that hold points, by the current cell_start).
+struct TileShapes {
+    static constexpr int kMax = 8;
+    int n = 0;
+    int tx[kMax], ty[kMax];
+};
+hipError_t launch_tile_census(const StepArgs &a, const TileShapes &shapes, long long n_cells, int *counts,
+                              hipStream_t s);
+// The tile table of the binned kernels (mpm_common.h) and its builder's memory.
+struct TileTable {
+    long long max_tiles = 0;
+    int n_work = 0;               // workgroups of a tile launch
+    TileWork *work = nullptr;
+    TileItem *tiles = nullptr;
+    TileRun *runs = nullptr;
+    int *n_tiles = nullptr;
+    int *tile_off = nullptr, *flag = nullptr, *pos = nullptr, *weight = nullptr, *scan_tmp = nullptr;
+};
+// Lays the table out from base (null: only counts); returns its bytes.
+size_t tile_table_layout(char *base, long long max_tiles, int tx, int nscenes, int n_work, TileTable &t);
+hipError_t launch_build_tiles(const StepArgs &a, const SceneDev *host_scenes, int nscenes, long long n_points,
+                              const TileTable &t, hipStream_t s);
 
 }  // namespace icempm

@@ -26,8 +26,13 @@ constexpr long long kMaxPointSpace = 1LL << 29;
 constexpr int kSegShift = 6, kSegNodes = 1 << kSegShift;
 // Segments per grid-update work item (one wave; one flag per lane): short runs
 // spread dense grids over many waves, long runs let a wave skip a large empty
-// grid with one flag load per 64 segments.
-inline int update_run_length(long long grid_nodes) { return grid_nodes > (8LL << 20) ? 64 : 16; }
+// grid with one flag load per 64 segments.  Grids of up to 2^18 nodes have
+// fewer runs of 2 segments than a launch has waves, so one more segment per
+// run is one more pass of the launch's slowest wave.
+inline int update_run_length(long long grid_nodes)
+{
+    return grid_nodes > (8LL << 20) ? 64 : grid_nodes > (1LL << 20) ? 16 : grid_nodes > (1LL << 18) ? 4 : 2;
+}
 
 // FP32 constants of the mixed form, converted by the host (the kernels keep
 // them in scalar registers).
@@ -110,10 +115,20 @@ struct SceneClock {
 // the points are those of the box's cells, and the tile's LDS window is the
 // box widened by the drift margin and the stencil's one node on every side.
 // Tiles of a sparse scene (floe edges, gaps) thus stage fewer empty nodes.
+// The points of the box's columns are runs of the sorted order, listed in
+// StepArgs::tile_runs (tx entries per tile), `total` points in all.
 struct TileItem {
     int scene;
     int col0, row0;
     int dims;
+    int total;
+    int pad[3];
+};
+
+// The run of one column of a tile's box: points [previous end, end) of the
+// tile's `total` are points k + off of the sorted order.
+struct TileRun {
+    int off, end;
 };
 
 // Node window of a tile in LDS: origin (c0, r0) in grid nodes, w x h nodes,
@@ -139,13 +154,26 @@ struct TileWindow {
     __device__ __forceinline__ int nodes() const { return w * h; }
 };
 
+// The tiles of one workgroup of a tile launch: first, first + step, ... < end
+// of the tile table, and a copy of the first one's item, so that a workgroup
+// has its work with one 64-byte load (first >= end: none).
+struct TileWork {
+    TileItem item;
+    int first, end, step;
+    int pad[5];
+};
+
 // A run of up to 64 node segments of one scene (up to 4096 nodes): the unit
 // of work of one wave in the grid update.
+// The scene's grid place is repeated here, so that a wave that clears a run
+// needs no second lookup.
 struct NodeChunk {
     int scene;
     int seg0;     // first segment (node seg0*64)
     int nseg;     // segments in the run, 1..64
-    int pad;
+    int flag0;    // segment flag of seg0 (in each buffer's part of StepArgs::dirty)
+    long long grid_off;   // SceneDev::grid_off[0]
+    long long gpitch;
 };
 
 // Arguments common to all stepping kernels.
@@ -159,7 +187,10 @@ struct StepArgs {
     long long pitch;
     const int *cell_start;    // per scene ncells+1 global point indices (from the last sort)
     const TileItem *tiles;
+    const TileRun *tile_runs; // tx entries per tile
+    const TileWork *tile_work; // one per workgroup of a tile launch
     const int *n_tiles;       // device-side count of live tiles
+    long long grid_buf_bytes; // bytes between a scene's grid buffers
     const NodeChunk *chunks;
     int n_chunks;
     int nscenes;
@@ -171,12 +202,13 @@ struct StepArgs {
     int *tile_queue;          // 8 queue counters + 1 finished-block counter, zero between launches
     int *dirty;               // segment flags: [buffer 0 of all scenes][buffer 1 ...][buffer 2 ...]
     long long dirty_stride;   // segments per buffer (all scenes)
-    // Points a kTileFromMomenta launch sets aside for its last workgroup (one
-    // slot per point of the point space; defer_count[0] = entries, [1] = the
-    // launch's finished workgroups; both zero between launches).
-    int *defer_pts;
+    int n_work;               // tile workgroups of a tile launch
+    int n_service, n_clear;   // workgroups before and after them in a kTileFromMomenta launch (side_work)
+    // Points that a thread of a kTileFromMomenta launch sets aside for the end
+    // of its work: a list per thread, linked through defer_next (one slot per
+    // point of the point space; -1 ends a list), and the points' scenes.
+    int *defer_next;
     int *defer_scene;
-    int *defer_count;
 };
 
 // The clock of the next substep (model.cpp:39-41): t += dt by repeated

@@ -99,7 +99,9 @@ __global__ void k_noalloc_setup(SceneDev d, SceneClock ck, SceneDev *scene, Scen
         r.scene = 0;
         r.seg0 = s0;
         r.nseg = min(run_len, n_segs - s0);
-        r.pad = 0;
+        r.flag0 = s0;
+        r.grid_off = 0;
+        r.gpitch = d.gpitch;
         runs[i] = r;
     }
 }

@@ -45,12 +45,12 @@ struct PtRef {
 };
 
 // Logical block index that keeps consecutive work items on one XCD: workgroups
-// are dispatched round-robin over the 8 XCDs, so block b runs on XCD b%8.
-__device__ __forceinline__ int xcd_block()
+// are dispatched round-robin over the 8 XCDs, so block b of G runs on XCD
+// b%8 (or, behind service blocks, on one that depends on b%8 alone).
+__device__ __forceinline__ int xcd_block(int b, int G)
 {
-    const int G = gridDim.x;
-    if ((G & 7) != 0) return blockIdx.x;
-    return (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
+    if ((G & 7) != 0) return b;
+    return (b & 7) * (G >> 3) + (b >> 3);
 }
 
 // G2P of one point: gathers v and C (kernels.cuh:344-372), advects x, updates F

@@ -13,6 +13,7 @@
 
 #include "kernels.h"
 #include "physics_fp64.h"
+#include "point_fp64.h"
 #include "physics_mixed.h"
 
 namespace icempm {
@@ -372,12 +373,7 @@ __device__ __forceinline__ void store_state_fused(const PtRef &R, long long pt, 
     }
 }
 
-__device__ __forceinline__ int xcd_block()
-{
-    const int G = gridDim.x;
-    if ((G & 7) != 0) return blockIdx.x;
-    return (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
-}
+using fp64::xcd_block;
 
 }  // namespace mixed
 }  // namespace icempm

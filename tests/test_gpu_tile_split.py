@@ -1,0 +1,64 @@
+"""The split of the tile table among the workgroups of a tile launch, and the
+tile shape a partition takes by itself, against the FP64 oracle.
+
+One block of 6,400 points stepped with shapes that give fewer tiles than
+workgroups, several tiles per workgroup (the table cut by weight into one range
+per XCD, taken in turn), and the smallest shape of the built-in rule; and blocks
+of sizes around the rule's changes of shape with no shape set.  Every field to
+1e-9 of its scale after 12 substeps, as for the other tile shapes."""
+import numpy as np
+import pytest
+
+import _oracle as O
+import icempm_multi_amd as im
+from icempm_multi_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = {"x": (4, 6), "v": (6, 8), "F": (8, 12), "C": (12, 16), "Jp": (3, 4)}
+
+
+def step_and_compare(P, h, n, shape, substeps=12):
+    r = np.random.default_rng(n)
+    h[6, :n] = 0.3 * np.sin(3 * h[4, :n])
+    h[7, :n] = -0.2 * np.cos(2 * h[5, :n])
+    h[8:12, :n] += 1e-5 * r.normal(size=(4, n))
+    part = im.Partition(0, 0, im.PRECISION_FP64)
+    part.allocate(h.shape[1], P.GridXTotal)
+    part.update_constants(P)
+    if shape:
+        part.set_tile_shape(*shape)
+    part.transfer_points_from_soa_to_device(h, 0, n)
+    print(f"{n} points, tile {shape}", flush=True)
+    part.step(substeps, im.STEP_GRAPH | im.STEP_RESORT)
+    config = part.tile_config()
+    out = np.zeros_like(h)
+    part.transfer_from_device(out, 0)
+    assert part.error_code == 0
+    part.close()
+    ref = h.copy()
+    O.sort(P, ref, n)
+    O.substeps(P, ref, n, substeps, 0.0, 0)
+    for name, (a, b) in FIELDS.items():
+        scale = np.abs(ref[a:b, :n]).max()
+        assert np.abs(out[a:b, :n] - ref[a:b, :n]).max() <= 1e-9 * scale, name
+    assert np.array_equal(out[0, :n].view(np.int64), ref[0, :n].view(np.int64))
+    return config
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (1, 2, 0), (2, 3, 1), (4, 8, 1), (32, 16, 0)])
+def test_tile_split_matches_oracle(shape):
+    P, h, n = scenes.block_scene(nx=80, ny=20, grid=(128, 64), n_grains=40)
+    c = step_and_compare(P, h, n, shape)
+    assert (c["tx"], c["ty"], c["margin"]) == shape
+
+
+# the second case's tiles lie in columns whose last tile is one cell wide
+@pytest.mark.parametrize("nx,ny", [(16, 4), (61, 33), (200, 128), (150, 400)])
+def test_shape_by_rule_matches_oracle(nx, ny):
+    P, h, n = scenes.block_scene(nx=nx, ny=ny, grid=(nx + 40, ny + 24), n_grains=40)
+    c = step_and_compare(P, h, n, None)
+    # no more cells per tile than the largest shape, and small scenes get the smallest
+    assert c["tx"] * c["ty"] <= 16 * 32
+    if n <= 4096:
+        assert (c["tx"], c["ty"]) == (4, 8)
