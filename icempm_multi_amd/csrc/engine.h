@@ -9,6 +9,7 @@
 
 #include <array>
 #include <map>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -56,9 +57,12 @@ struct SceneHost {
     int sim_step = 0;         // SimulationStep
 };
 
+class CopyPool;   // transfer.hip
+
 class Engine {
 public:
     // Units of a substep call (see emit_units in engine.hip).
+    static constexpr int kStageDepth = 3;   // chunks in flight of a point transfer
     enum UnitKind { kUnitHead = 0, kUnitChain, kUnitTail, kUnitUnfused, kUnitDirect };
 
     Engine(int device, int precision);
@@ -123,6 +127,10 @@ private:
     int push_scenes();
     int push_clocks();
     int build_tiles();
+    // points between a HostSideSOA buffer and the device, through pinned staging
+    int stage_for(long long n, long long &chunk, int &depth);
+    int import_points(int scene, const double *hssoa, size_t capacity, long long offset, long long n);
+    int export_points(int scene, double *hssoa, size_t capacity, long long offset, long long n);
     int alloc_bins();
     int alloc_tiles();
     long long count_tiles(int tx, int ty) const;
@@ -178,6 +186,12 @@ private:
     NodeChunk *d_chunks_ = nullptr;
     int n_chunks_ = 0;
     int n_service_ = 0;            // workgroups for the indenter force in a substep launch
+
+    // pinned staging of the point transfers, and the threads that help with large ones
+    std::shared_ptr<CopyPool> copy_pool_;
+    void *stage_ = nullptr;
+    size_t stage_bytes_ = 0;
+    hipEvent_t stage_ev_[kStageDepth] = {nullptr, nullptr, nullptr};
 
     // binning
     BinWork bins_{};

@@ -69,6 +69,9 @@ Engine::~Engine()
                     bin_mem_, tile_mem_, d_tile_queue_, d_dirty_, d_defer_};
     for (void *b : bufs)
         if (b) hipFree(b);
+    if (stage_) hipHostFree(stage_);
+    for (hipEvent_t e : stage_ev_)
+        if (e) hipEventDestroy(e);
     if (stream_) hipStreamDestroy(stream_);
 }
 
@@ -680,47 +683,7 @@ int Engine::upload(int scene, const double *hssoa, unsigned capacity, int offset
     if (n < 0 || n > s.cap_pts) return fail(ICEMPM_ERR_CAPACITY, "transfer_points_from_soa_to_device: capacity");
     if (offset < 0 || (long long)offset + n > (long long)capacity)
         return fail(ICEMPM_ERR_CAPACITY, "transfer_points_from_soa_to_device: HSSOA capacity");
-    if (precision_ == ICEMPM_PRECISION_FP64) {
-        for (int line = 0; line < kNumPtsLines && n > 0; line++)
-            HIPCHK(hipMemcpyAsync((double *)pts_[0] + line * pitch_ + s.pt_off, hssoa + (size_t)line * capacity + offset,
-                                  sizeof(double) * n, hipMemcpyHostToDevice, stream_));
-    } else {
-        const SceneDev &d = host_dev_[scene];
-        const double scale = std::ldexp(1.0, d.c.frac_bits);
-        const double lim = 4294967295.0;
-        std::vector<uint32_t> buf((size_t)kNumPtsLines * n);
-        auto L = [&](int line, int i) { return hssoa[(size_t)line * capacity + offset + i]; };
-        for (int i = 0; i < n; i++) {
-            long long ud;
-            std::memcpy(&ud, hssoa + offset + i, 8);
-            buf[(size_t)0 * n + i] = (uint32_t)ud;
-            const int org[2] = {d.c.origin, d.c.origin_y};
-            for (int k = 0; k < 2; k++) {
-                double q = std::nearbyint((L(kLinePosX + k, i) * d.c.hinv + org[k]) * scale);
-                q = std::min(std::max(q, 0.0), lim);
-                buf[(size_t)(kLinePosX + k) * n + i] = (uint32_t)q;
-            }
-            auto putf = [&](int line, double v) {
-                const float f = (float)v;
-                std::memcpy(&buf[(size_t)line * n + i], &f, 4);
-            };
-            putf(kLineP, L(kLineP, i));
-            putf(kLineQ, L(kLineQ, i));
-            putf(kLineJp, L(kLineJp, i) - 1.0);   // the mixed form stores Jp_inv - 1
-            putf(kLineVelX, L(kLineVelX, i));
-            putf(kLineVelX + 1, L(kLineVelX + 1, i));
-            putf(kLineFe00, L(kLineFe00, i) - 1.0);
-            putf(kLineFe00 + 1, L(kLineFe00 + 1, i));
-            putf(kLineFe00 + 2, L(kLineFe00 + 2, i));
-            putf(kLineFe00 + 3, L(kLineFe00 + 3, i) - 1.0);
-            for (int k = 0; k < 4; k++) putf(kLineBp00 + k, L(kLineBp00 + k, i));
-        }
-        for (int line = 0; line < kNumPtsLines && n > 0; line++)
-            HIPCHK(hipMemcpyAsync((uint32_t *)pts_[0] + line * pitch_ + s.pt_off, buf.data() + (size_t)line * n,
-                                  sizeof(uint32_t) * n, hipMemcpyHostToDevice, stream_));
-        HIPCHK(hipStreamSynchronize(stream_));
-    }
-    HIPCHK(hipStreamSynchronize(stream_));
+    RC(import_points(scene, hssoa, capacity, offset, n));
     s.n_pts = n;
     bins_valid_ = false;
     invalidate_graphs();
@@ -735,43 +698,7 @@ int Engine::download(int scene, double *hssoa, unsigned capacity, int offset, in
     const int n = s.n_pts;
     if (offset < 0 || (long long)offset + n > (long long)capacity)
         return fail(ICEMPM_ERR_CAPACITY, "transfer_from_device() HSSOA capacity");
-    if (precision_ == ICEMPM_PRECISION_FP64) {
-        for (int line = 0; line < kNumPtsLines && n > 0; line++)
-            HIPCHK(hipMemcpyAsync(hssoa + (size_t)line * capacity + offset, (double *)pts_[0] + line * pitch_ + s.pt_off,
-                                  sizeof(double) * n, hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipStreamSynchronize(stream_));
-    } else {
-        std::vector<uint32_t> buf((size_t)kNumPtsLines * std::max(n, 1));
-        for (int line = 0; line < kNumPtsLines && n > 0; line++)
-            HIPCHK(hipMemcpyAsync(buf.data() + (size_t)line * n, (uint32_t *)pts_[0] + line * pitch_ + s.pt_off,
-                                  sizeof(uint32_t) * n, hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipStreamSynchronize(stream_));
-        const SceneDev &d = host_dev_[scene];
-        const double inv = std::ldexp(1.0, -d.c.frac_bits);
-        for (int i = 0; i < n; i++) {
-            auto getf = [&](int line) {
-                float f;
-                std::memcpy(&f, &buf[(size_t)line * n + i], 4);
-                return (double)f;
-            };
-            auto put = [&](int line, double v) { hssoa[(size_t)line * capacity + offset + i] = v; };
-            const long long ud = (long long)buf[i];
-            std::memcpy(hssoa + offset + i, &ud, 8);
-            const int org[2] = {d.c.origin, d.c.origin_y};
-            for (int k = 0; k < 2; k++)
-                put(kLinePosX + k, ((double)buf[(size_t)(kLinePosX + k) * n + i] * inv - org[k]) * d.c.h);
-            put(kLineP, getf(kLineP));
-            put(kLineQ, getf(kLineQ));
-            put(kLineJp, getf(kLineJp) + 1.0);
-            put(kLineVelX, getf(kLineVelX));
-            put(kLineVelX + 1, getf(kLineVelX + 1));
-            put(kLineFe00, getf(kLineFe00) + 1.0);
-            put(kLineFe00 + 1, getf(kLineFe00 + 1));
-            put(kLineFe00 + 2, getf(kLineFe00 + 2));
-            put(kLineFe00 + 3, getf(kLineFe00 + 3) + 1.0);
-            for (int k = 0; k < 4; k++) put(kLineBp00 + k, getf(kLineBp00 + k));
-        }
-    }
+    RC(export_points(scene, hssoa, capacity, offset, n));
     if (n_out) *n_out = n;
     return ICEMPM_OK;
 }

@@ -1,0 +1,386 @@
+// transfer.hip -- points between HostSideSOA buffers and the device
+// (GPU_Partition::transfer_points_from_soa_to_device and transfer_from_device,
+// gpu_partition.cu:16-68).
+//
+// Chunks of points go through pinned staging memory that kernels read and
+// write over the link, converting the mixed form's elements on the way, while
+// the host copies the chunk before (or after) between staging and the
+// caller's lines.  Before, each line was one copy from or to pageable memory
+// (16 of them per call, 20 us each for any size, 18 GB/s for large ones) and
+// one host thread converted the mixed form's elements.  Per call, before and
+// after: download of 1.6k points 317 -> 29 us, of 4.0M points (512 MB) 30 -> 10
+// ms, in the mixed form 172 -> 10 ms; upload of 4.0M points 17.7 -> 12.5 ms, of
+// 410k points in the mixed form 13 -> 1.4 ms.  The large ones move 41 to 51
+// GB/s over a link whose plain pinned copies reach 57.
+//
+// Built with -ffp-contract=off: the conversions round each operation, as the
+// host code that they replace did.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <cmath>
+#include <condition_variable>
+#include <cstring>
+#include <list>
+#include <memory>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "engine.h"
+#include "icempm_host.h"
+
+namespace icempm {
+
+namespace {
+
+constexpr int kBlock = 256;
+typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+
+// The mixed form's position map: x/h = q*2^-frac_bits - origin.
+struct PosMap {
+    double h, hinv, scale, inv;   // scale = 2^frac_bits, inv = 2^-frac_bits
+    int origin[2];
+};
+
+// One element of a line from the mixed form to FP64 bits.
+__device__ __forceinline__ unsigned long long widen(int line, unsigned v, const PosMap &m)
+{
+    if (line == kLineUtility) return v;
+    double d;
+    if (line == kLinePosX || line == kLinePosX + 1) {
+        d = ((double)v * m.inv - m.origin[line - kLinePosX]) * m.h;
+    } else {
+        d = (double)__uint_as_float(v);
+        if (line == kLineJp || line == kLineFe00 || line == kLineFe00 + 3) d += 1.0;   // stored as the difference from 1
+    }
+    return (unsigned long long)__double_as_longlong(d);
+}
+
+// And back.
+__device__ __forceinline__ unsigned narrow(int line, unsigned long long v, const PosMap &m)
+{
+    if (line == kLineUtility) return (unsigned)v;
+    double d = __longlong_as_double((long long)v);
+    if (line == kLinePosX || line == kLinePosX + 1) {
+        const double q = rint((d * m.hinv + m.origin[line - kLinePosX]) * m.scale);
+        return q > 0 ? (unsigned)fmin(q, 4294967295.0) : 0u;   // clamped to the fixed-point range (NaN: 0)
+    }
+    if (line == kLineJp || line == kLineFe00 || line == kLineFe00 + 3) d -= 1.0;
+    return __float_as_uint((float)d);
+}
+
+// Points [first, first + m) of the device lines to staging, line l at
+// l * stage_pitch; a line per blockIdx.y, two points per thread (first and
+// stage_pitch are even; a last odd point's neighbour lies in the scene's
+// capacity, which is a multiple of 256, and in the staging line).
+template <int EB>
+__global__ void __launch_bounds__(kBlock) k_export(const void *pts, long long pitch, long long first, int m,
+                                                   unsigned long long *stage, long long stage_pitch, PosMap map)
+{
+    const int i = 2 * (blockIdx.x * kBlock + threadIdx.x), line = blockIdx.y;
+    if (i >= m) return;
+    u64x2 out;
+    if (EB == 8) {
+        out = *(const u64x2 *)((const unsigned long long *)pts + line * pitch + first + i);
+    } else {
+        const u32x2 v = *(const u32x2 *)((const unsigned *)pts + line * pitch + first + i);
+        out = u64x2{widen(line, v.x, map), widen(line, v.y, map)};
+    }
+    *(u64x2 *)(stage + line * stage_pitch + i) = out;
+}
+
+template <int EB>
+__global__ void __launch_bounds__(kBlock) k_import(void *pts, long long pitch, long long first, int m,
+                                                   const unsigned long long *stage, long long stage_pitch, PosMap map)
+{
+    const int i = 2 * (blockIdx.x * kBlock + threadIdx.x), line = blockIdx.y;
+    if (i >= m) return;
+    const u64x2 v = *(const u64x2 *)(stage + line * stage_pitch + i);
+    const bool both = i + 1 < m;
+    if (EB == 8) {
+        unsigned long long *d = (unsigned long long *)pts + line * pitch + first + i;
+        if (both) *(u64x2 *)d = v;
+        else *d = v.x;
+    } else {
+        unsigned *d = (unsigned *)pts + line * pitch + first + i;
+        const u32x2 w = {narrow(line, v.x, map), narrow(line, v.y, map)};
+        if (both) *(u32x2 *)d = w;
+        else *d = w.x;
+    }
+}
+
+}  // namespace
+
+// The line copies of one transfer.  The caller declares chunk after chunk
+// ready and copies lines itself; pool threads take lines as they get a CPU.
+// Nobody waits for a helper that has not started on a line: where other
+// threads of the program keep the CPUs busy (an OpenMP pool that spins after
+// its last loop), a fixed share per helper made the upload of 410k points 5
+// times slower, and joining the helpers after the transfer 2 to 3 times.
+struct CopyJob {
+    double *stage;
+    long long chunk, n;            // points per chunk, points in all
+    int depth;
+    double *host;                  // the caller's line 0, first point
+    size_t capacity;
+    bool to_host;
+    std::atomic<long long> ready{0}, next{0};
+    std::atomic<int> left[Engine::kStageDepth];
+    std::atomic<bool> done{false};
+
+    void copy(long long k, int line) const
+    {
+        const long long at = k * chunk, m = std::min(chunk, n - at);
+        double *const s = stage + ((k % depth) * kNumPtsLines + line) * chunk, *const h = host + line * capacity + at;
+        std::memcpy(to_host ? h : s, to_host ? s : h, sizeof(double) * m);
+    }
+    // one line of a ready chunk, if there is one left
+    bool take()
+    {
+        long long i = next.load(std::memory_order_relaxed);
+        do {
+            if (i >= ready.load(std::memory_order_acquire)) return false;
+        } while (!next.compare_exchange_weak(i, i + 1, std::memory_order_acq_rel));
+        copy(i / kNumPtsLines, (int)(i % kNumPtsLines));
+        left[(i / kNumPtsLines) % depth].fetch_sub(1, std::memory_order_acq_rel);
+        return true;
+    }
+    // The caller's part: copies chunk k, the next one; returns when all of it is copied.
+    void run_chunk(long long k)
+    {
+        left[k % depth].store(kNumPtsLines, std::memory_order_relaxed);
+        ready.store((k + 1) * kNumPtsLines, std::memory_order_release);
+        while (take()) {
+        }
+        while (left[k % depth].load(std::memory_order_acquire) > 0) std::this_thread::yield();
+    }
+};
+
+// The helper threads, shared by the engines of the process and ended with the
+// last one that made a large transfer.  Asleep unless one is under way.
+class CopyPool {
+public:
+    static std::shared_ptr<CopyPool> get()
+    {
+        static std::mutex m;
+        static std::weak_ptr<CopyPool> pool;
+        std::lock_guard<std::mutex> lock(m);
+        std::shared_ptr<CopyPool> p = pool.lock();
+        if (!p) pool = p = std::make_shared<CopyPool>();
+        return p;
+    }
+    CopyPool()
+    {
+        const unsigned hw = std::thread::hardware_concurrency();
+        try {
+            for (int t = 0; t < (hw >= 8 ? 3 : hw >= 4 ? 1 : 0); t++) threads_.emplace_back([this] { work(); });
+        } catch (const std::exception &) {
+            // fewer helpers, perhaps none
+        }
+    }
+    ~CopyPool()
+    {
+        {
+            std::lock_guard<std::mutex> lock(m_);
+            stop_ = true;
+        }
+        cv_.notify_all();
+        for (auto &t : threads_) t.join();
+    }
+    void begin(const std::shared_ptr<CopyJob> &job)
+    {
+        {
+            std::lock_guard<std::mutex> lock(m_);
+            jobs_.push_back(job);
+        }
+        cv_.notify_all();
+    }
+    void end(const std::shared_ptr<CopyJob> &job)
+    {
+        job->done.store(true, std::memory_order_release);
+        std::lock_guard<std::mutex> lock(m_);
+        jobs_.remove(job);
+    }
+
+private:
+    void work()
+    {
+        std::unique_lock<std::mutex> lock(m_);
+        for (;;) {
+            cv_.wait(lock, [this] { return stop_ || !jobs_.empty(); });
+            if (stop_) return;
+            const std::shared_ptr<CopyJob> job = jobs_.front();
+            lock.unlock();
+            while (!job->done.load(std::memory_order_acquire))
+                if (!job->take()) std::this_thread::yield();
+            lock.lock();
+        }
+    }
+    std::mutex m_;
+    std::condition_variable cv_;
+    std::list<std::shared_ptr<CopyJob>> jobs_;
+    bool stop_ = false;
+    std::vector<std::thread> threads_;
+};
+
+namespace {
+
+// A job under way: known to the pool from a size on, and taken from it again
+// when the transfer ends, at whatever point.  One thread copies about 20 GB/s
+// between staging and memory that is not in its cache, three more keep up with
+// the link; waking them pays from 16 MB on.
+struct JobScope {
+    std::shared_ptr<CopyJob> job = std::make_shared<CopyJob>();
+    CopyPool *pool = nullptr;
+    void begin(std::shared_ptr<CopyPool> &engine_pool)
+    {
+        if (job->n < 128 * 1024) return;
+        if (!engine_pool) engine_pool = CopyPool::get();
+        pool = engine_pool.get();
+        pool->begin(job);
+    }
+    ~JobScope()
+    {
+        if (pool) pool->end(job);
+    }
+};
+
+// Chunks: at most 32k points (4 MB), and at least four from 16k points on, so
+// that the link and the host copies overlap.
+constexpr int kChunkMax = 32768, kChunkMin = 4096;
+long long chunk_points(long long n)
+{
+    const long long q = ((n + 3) / 4 + 255) / 256 * 256;
+    return std::min<long long>(std::max<long long>(q, kChunkMin), kChunkMax);
+}
+
+#define LAUNCH_EB(kernel, grid, ...)                                                       \
+    do {                                                                                   \
+        if (elem_bytes() == 8) hipLaunchKernelGGL(kernel<8>, grid, dim3(kBlock), 0, stream_, __VA_ARGS__); \
+        else hipLaunchKernelGGL(kernel<4>, grid, dim3(kBlock), 0, stream_, __VA_ARGS__);   \
+    } while (0)
+
+}  // namespace
+
+// Staging for a transfer of n points: `depth` chunks of `chunk` points, kept
+// for the next transfer (at most 12 MB).
+int Engine::stage_for(long long n, long long &chunk, int &depth)
+{
+    chunk = chunk_points(n);
+    depth = (int)std::min<long long>(kStageDepth, (n + chunk - 1) / chunk);
+    const size_t bytes = (size_t)chunk * depth * kNumPtsLines * sizeof(double);
+    if (bytes > stage_bytes_) {
+        if (stage_) { hipHostFree(stage_); stage_ = nullptr; }
+        stage_bytes_ = 0;
+        hipError_t e = hipHostMalloc(&stage_, bytes, 0);
+        if (e != hipSuccess) return hipfail(e, "hipHostMalloc(staging)");
+        stage_bytes_ = bytes;
+    }
+    for (int k = 0; k < depth; k++)
+        if (!stage_ev_[k]) {
+            const hipError_t e = hipEventCreateWithFlags(&stage_ev_[k], hipEventDisableTiming);
+            if (e != hipSuccess) return hipfail(e, "hipEventCreateWithFlags(staging)");
+        }
+    return ICEMPM_OK;
+}
+
+static PosMap position_map(const SceneConsts &c)
+{
+    PosMap m;
+    m.h = c.h;
+    m.hinv = c.hinv;
+    m.scale = std::ldexp(1.0, c.frac_bits);
+    m.inv = std::ldexp(1.0, -c.frac_bits);
+    m.origin[0] = c.origin;
+    m.origin[1] = c.origin_y;
+    return m;
+}
+
+int Engine::import_points(int scene, const double *hssoa, size_t capacity, long long offset, long long n)
+{
+    if (n <= 0) return ICEMPM_OK;
+    long long chunk;
+    int depth;
+    int rc = stage_for(n, chunk, depth);
+    if (rc != ICEMPM_OK) return rc;
+    const long long n_chunks = (n + chunk - 1) / chunk, first = scenes_[scene].pt_off;
+    const PosMap map = position_map(host_dev_[scene].c);
+    double *const stage = (double *)stage_;
+    hipError_t e = hipSuccess;
+    {
+        JobScope scope;
+        CopyJob &job = *scope.job;
+        job.stage = stage;
+        job.chunk = chunk;
+        job.n = n;
+        job.depth = depth;
+        job.host = const_cast<double *>(hssoa) + offset;   // read only: to_host is false
+        job.capacity = capacity;
+        job.to_host = false;
+        scope.begin(copy_pool_);
+        for (long long k = 0; k < n_chunks && e == hipSuccess; k++) {
+            const int slot = (int)(k % depth);
+            if (k >= depth) e = hipEventSynchronize(stage_ev_[slot]);   // the kernel that read this slot
+            if (e != hipSuccess) break;
+            job.run_chunk(k);
+            const int m = (int)std::min(chunk, n - k * chunk);
+            LAUNCH_EB(k_import, dim3((m + 2 * kBlock - 1) / (2 * kBlock), kNumPtsLines), pts_[0], pitch_,
+                      first + k * chunk, m, (const unsigned long long *)(stage + slot * chunk * kNumPtsLines), chunk, map);
+            e = hipGetLastError();
+            if (e == hipSuccess && n_chunks > depth) e = hipEventRecord(stage_ev_[slot], stream_);
+        }
+    }
+    const hipError_t es = hipStreamSynchronize(stream_);   // the staging is read
+    if (e == hipSuccess) e = es;
+    return e == hipSuccess ? ICEMPM_OK : hipfail(e, "point upload");
+}
+
+int Engine::export_points(int scene, double *hssoa, size_t capacity, long long offset, long long n)
+{
+    if (n <= 0) {
+        const hipError_t e = hipStreamSynchronize(stream_);
+        return e == hipSuccess ? ICEMPM_OK : hipfail(e, "point download");
+    }
+    long long chunk;
+    int depth;
+    int rc = stage_for(n, chunk, depth);
+    if (rc != ICEMPM_OK) return rc;
+    const long long n_chunks = (n + chunk - 1) / chunk, first = scenes_[scene].pt_off;
+    const PosMap map = position_map(host_dev_[scene].c);
+    double *const stage = (double *)stage_;
+    auto launch = [&](long long k) {
+        const int slot = (int)(k % depth), m = (int)std::min(chunk, n - k * chunk);
+        LAUNCH_EB(k_export, dim3((m + 2 * kBlock - 1) / (2 * kBlock), kNumPtsLines), (const void *)pts_[0], pitch_,
+                  first + k * chunk, m, (unsigned long long *)(stage + slot * chunk * kNumPtsLines), chunk, map);
+        hipError_t e = hipGetLastError();
+        if (e == hipSuccess) e = hipEventRecord(stage_ev_[slot], stream_);
+        return e;
+    };
+    hipError_t e = hipSuccess;
+    for (long long k = 0; k < depth && e == hipSuccess; k++) e = launch(k);
+    if (e == hipSuccess) {
+        JobScope scope;
+        CopyJob &job = *scope.job;
+        job.stage = stage;
+        job.chunk = chunk;
+        job.n = n;
+        job.depth = depth;
+        job.host = hssoa + offset;
+        job.capacity = capacity;
+        job.to_host = true;
+        scope.begin(copy_pool_);
+        for (long long k = 0; k < n_chunks; k++) {
+            if ((e = hipEventSynchronize(stage_ev_[k % depth])) != hipSuccess) break;
+            job.run_chunk(k);
+            if (k + depth < n_chunks && (e = launch(k + depth)) != hipSuccess) break;
+        }
+    }
+    const hipError_t es = hipStreamSynchronize(stream_);
+    if (e == hipSuccess) e = es;
+    return e == hipSuccess ? ICEMPM_OK : hipfail(e, "point download");
+}
+
+}  // namespace icempm
