@@ -26,6 +26,10 @@ namespace fp64 {
 hipError_t launch_tiles(const StepArgs &a, int mode, int rbuf, int wbuf, int zbuf, int record_mode, hipStream_t s);
 hipError_t launch_p2g_direct(const StepArgs &a, int scene, int n_pts, int wbuf, hipStream_t s);
 hipError_t launch_g2p_direct(const StepArgs &a, int scene, int n_pts, int rbuf, int record_pq, hipStream_t s);
+// One substep of a scene's points in their own order: grid update folded in,
+// G2P from grid[rbuf]'s momenta and, with next, P2G into grid[wbuf]; clears
+// grid[zbuf].  a.n_work: workgroups of 256 points.
+hipError_t launch_points(const StepArgs &a, int scene, bool next, int rbuf, int wbuf, int zbuf, hipStream_t s);
 // Grid update of both precision forms: their grids share one layout (3 FP64
 // lines per buffer) and the update works in FP64.
 hipError_t launch_update(const StepArgs &a, int buf, int zero_other, int advance_clock, int n_blocks, hipStream_t s);

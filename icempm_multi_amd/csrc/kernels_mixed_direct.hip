@@ -1,40 +1,44 @@
 // kernels_mixed_direct.hip -- unbinned mixed-precision P2G and G2P (one thread
-// per point; P2G adds every contribution with FP64 global atomics).  Separate
-// translation unit for the same compiler reason as kernels_fp64_direct.hip.
+// per point).  Separate translation unit for the same compiler reason as
+// kernels_fp64_direct.hip.
 #include <hip/hip_runtime.h>
 
+#include "block_window.h"
 #include "point_mixed.h"
 
 namespace icempm {
 namespace mixed {
 
+// P2G summed in LDS per workgroup, as in the FP64 form.
 __global__ void __launch_bounds__(kBlock) k_p2g_direct(StepArgs a, int scene, int wbuf)
 {
     const SceneDev &S = a.scenes[scene];
     const SceneConsts c = uniform_copy(S.c);
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= S.n_pts) return;
+    const int i = blockIdx.x * kBlock + spread_point(threadIdx.x);
     const long long pt = S.pt_off + i;
     const PtRef R{(unsigned *)a.pts, a.pitch};
-    const unsigned ud = R.u(kLineUtility, pt);
-    if (ud & (unsigned)kDisabled) return;
+    unsigned ud = (unsigned)kDisabled;
+    if (i < S.n_pts) ud = R.u(kLineUtility, pt);
+    bool have = !(ud & (unsigned)kDisabled);
     const ConstsF cf = to_float(c);
-    unsigned xq, yq;
-    float D[4], Jm1, v[2], C[4];
-    load_state(R, pt, xq, yq, D, Jm1);
-    v[0] = R.f(kLineVelX, pt);
-    v[1] = R.f(kLineVelX + 1, pt);
+    P2GStencil st;
+    if (have) {
+        unsigned xq, yq;
+        float D[4], Jm1, v[2], C[4];
+        load_state(R, pt, xq, yq, D, Jm1);
+        v[0] = R.f(kLineVelX, pt);
+        v[1] = R.f(kLineVelX + 1, pt);
 #pragma unroll
-    for (int m = 0; m < 4; m++) C[m] = R.f(kLineBp00 + m, pt);
-    glb_d *gw = (glb_d *)(a.grid_mem + S.grid_off[wbuf]);
-    const long long gp = S.gpitch;
-    const int gridY = c.gridY;
-    const unsigned e = p2g_point(c, cf, xq, yq, v, C, D, Jm1, ud, [&](int col, int row, double dm, double dpx, double dpy) {
-        const long long gi = (long long)col * gridY + row;
-        grid_add(gw, gp, gi, dm, dpx, dpy);
-        mark_dirty(a, S, wbuf, gi);
-    });
-    if (e) atomicMax(&a.err[scene], e);
+        for (int m = 0; m < 4; m++) C[m] = R.f(kLineBp00 + m, pt);
+        StressTerms none;
+        none.valid = false;
+        const unsigned e = p2g_stencil(c, cf, xq, yq, v, C, D, Jm1, ud, none, st);
+        if (e) {
+            atomicMax(&a.err[scene], e);
+            have = false;
+        }
+    }
+    block_p2g(a, S, c.gridY, wbuf, have, st.bxc, st.by, [&](auto &&sink) { st.nodes(cf, sink); });
 }
 
 __global__ void __launch_bounds__(kBlock) k_g2p_direct(StepArgs a, int scene, int rbuf, int record)

@@ -10,9 +10,11 @@
 // largest part is the grid, so scenes are limited to kNoAllocMaxNodes nodes.
 //
 // The substeps are those of icempm_partition_step with ICEMPM_STEP_DIRECT_P2G
-// (unbinned P2G and G2P, one thread per point, the reference's launch shape):
-// per substep the grid is cleared, P2G scatters with global atomics, the grid
-// update advances the clock, G2P gathers.  The same kernels run.
+// (one thread per point, the points in the caller's order).  Where three grids
+// fit the array, as for most scenes of that size, a substep is one launch
+// (launch_points): it reads one grid's momenta, accumulates into the second
+// and clears the third.  Larger grids take the separate launches: the grid is
+// cleared, P2G, the grid update advances the clock, G2P.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -36,7 +38,7 @@ constexpr size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 // parts of the array, each 256-byte aligned
 constexpr size_t kOffGrid = 0;
 constexpr size_t kOffFlags = kOffGrid + align256(3 * kNoAllocMaxNodes * sizeof(double));
-constexpr size_t kOffRuns = kOffFlags + align256(2 * kNoAllocMaxSegs * sizeof(int));
+constexpr size_t kOffRuns = kOffFlags + align256((kNoAllocMaxSegs + 3) * sizeof(int));   // of one grid, or of three
 constexpr size_t kOffScene = kOffRuns + align256(kNoAllocMaxRuns * sizeof(NodeChunk));
 constexpr size_t kOffClocks = kOffScene + align256(sizeof(SceneDev));
 constexpr size_t kOffErr = kOffClocks + align256(2 * sizeof(SceneClock));
@@ -181,8 +183,7 @@ int icempm_substeps_noalloc(int device, const icempm_simparams *prms, size_t prm
     } restore{prev};
     hipStream_t s = (hipStream_t)stream;
 
-    // the scene: one, at point 0, with both grid buffers on the one grid
-    // (the unbinned pipeline reads and writes buffer 0 only)
+    // the scene: one, at point 0
     const long long gpitch = (nodes + kSegNodes - 1) / kSegNodes * kSegNodes;
     const int n_segs = (int)(gpitch >> kSegShift);
     const int run_len = update_run_length(gpitch);
@@ -194,7 +195,9 @@ int icempm_substeps_noalloc(int device, const icempm_simparams *prms, size_t prm
     d.pt_off = 0;
     d.n_pts = n_points;
     d.cap_pts = (int)pitch;
-    d.grid_off[0] = d.grid_off[1] = 0;
+    const long long grid_bytes = 3 * gpitch * (long long)sizeof(double);
+    const bool three = 3 * gpitch <= kNoAllocMaxNodes;
+    for (int b = 0; b < 3; b++) d.grid_off[b] = three ? b * grid_bytes : 0;
     d.gpitch = gpitch;
     d.ncells = (int)nodes;
     d.force_off = 0;
@@ -237,7 +240,22 @@ int icempm_substeps_noalloc(int device, const icempm_simparams *prms, size_t prm
     }
     const int upd_blocks = std::max(1, std::min((n_runs + 3) / 4, n_cus * 8));
     int cs = 0;
-    for (int k = 0; k < n_substeps; k++) {
+    if (three && n_points > 0) {
+        a.grid_buf_bytes = grid_bytes;
+        a.n_work = (n_points + 255) / 256;
+        a.n_service = d.c.ind_rsq > 0 ? 1 : 0;
+        a.n_clear = std::max(1, std::min((n_runs + 3) / 4, n_cus * 8));
+        NA_HIPCHK(launch_fill_zero(base + kOffGrid, (size_t)3 * grid_bytes, s));
+        NA_HIPCHK(launch_fill_zero(d_flags, sizeof(int) * 3 * n_segs, s));
+        NA_HIPCHK(fp64::launch_p2g_direct(a, 0, n_points, 0, s));
+        for (int k = 0; k < n_substeps; k++) {
+            a.clocks = d_clocks + cs;
+            a.clocks_next = d_clocks + (cs ^ 1);
+            NA_HIPCHK(fp64::launch_points(a, 0, k + 1 < n_substeps, k % 3, (k + 1) % 3, (k + 2) % 3, s));
+            cs ^= 1;
+        }
+    }
+    for (int k = 0; k < n_substeps && !(three && n_points > 0); k++) {
         StepArgs au = a, an = a;
         au.clocks = d_clocks + cs;         // the update reads this slot and writes the next clock to the other
         au.clocks_next = d_clocks + (cs ^ 1);

@@ -237,22 +237,6 @@ __device__ __forceinline__ unsigned p2g_stencil(const SceneConsts &c, double x, 
     return 0;
 }
 
-// P2G contributions of one point.  Calls sink(col, row, dm, dpx, dpy) for
-// the 9 stencil nodes; returns the error byte (0 = ok).
-template <class Sink>
-__device__ __forceinline__ unsigned p2g_point(const SceneConsts &c, double x, double y, const double v[2],
-                                              const double B[4], const double F[4], double Jp, long long ud,
-                                              Sink &&sink)
-{
-    P2GStencil st;
-    StressTerms none;
-    none.valid = false;
-    const unsigned e = p2g_stencil(c, x, y, v, B, F, Jp, ud, none, st);
-    if (e) return e;
-    st.nodes(c, [&](int i, int j, double dm, double dpx, double dpy) { sink(st.bxc + i, st.by + j, dm, dpx, dpy); });
-    return 0;
-}
-
 __device__ __forceinline__ void load_state(const PtRef &R, long long pt, double &x, double &y, double F[4],
                                            double &Jp)
 {

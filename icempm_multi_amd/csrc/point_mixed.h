@@ -307,21 +307,6 @@ __device__ __forceinline__ unsigned p2g_stencil(const SceneConsts &c, const Cons
     return 0;
 }
 
-// P2G contributions of one point; calls sink(col, row, dm, dpx, dpy) (FP64 terms).
-template <class Sink>
-__device__ __forceinline__ unsigned p2g_point(const SceneConsts &c, const ConstsF &cf, unsigned xq, unsigned yq,
-                                              const float v[2], const float C[4], const float D[4], float Jm1,
-                                              unsigned ud, Sink &&sink)
-{
-    P2GStencil st;
-    StressTerms none;
-    none.valid = false;
-    const unsigned e = p2g_stencil(c, cf, xq, yq, v, C, D, Jm1, ud, none, st);
-    if (e) return e;
-    st.nodes(cf, [&](int i, int j, double dm, double dpx, double dpy) { sink(st.bxc + i, st.by + j, dm, dpx, dpy); });
-    return 0;
-}
-
 __device__ __forceinline__ void load_state(const PtRef &R, long long pt, unsigned &xq, unsigned &yq, float D[4],
                                            float &Jm1)
 {

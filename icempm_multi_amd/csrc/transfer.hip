@@ -248,12 +248,12 @@ struct JobScope {
     }
 };
 
-// Chunks: at most 32k points (4 MB), and at least four from 16k points on, so
-// that the link and the host copies overlap.
+// Chunks: at most 32k points (4 MB), and eight from 32k points on, so that the
+// link and the host copies overlap and the staging of a small scene is small.
 constexpr int kChunkMax = 32768, kChunkMin = 4096;
 long long chunk_points(long long n)
 {
-    const long long q = ((n + 3) / 4 + 255) / 256 * 256;
+    const long long q = ((n + 7) / 8 + 255) / 256 * 256;
     return std::min<long long>(std::max<long long>(q, kChunkMin), kChunkMax);
 }
 
