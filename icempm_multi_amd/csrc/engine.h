@@ -57,12 +57,11 @@ struct SceneHost {
     int sim_step = 0;         // SimulationStep
 };
 
-class CopyPool;   // transfer.hip
+class TransferPool;   // transfer.hip
 
 class Engine {
 public:
     // Units of a substep call (see emit_units in engine.hip).
-    static constexpr int kStageDepth = 3;   // chunks in flight of a point transfer
     enum UnitKind { kUnitHead = 0, kUnitChain, kUnitTail, kUnitUnfused, kUnitDirect };
 
     Engine(int device, int precision);
@@ -128,7 +127,7 @@ private:
     int push_clocks();
     int build_tiles();
     // points between a HostSideSOA buffer and the device, through pinned staging
-    int stage_for(long long n, long long &chunk, int &depth);
+    const std::shared_ptr<TransferPool> &transfer_pool();
     int import_points(int scene, const double *hssoa, size_t capacity, long long offset, long long n);
     int export_points(int scene, double *hssoa, size_t capacity, long long offset, long long n);
     int alloc_bins();
@@ -187,11 +186,7 @@ private:
     int n_chunks_ = 0;
     int n_service_ = 0;            // workgroups for the indenter force in a substep launch
 
-    // pinned staging of the point transfers, and the threads that help with large ones
-    std::shared_ptr<CopyPool> copy_pool_;
-    void *stage_ = nullptr;
-    size_t stage_bytes_ = 0;
-    hipEvent_t stage_ev_[kStageDepth] = {nullptr, nullptr, nullptr};
+    std::shared_ptr<TransferPool> transfer_pool_;   // staging and helper threads, from the first transfer on
 
     // binning
     BinWork bins_{};

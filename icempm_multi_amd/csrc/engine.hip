@@ -69,9 +69,6 @@ Engine::~Engine()
                     bin_mem_, tile_mem_, d_tile_queue_, d_dirty_, d_defer_};
     for (void *b : bufs)
         if (b) hipFree(b);
-    if (stage_) hipHostFree(stage_);
-    for (hipEvent_t e : stage_ev_)
-        if (e) hipEventDestroy(e);
     if (stream_) hipStreamDestroy(stream_);
 }
 

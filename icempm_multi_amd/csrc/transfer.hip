@@ -36,6 +36,7 @@ namespace icempm {
 namespace {
 
 constexpr int kBlock = 256;
+constexpr int kStageDepth = 3;   // chunks in flight of a transfer
 typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
@@ -114,6 +115,22 @@ __global__ void __launch_bounds__(kBlock) k_import(void *pts, long long pitch, l
 
 }  // namespace
 
+// Pinned memory for the chunks in flight of one transfer, and an event per
+// chunk, of one device.
+struct Staging {
+    int device = 0;
+    double *mem = nullptr;
+    size_t bytes = 0;
+    hipEvent_t ev[kStageDepth] = {nullptr, nullptr, nullptr};
+
+    ~Staging()
+    {
+        if (mem) hipHostFree(mem);
+        for (hipEvent_t e : ev)
+            if (e) hipEventDestroy(e);
+    }
+};
+
 // The line copies of one transfer.  The caller declares chunk after chunk
 // ready and copies lines itself; pool threads take lines as they get a CPU.
 // Nobody waits for a helper that has not started on a line: where other
@@ -128,7 +145,7 @@ struct CopyJob {
     size_t capacity;
     bool to_host;
     std::atomic<long long> ready{0}, next{0};
-    std::atomic<int> left[Engine::kStageDepth];
+    std::atomic<int> left[kStageDepth];
     std::atomic<bool> done{false};
 
     void copy(long long k, int line) const
@@ -159,29 +176,23 @@ struct CopyJob {
     }
 };
 
-// The helper threads, shared by the engines of the process and ended with the
-// last one that made a large transfer.  Asleep unless one is under way.
-class CopyPool {
+// What the engines of the process share for their transfers, freed with the
+// last engine that made one: the staging memory (making and freeing it per
+// engine cost 0.8 ms each; a transfer takes a piece of its own for its time,
+// and at most kIdleMost idle ones of at most 12 MB are kept) and the helper
+// threads (started by the first large transfer, asleep unless one is under way).
+class TransferPool {
 public:
-    static std::shared_ptr<CopyPool> get()
+    static std::shared_ptr<TransferPool> get()
     {
         static std::mutex m;
-        static std::weak_ptr<CopyPool> pool;
+        static std::weak_ptr<TransferPool> pool;
         std::lock_guard<std::mutex> lock(m);
-        std::shared_ptr<CopyPool> p = pool.lock();
-        if (!p) pool = p = std::make_shared<CopyPool>();
+        std::shared_ptr<TransferPool> p = pool.lock();
+        if (!p) pool = p = std::make_shared<TransferPool>();
         return p;
     }
-    CopyPool()
-    {
-        const unsigned hw = std::thread::hardware_concurrency();
-        try {
-            for (int t = 0; t < (hw >= 8 ? 3 : hw >= 4 ? 1 : 0); t++) threads_.emplace_back([this] { work(); });
-        } catch (const std::exception &) {
-            // fewer helpers, perhaps none
-        }
-    }
-    ~CopyPool()
+    ~TransferPool()
     {
         {
             std::lock_guard<std::mutex> lock(m_);
@@ -190,10 +201,50 @@ public:
         cv_.notify_all();
         for (auto &t : threads_) t.join();
     }
+    // Staging of at least `bytes` on the current device; null and e set if there is none to be had.
+    std::unique_ptr<Staging> take(int device, size_t bytes, hipError_t &e)
+    {
+        {
+            std::lock_guard<std::mutex> lock(m_);
+            for (auto it = idle_.begin(); it != idle_.end(); ++it)
+                if ((*it)->device == device && (*it)->bytes >= bytes) {
+                    std::unique_ptr<Staging> st = std::move(*it);
+                    idle_.erase(it);
+                    return st;
+                }
+        }
+        std::unique_ptr<Staging> st(new Staging);
+        st->device = device;
+        if ((e = hipHostMalloc((void **)&st->mem, bytes, hipHostMallocPortable)) != hipSuccess) return nullptr;
+        st->bytes = bytes;
+        for (hipEvent_t &ev : st->ev)
+            if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return nullptr;
+        return st;
+    }
+    void give_back(std::unique_ptr<Staging> st)
+    {
+        std::unique_ptr<Staging> least;   // freed outside the lock
+        std::lock_guard<std::mutex> lock(m_);
+        idle_.push_back(std::move(st));
+        if (idle_.size() > kIdleMost) {
+            auto it = std::min_element(idle_.begin(), idle_.end(),
+                                       [](const auto &x, const auto &y) { return x->bytes < y->bytes; });
+            least = std::move(*it);
+            idle_.erase(it);
+        }
+    }
     void begin(const std::shared_ptr<CopyJob> &job)
     {
         {
             std::lock_guard<std::mutex> lock(m_);
+            if (threads_.empty()) {
+                const unsigned hw = std::thread::hardware_concurrency();
+                try {
+                    for (int t = 0; t < (hw >= 8 ? 3 : hw >= 4 ? 1 : 0); t++) threads_.emplace_back([this] { work(); });
+                } catch (const std::exception &) {
+                    // fewer helpers, perhaps none
+                }
+            }
             jobs_.push_back(job);
         }
         cv_.notify_all();
@@ -219,8 +270,10 @@ private:
             lock.lock();
         }
     }
+    static constexpr size_t kIdleMost = 4;
     std::mutex m_;
     std::condition_variable cv_;
+    std::list<std::unique_ptr<Staging>> idle_;
     std::list<std::shared_ptr<CopyJob>> jobs_;
     bool stop_ = false;
     std::vector<std::thread> threads_;
@@ -228,23 +281,32 @@ private:
 
 namespace {
 
-// A job under way: known to the pool from a size on, and taken from it again
-// when the transfer ends, at whatever point.  One thread copies about 20 GB/s
-// between staging and memory that is not in its cache, three more keep up with
-// the link; waking them pays from 16 MB on.
-struct JobScope {
+// A transfer under way: its staging, and its job, known to the pool's helpers
+// from a size on.  Ends at whatever point its scope is left: the stream has
+// read or written the staging before it is given back.
+// One thread copies about 20 GB/s between staging and memory that is not in
+// its cache, three more keep up with the link; waking them pays from 16 MB on.
+struct Transfer {
+    std::shared_ptr<TransferPool> pool;
+    hipStream_t stream;
+    std::unique_ptr<Staging> st;
     std::shared_ptr<CopyJob> job = std::make_shared<CopyJob>();
-    CopyPool *pool = nullptr;
-    void begin(std::shared_ptr<CopyPool> &engine_pool)
+    bool helped = false;
+
+    Transfer(std::shared_ptr<TransferPool> p, hipStream_t s) : pool(std::move(p)), stream(s) {}
+    void begin()
     {
         if (job->n < 128 * 1024) return;
-        if (!engine_pool) engine_pool = CopyPool::get();
-        pool = engine_pool.get();
         pool->begin(job);
+        helped = true;
     }
-    ~JobScope()
+    ~Transfer()
     {
-        if (pool) pool->end(job);
+        if (helped) pool->end(job);
+        if (st) {
+            hipStreamSynchronize(stream);
+            pool->give_back(std::move(st));
+        }
     }
 };
 
@@ -265,28 +327,6 @@ long long chunk_points(long long n)
 
 }  // namespace
 
-// Staging for a transfer of n points: `depth` chunks of `chunk` points, kept
-// for the next transfer (at most 12 MB).
-int Engine::stage_for(long long n, long long &chunk, int &depth)
-{
-    chunk = chunk_points(n);
-    depth = (int)std::min<long long>(kStageDepth, (n + chunk - 1) / chunk);
-    const size_t bytes = (size_t)chunk * depth * kNumPtsLines * sizeof(double);
-    if (bytes > stage_bytes_) {
-        if (stage_) { hipHostFree(stage_); stage_ = nullptr; }
-        stage_bytes_ = 0;
-        hipError_t e = hipHostMalloc(&stage_, bytes, 0);
-        if (e != hipSuccess) return hipfail(e, "hipHostMalloc(staging)");
-        stage_bytes_ = bytes;
-    }
-    for (int k = 0; k < depth; k++)
-        if (!stage_ev_[k]) {
-            const hipError_t e = hipEventCreateWithFlags(&stage_ev_[k], hipEventDisableTiming);
-            if (e != hipSuccess) return hipfail(e, "hipEventCreateWithFlags(staging)");
-        }
-    return ICEMPM_OK;
-}
-
 static PosMap position_map(const SceneConsts &c)
 {
     PosMap m;
@@ -302,36 +342,29 @@ static PosMap position_map(const SceneConsts &c)
 int Engine::import_points(int scene, const double *hssoa, size_t capacity, long long offset, long long n)
 {
     if (n <= 0) return ICEMPM_OK;
-    long long chunk;
-    int depth;
-    int rc = stage_for(n, chunk, depth);
-    if (rc != ICEMPM_OK) return rc;
-    const long long n_chunks = (n + chunk - 1) / chunk, first = scenes_[scene].pt_off;
-    const PosMap map = position_map(host_dev_[scene].c);
-    double *const stage = (double *)stage_;
     hipError_t e = hipSuccess;
-    {
-        JobScope scope;
-        CopyJob &job = *scope.job;
-        job.stage = stage;
-        job.chunk = chunk;
-        job.n = n;
-        job.depth = depth;
-        job.host = const_cast<double *>(hssoa) + offset;   // read only: to_host is false
-        job.capacity = capacity;
-        job.to_host = false;
-        scope.begin(copy_pool_);
-        for (long long k = 0; k < n_chunks && e == hipSuccess; k++) {
-            const int slot = (int)(k % depth);
-            if (k >= depth) e = hipEventSynchronize(stage_ev_[slot]);   // the kernel that read this slot
-            if (e != hipSuccess) break;
-            job.run_chunk(k);
-            const int m = (int)std::min(chunk, n - k * chunk);
-            LAUNCH_EB(k_import, dim3((m + 2 * kBlock - 1) / (2 * kBlock), kNumPtsLines), pts_[0], pitch_,
-                      first + k * chunk, m, (const unsigned long long *)(stage + slot * chunk * kNumPtsLines), chunk, map);
-            e = hipGetLastError();
-            if (e == hipSuccess && n_chunks > depth) e = hipEventRecord(stage_ev_[slot], stream_);
-        }
+    Transfer t(transfer_pool(), stream_);
+    CopyJob &job = *t.job;
+    job.n = n;
+    job.chunk = chunk_points(n);
+    job.host = const_cast<double *>(hssoa) + offset;   // read only: to_host is false
+    job.capacity = capacity;
+    job.to_host = false;
+    const long long chunk = job.chunk, n_chunks = (n + chunk - 1) / chunk, first = scenes_[scene].pt_off;
+    const int depth = job.depth = (int)std::min<long long>(kStageDepth, n_chunks);
+    t.st = t.pool->take(device_, (size_t)chunk * depth * kNumPtsLines * sizeof(double), e);
+    if (!t.st) return hipfail(e, "transfer staging");
+    job.stage = t.st->mem;
+    const PosMap map = position_map(host_dev_[scene].c);
+    t.begin();
+    for (long long k = 0; k < n_chunks && e == hipSuccess; k++) {
+        const int slot = (int)(k % depth), m = (int)std::min(chunk, n - k * chunk);
+        if (k >= depth && (e = hipEventSynchronize(t.st->ev[slot])) != hipSuccess) break;   // read by its kernel
+        job.run_chunk(k);
+        LAUNCH_EB(k_import, dim3((m + 2 * kBlock - 1) / (2 * kBlock), kNumPtsLines), pts_[0], pitch_, first + k * chunk,
+                  m, (const unsigned long long *)(job.stage + slot * chunk * kNumPtsLines), chunk, map);
+        e = hipGetLastError();
+        if (e == hipSuccess && n_chunks > depth) e = hipEventRecord(t.st->ev[slot], stream_);
     }
     const hipError_t es = hipStreamSynchronize(stream_);   // the staging is read
     if (e == hipSuccess) e = es;
@@ -340,47 +373,47 @@ int Engine::import_points(int scene, const double *hssoa, size_t capacity, long 
 
 int Engine::export_points(int scene, double *hssoa, size_t capacity, long long offset, long long n)
 {
+    hipError_t e = hipSuccess;
     if (n <= 0) {
-        const hipError_t e = hipStreamSynchronize(stream_);
+        e = hipStreamSynchronize(stream_);
         return e == hipSuccess ? ICEMPM_OK : hipfail(e, "point download");
     }
-    long long chunk;
-    int depth;
-    int rc = stage_for(n, chunk, depth);
-    if (rc != ICEMPM_OK) return rc;
-    const long long n_chunks = (n + chunk - 1) / chunk, first = scenes_[scene].pt_off;
+    Transfer t(transfer_pool(), stream_);
+    CopyJob &job = *t.job;
+    job.n = n;
+    job.chunk = chunk_points(n);
+    job.host = hssoa + offset;
+    job.capacity = capacity;
+    job.to_host = true;
+    const long long chunk = job.chunk, n_chunks = (n + chunk - 1) / chunk, first = scenes_[scene].pt_off;
+    const int depth = job.depth = (int)std::min<long long>(kStageDepth, n_chunks);
+    t.st = t.pool->take(device_, (size_t)chunk * depth * kNumPtsLines * sizeof(double), e);
+    if (!t.st) return hipfail(e, "transfer staging");
+    job.stage = t.st->mem;
     const PosMap map = position_map(host_dev_[scene].c);
-    double *const stage = (double *)stage_;
     auto launch = [&](long long k) {
         const int slot = (int)(k % depth), m = (int)std::min(chunk, n - k * chunk);
         LAUNCH_EB(k_export, dim3((m + 2 * kBlock - 1) / (2 * kBlock), kNumPtsLines), (const void *)pts_[0], pitch_,
-                  first + k * chunk, m, (unsigned long long *)(stage + slot * chunk * kNumPtsLines), chunk, map);
-        hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = hipEventRecord(stage_ev_[slot], stream_);
-        return e;
+                  first + k * chunk, m, (unsigned long long *)(job.stage + slot * chunk * kNumPtsLines), chunk, map);
+        const hipError_t el = hipGetLastError();
+        return el == hipSuccess ? hipEventRecord(t.st->ev[slot], stream_) : el;
     };
-    hipError_t e = hipSuccess;
     for (long long k = 0; k < depth && e == hipSuccess; k++) e = launch(k);
-    if (e == hipSuccess) {
-        JobScope scope;
-        CopyJob &job = *scope.job;
-        job.stage = stage;
-        job.chunk = chunk;
-        job.n = n;
-        job.depth = depth;
-        job.host = hssoa + offset;
-        job.capacity = capacity;
-        job.to_host = true;
-        scope.begin(copy_pool_);
-        for (long long k = 0; k < n_chunks; k++) {
-            if ((e = hipEventSynchronize(stage_ev_[k % depth])) != hipSuccess) break;
-            job.run_chunk(k);
-            if (k + depth < n_chunks && (e = launch(k + depth)) != hipSuccess) break;
-        }
+    if (e == hipSuccess) t.begin();
+    for (long long k = 0; k < n_chunks && e == hipSuccess; k++) {
+        if ((e = hipEventSynchronize(t.st->ev[k % depth])) != hipSuccess) break;
+        job.run_chunk(k);
+        if (k + depth < n_chunks) e = launch(k + depth);
     }
     const hipError_t es = hipStreamSynchronize(stream_);
     if (e == hipSuccess) e = es;
     return e == hipSuccess ? ICEMPM_OK : hipfail(e, "point download");
+}
+
+const std::shared_ptr<TransferPool> &Engine::transfer_pool()
+{
+    if (!transfer_pool_) transfer_pool_ = TransferPool::get();
+    return transfer_pool_;
 }
 
 }  // namespace icempm
