@@ -137,6 +137,7 @@ private:
     int apply_tile_shape(int tx, int ty, int margin);
     int choose_tile_shape();
     StepArgs args() const;
+    StepArgs scene_runs(int scene, int &n_runs) const;
     // timed: record hipEvents around the launches of every sample-th substep
     int launch_substeps(int nsub, int start_buf, bool fused, bool direct, bool timed, int sample = 1);
     struct GraphExec;

@@ -779,10 +779,31 @@ int Engine::zero_grid(int scene, int buf)
 int Engine::reset_grid(int scene)
 {
     RC(ensure_committed());
+    int n_runs = 0;
+    const StepArgs a = scene_runs(scene, n_runs);
     timed_begin(true);
-    const int rc = zero_grid(scene, 0);
+    HIPCHK(fp64::launch_clear(a, 0, update_blocks(n_runs), stream_));
     timed_end(true, kClsZero);
-    return rc;
+    scenes_[scene].clean[0] = true;
+    return ICEMPM_OK;
+}
+
+// The launch arguments with the run table narrowed to one scene's runs (the
+// table is scene-major).
+StepArgs Engine::scene_runs(int scene, int &n_runs) const
+{
+    long long first = 0;
+    for (int i = 0;; i++) {
+        const long long nseg = scenes_[i].grid_elems >> kSegShift;
+        const int len = update_run_length(scenes_[i].grid_elems);
+        n_runs = (int)((nseg + len - 1) / len);
+        if (i == scene) break;
+        first += n_runs;
+    }
+    StepArgs a = args();
+    a.chunks = d_chunks_ + first;
+    a.n_chunks = n_runs;
+    return a;
 }
 
 int Engine::p2g(int scene)
@@ -809,28 +830,11 @@ int Engine::update_nodes(int scene, double t, double ind_x, double ind_y)
     ck.ind_y = ind_y;
     ck.step = scenes_[scene].sim_step;
     ck.next_step = scenes_[scene].sim_step;
-    HIPCHK(hipMemcpyAsync(d_clocks_ + clock_slot_ * nscenes() + scene, &ck, sizeof ck, hipMemcpyHostToDevice,
-                          stream_));
-    StepArgs a = args();
-    // only this scene's chunks: the chunk table is scene-major
-    const NodeChunk *first = nullptr;
-    int nchunks = 0;
-    {
-        long long k = 0;
-        for (int i = 0; i < nscenes(); i++) {
-            const long long nseg = scenes_[i].grid_elems >> kSegShift;
-            const int len = update_run_length(scenes_[i].grid_elems);
-            const int nc = (int)((nseg + len - 1) / len);
-            if (i == scene) { first = d_chunks_ + k; nchunks = nc; }
-            k += nc;
-        }
-    }
-    a.chunks = first;
-    a.n_chunks = nchunks;
+    int n_runs = 0;
+    const StepArgs a = scene_runs(scene, n_runs);
     timed_begin(true);
-    HIPCHK(fp64::launch_update(a, 0, 0, 0, update_blocks(nchunks), stream_));
+    HIPCHK(fp64::launch_update_at(a, 0, ck, d_clocks_ + clock_slot_ * nscenes() + scene, update_blocks(n_runs), stream_));
     timed_end(true, kClsUpdate);
-    HIPCHK(hipStreamSynchronize(stream_));   // ck lives on this stack frame
     return ICEMPM_OK;
 }
 

@@ -33,6 +33,9 @@ hipError_t launch_points(const StepArgs &a, int scene, bool next, int rbuf, int 
 // Grid update of both precision forms: their grids share one layout (3 FP64
 // lines per buffer) and the update works in FP64.
 hipError_t launch_update(const StepArgs &a, int buf, int zero_other, int advance_clock, int n_blocks, hipStream_t s);
+hipError_t launch_update_at(StepArgs a, int buf, const SceneClock &clock, SceneClock *slot, int n_blocks,
+                            hipStream_t s);
+hipError_t launch_clear(const StepArgs &a, int buf, int n_blocks, hipStream_t s);
 size_t tile_lds_bytes(const StepArgs &a, int mode);
 // Workgroups of the tile kernel for this mode and window that one CU holds at
 // once (registers and LDS); 0 if the runtime cannot tell.

@@ -8,6 +8,7 @@
 
 #include "kernels.h"
 #include "point_fp64.h"
+#include "tile_common.h"
 
 namespace icempm {
 namespace fp64 {
@@ -18,8 +19,10 @@ namespace fp64 {
 // accumulation grid for the next P2G; with advance_clock set it computes the
 // substep's clock from the current slot and block 0 writes it to the next.
 // ---------------------------------------------------------------------------
+// With a.clocks null (the phase call) the clock of its one scene is `given`,
+// and goes into a.clocks_next.
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) k_update(StepArgs a, int buf, int zero_other,
-                                                                                            int advance_clock)
+                                                                                            int advance_clock, SceneClock given)
 {
     // A wave takes a run of up to 64 node segments: lane l loads the flags of
     // segment l of the run for both buffers, a ballot gives the flagged ones.
@@ -33,7 +36,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))
         const NodeChunk run = uniform_copy(a.chunks[r]);
         const SceneDev &S = a.scenes[run.scene];
         const SceneConsts c = uniform_copy(S.c);
-        SceneClock clk = uniform_copy(a.clocks[run.scene]);
+        SceneClock clk = a.clocks ? uniform_copy(a.clocks[run.scene]) : given;
         if (advance_clock) clk = next_clock(c, clk);
         double *g = (double *)(a.grid_mem + S.grid_off[buf]);
         double *go = (double *)(a.grid_mem + S.grid_off[buf ^ 1]);
@@ -84,6 +87,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))
             }
         }
     }
+    if (!a.clocks && blockIdx.x == 0 && threadIdx.x == 0) *a.clocks_next = given;
     // the advanced clocks go to the other slot, which no block reads here
     if (advance_clock && blockIdx.x == 0)
         for (int sc = threadIdx.x; sc < a.nscenes; sc += kBlock)
@@ -93,7 +97,34 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))
 hipError_t launch_update(const StepArgs &a, int buf, int zero_other, int advance_clock, int n_blocks, hipStream_t s)
 {
     if (n_blocks <= 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_update, dim3(n_blocks), dim3(kBlock), 0, s, a, buf, zero_other, advance_clock);
+    hipLaunchKernelGGL(k_update, dim3(n_blocks), dim3(kBlock), 0, s, a, buf, zero_other, advance_clock, SceneClock{});
+    return hipGetLastError();
+}
+
+// Grid update of the runs a.chunks of one scene with a clock given by the
+// caller, which becomes the scene's current clock.
+hipError_t launch_update_at(StepArgs a, int buf, const SceneClock &clock, SceneClock *slot, int n_blocks, hipStream_t s)
+{
+    if (n_blocks <= 0) return hipErrorInvalidValue;
+    a.clocks = nullptr;
+    a.clocks_next = slot;
+    hipLaunchKernelGGL(k_update, dim3(n_blocks), dim3(kBlock), 0, s, a, buf, 0, 0, clock);
+    return hipGetLastError();
+}
+
+// Clears the flagged segments of the runs a.chunks in grid buffer buf, and
+// their flags: the whole buffer, since everything that adds to a node flags its
+// segment.
+__global__ void __launch_bounds__(kBlock) k_clear(StepArgs a, int buf)
+{
+    constexpr int per = kBlock / 64;
+    clear_flagged(a, buf, blockIdx.x * per + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), gridDim.x * per);
+}
+
+hipError_t launch_clear(const StepArgs &a, int buf, int n_blocks, hipStream_t s)
+{
+    if (n_blocks <= 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_clear, dim3(n_blocks), dim3(kBlock), 0, s, a, buf);
     return hipGetLastError();
 }
 
