@@ -719,8 +719,8 @@ void Engine::timed_begin(bool timed)
     if (ev_used_ >= 4096 && !capturing_) collect_timings();
     if (ev_used_ == ev_pool_.size()) {
         hipEvent_t a, b;
-        hipEventCreate(&a);
-        hipEventCreate(&b);
+        hipEventCreateWithFlags(&a, hipEventDisableSystemFence);
+        hipEventCreateWithFlags(&b, hipEventDisableSystemFence);
         ev_pool_.push_back({a, b});
         ev_cls_.push_back(0);
         ev_w_.push_back(1);
