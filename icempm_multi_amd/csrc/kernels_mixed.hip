@@ -140,6 +140,9 @@ k_tiles(StepArgs a, int rbuf, int wbuf, int zbuf, int record_mode)
         if (work.first >= work.end) break;
         const int w = work.first;
         const TileItem ti = work.item;
+        // All constants before the tile's loads: reading them between the loads
+        // and the point loop, as the FP64 kernel does, keeps more values live
+        // at four waves per SIMD and measured 19.2 us for 18.0 at 250k points.
         const SceneConsts c = sl.copy<SceneConsts>(offsetof(SceneDev, c));
         const long long off_r = sl.copy<long long>(offsetof(SceneDev, grid_off)) + rbuf * a.grid_buf_bytes;
         const long long off_w = sl.copy<long long>(offsetof(SceneDev, grid_off)) + wbuf * a.grid_buf_bytes;
@@ -363,6 +366,7 @@ k_tiles(StepArgs a, int rbuf, int wbuf, int zbuf, int record_mode)
                 dflag[gi >> kSegShift] = 1;
             }
         }
+        if (!dyn && work.first >= work.end) break;   // before the next tile's loads
     }
     if (dyn && tid == 0) {
         if (atomicAdd(a.tile_queue + 8, 1) == n_blocks - 1)
