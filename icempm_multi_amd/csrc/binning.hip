@@ -278,28 +278,54 @@ __global__ void __launch_bounds__(kBlock) k_tile_emit(StepArgs a, const int *til
         it.row0 = row0 + r_lo;
         it.dims = (c_hi - c_lo + 1) | ((r_hi - r_lo + 1) << 16);
         it.total = total;
+        it.runs = pos;
         tiles[pos] = it;
         weight[pos] = total + tile_cost;
     }
 }
 
+// Smallest of the wave's values, in every lane.
+__device__ __forceinline__ unsigned wave_min(unsigned v)
+{
+    // DPP: row_shr 1, 2, 4, 8 within 16 lanes, then row_bcast 15 and 31
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x111, 0xf, 0xf, false));
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x112, 0xf, 0xf, false));
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x114, 0xf, 0xf, false));
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x118, 0xf, 0xf, false));
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x142, 0xa, 0xf, false));
+    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x143, 0xc, 0xf, false));
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 // Splits the tiles among the workgroups of a tile launch.  The table is cut
 // into `parts` ranges, one per XCD (the workgroups of a range run on one XCD,
 // see xcd_block), of equal count if no workgroup gets two tiles, else of equal
-// summed weight (points, plus tile_cost per tile).  The workgroups of a range
-// take its tiles in turn: those at work at the same time are neighbours, whose
-// window nodes overlap in the XCD's L2 (with neighbours one after the other in
-// one workgroup instead, the launch of the 4M-point sheet was 13% slower at
-// 14x32 cells).  Before, the whole table was taken in turn by all workgroups,
-// and the last, partial round ran on the first XCDs alone: 12.7% slower on 1.2M
-// points of floes (8x32 cells), 26% on the 2.0M-point sheet in the mixed form
-// (14x32).  pre: exclusive prefix sums of the weights.
+// summed weight (points, plus tile_cost per tile).  One workgroup per range.
+//
+// Where a workgroup gets at most kPackTiles tiles on average, each tile goes to
+// the workgroup with the least weight so far, the heavy tiles first: the launch
+// lasts as long as its most loaded workgroup, and the tiles of a scene of floes
+// hold between 1 and all of their points (1.2M points of floes: 63.8 -> 54.5 us
+// per substep in FP64, 57 -> 48 in the mixed form).  The order of weights is coarse
+// (eighths of the largest) and full tiles count alike, so that tiles of about
+// one size go in turn and workgroups at work at the same time are neighbours, whose window
+// nodes overlap in the XCD's L2 (with neighbours one after the other in one
+// workgroup instead, the launch of the 4M-point sheet was 13% slower at 14x32
+// cells).
+//
+// Past that, and where there is at most one tile each, the workgroups take the
+// range's tiles in turn: the loads then differ by little, and the assignment,
+// which is serial, would take longer than it saves.  pre: exclusive prefix sums
+// of the weights; place: one int per tile.
+constexpr int kPackTiles = 8, kPackBins = 256, kPackLane = kPackBins / 64;
+
 __global__ void __launch_bounds__(kBlock) k_tile_split(const TileItem *tiles, const int *weight, const int *pre,
-                                                       const int *n_tiles, TileWork *work, int n_work, int parts)
+                                                       const int *n_tiles, TileItem *list, int *place, TileWork *work,
+                                                       int n_work, int parts)
 {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n_work) return;
-    const int n = *n_tiles, per = n_work / parts, part = i / per;
+    static_assert(kPackBins == kBlock, "one workgroup's tile count per thread");
+    __shared__ int base[kPackBins + 1];
+    const int tid = threadIdx.x, n = *n_tiles, per = n_work / parts, part = blockIdx.x;
     // first tile of range k: the first whose middle (doubled) reaches k parts of the weight
     auto start = [&](int k) {
         if (n <= n_work) return (int)((long long)n * k / parts);
@@ -312,12 +338,81 @@ __global__ void __launch_bounds__(kBlock) k_tile_split(const TileItem *tiles, co
         }
         return lo;
     };
-    TileWork out{};
-    out.first = start(part) + i % per;
-    out.end = start(part + 1);
-    out.step = per;
-    if (out.first < out.end) out.item = tiles[out.first];
-    work[i] = out;
+    const int t0 = start(part), t1 = start(part + 1);
+    const bool pack = n > n_work && per <= kPackBins && t1 - t0 <= kPackTiles * per;
+    if (pack && tid < 64) {
+        // workgroup b of the range is kept by lane b / J
+        const int J = (per + 63) / 64;
+        unsigned load[kPackLane];
+        int count[kPackLane];
+#pragma unroll
+        for (int j = 0; j < kPackLane; j++) {
+            load[j] = j < J && tid * J + j < per ? 0u : ~0u;
+            count[j] = 0;
+        }
+        unsigned most = 1;
+        for (int t = t0 + tid; t < t1; t += 64) most = max(most, (unsigned)weight[t]);
+        most = ~wave_min(~most);
+        for (int c = 7; c >= 0; c--) {
+            for (int first = t0; first < t1; first += 64) {
+                const int t = first + tid;
+                const int w = t < t1 ? weight[t] : 0;
+                const int cls = min(7, (int)(8.0f * (float)w / (float)most));
+                for (unsigned long long m = __ballot(t < t1 && cls == c); m; m &= m - 1) {
+                    const int i = __builtin_ctzll(m);
+                    // (the full tiles count alike: theirs go in turn)
+                    const unsigned wi = c == 7 ? most : (unsigned)__builtin_amdgcn_readlane(w, i);
+                    const unsigned mine = min(min(load[0], load[1]), min(load[2], load[3]));
+                    const unsigned least = wave_min(mine);
+                    const int owner = __builtin_ctzll(__ballot(mine == least));
+                    bool todo = tid == owner;
+#pragma unroll
+                    for (int j = 0; j < kPackLane; j++)
+                        if (todo && load[j] == least) {
+                            load[j] += wi;
+                            place[first + i] = (tid * J + j) << 16 | count[j]++;
+                            todo = false;
+                        }
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kPackLane; j++)
+            if (j < J && tid * J + j < kPackBins) base[tid * J + j + 1] = count[j];
+    }
+    __syncthreads();
+    if (!pack) {
+        for (int t = t0 + tid; t < t1; t += kBlock) list[t] = tiles[t];
+        for (int i = tid; i < per; i += kBlock) {
+            TileWork out{};
+            out.first = t0 + i;
+            out.end = t1;
+            out.step = per;
+            if (out.first < out.end) out.item = tiles[out.first];
+            work[part * per + i] = out;
+        }
+        return;
+    }
+    // counts to exclusive sums
+    if (tid >= per) base[tid + 1] = 0;
+    if (tid == 0) base[0] = 0;
+    __syncthreads();
+    for (int o = 1; o <= kPackBins; o <<= 1) {
+        const int v = tid + 1 >= o ? base[tid + 1 - o] : 0;
+        __syncthreads();
+        if (tid + 1 >= o) base[tid + 1] += v;
+        __syncthreads();
+    }
+    for (int t = t0 + tid; t < t1; t += kBlock) list[t0 + base[place[t] >> 16] + (place[t] & 0xffff)] = tiles[t];
+    __syncthreads();
+    if (tid < per) {
+        TileWork out{};
+        out.first = t0 + base[tid];
+        out.end = t0 + base[tid + 1];
+        out.step = 1;
+        if (out.first < out.end) out.item = list[out.first];
+        work[part * per + tid] = out;
+    }
 }
 
 // Tiles that hold points under each of several shapes (blockIdx.y).
@@ -416,6 +511,7 @@ size_t tile_table_layout(char *base, long long max_tiles, int tx, int nscenes, i
     t.n_work = n_work;
     t.work = (TileWork *)part(sizeof(TileWork) * n_work);
     t.tiles = (TileItem *)part(sizeof(TileItem) * max_tiles);
+    t.list = (TileItem *)part(sizeof(TileItem) * max_tiles);
     t.runs = (TileRun *)part(sizeof(TileRun) * tx * max_tiles);
     t.n_tiles = (int *)part(sizeof(int));
     t.tile_off = (int *)part(sizeof(int) * (nscenes + 1));
@@ -450,8 +546,9 @@ hipError_t launch_build_tiles(const StepArgs &a, const SceneDev *host_scenes, in
                        t.runs, t.weight, tile_cost, t.n_tiles);
     // (weights past the live tiles are not read from the sums)
     if ((e = scan_exclusive(t.weight, t.pos, total, t.scan_tmp, s)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_tile_split, dim3(nblk(t.n_work, kBlock)), dim3(kBlock), 0, s, t.tiles, t.weight, t.pos,
-                       t.n_tiles, t.work, t.n_work, t.n_work % 8 ? 1 : 8);
+    const int parts = t.n_work % 8 ? 1 : 8;
+    hipLaunchKernelGGL(k_tile_split, dim3(parts), dim3(kBlock), 0, s, t.tiles, t.weight, t.pos, t.n_tiles, t.list,
+                       t.flag, t.work, t.n_work, parts);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     // the host copy of off[] must stay alive until the copy ran

@@ -567,6 +567,7 @@ StepArgs Engine::args() const
     a.pitch = pitch_;
     a.cell_start = bins_.cell_start;
     a.tiles = tiles_.tiles;
+    a.tile_list = tiles_.list;
     a.tile_runs = tiles_.runs;
     a.tile_work = tiles_.work;
     a.grid_buf_bytes = grid_buf_bytes_;

@@ -87,7 +87,8 @@ struct TileTable {
     long long max_tiles = 0;
     int n_work = 0;               // workgroups of a tile launch
     TileWork *work = nullptr;
-    TileItem *tiles = nullptr;
+    TileItem *tiles = nullptr;    // in spatial order
+    TileItem *list = nullptr;     // by workgroup
     TileRun *runs = nullptr;
     int *n_tiles = nullptr;
     int *tile_off = nullptr, *flag = nullptr, *pos = nullptr, *weight = nullptr, *scan_tmp = nullptr;

@@ -173,7 +173,6 @@ k_tiles(StepArgs a, int rbuf, int wbuf, int zbuf, int record_mode)
         SceneClock clk = scalar_load(clock);
         pin(work);
         if (work.first >= work.end) break;
-        const int w = work.first;
         const TileItem ti = work.item;
         // What the tile's loads need first; the rest of the constants are read
         // out of the lanes while those loads are under way.  The serial start is
@@ -196,7 +195,7 @@ k_tiles(StepArgs a, int rbuf, int wbuf, int zbuf, int record_mode)
         constexpr int kU = 4;
         double m[kU], px[kU], py[kU];
         TileRun my_run{0, kRunEnd};
-        if (tid < ncol) my_run = a.tile_runs[(long long)w * a.tx + tid];
+        if (tid < ncol) my_run = a.tile_runs[(long long)ti.runs * a.tx + tid];
         static_assert(kFailTab <= kBlock, "one table entry per thread");
         const bool new_table = DO_G2P && ti.scene != tab_scene;
         double my_fail = 0;
@@ -405,7 +404,7 @@ k_tiles(StepArgs a, int rbuf, int wbuf, int zbuf, int record_mode)
         }
         if (err) atomicMax(&a.err[ti.scene], err);
         work.first += work.step;
-        if (work.first < work.end) work.item = scalar_load(a.tiles + work.first);
+        if (work.first < work.end) work.item = scalar_load(a.tile_list + work.first);
         __syncthreads();
         if (DO_P2G) {
             for (int i = tid; i < WN; i += kBlock) {

@@ -138,7 +138,6 @@ k_tiles(StepArgs a, int rbuf, int wbuf, int zbuf, int record_mode)
         pin(work);
         pin(clk);
         if (work.first >= work.end) break;
-        const int w = work.first;
         const TileItem ti = work.item;
         // All constants before the tile's loads: reading them between the loads
         // and the point loop, as the FP64 kernel does, keeps more values live
@@ -190,7 +189,7 @@ k_tiles(StepArgs a, int rbuf, int wbuf, int zbuf, int record_mode)
         // tile where there is no flush).
         if (tid < kMaxTX) {
             TileRun r{0, kRunEnd};
-            if (tid < ncol) r = a.tile_runs[(long long)w * a.tx + tid];
+            if (tid < ncol) r = a.tile_runs[(long long)ti.runs * a.tx + tid];
             runs[tid].off = r.off;
             runs[tid].end = r.end;
         }
@@ -351,7 +350,7 @@ k_tiles(StepArgs a, int rbuf, int wbuf, int zbuf, int record_mode)
         }
         if (err) atomicMax(&a.err[ti.scene], err);
         work.first += work.step;
-        if (work.first < work.end) work.item = scalar_load(a.tiles + work.first);
+        if (work.first < work.end) work.item = scalar_load(a.tile_list + work.first);
         __syncthreads();
         if (DO_P2G) {
             for (int i = tid; i < WN; i += kBlock) {

@@ -122,7 +122,8 @@ struct TileItem {
     int col0, row0;
     int dims;
     int total;
-    int pad[3];
+    int runs;      // its place in the spatial order: its runs start at runs * tx
+    int pad[2];
 };
 
 // The run of one column of a tile's box: points [previous end, end) of the
@@ -155,8 +156,8 @@ struct TileWindow {
 };
 
 // The tiles of one workgroup of a tile launch: first, first + step, ... < end
-// of the tile table, and a copy of the first one's item, so that a workgroup
-// has its work with one 64-byte load (first >= end: none).
+// of StepArgs::tile_list, and a copy of the first one's item, so that a
+// workgroup has its work with one 64-byte load (first >= end: none).
 struct TileWork {
     TileItem item;
     int first, end, step;
@@ -187,6 +188,7 @@ struct StepArgs {
     long long pitch;
     const int *cell_start;    // per scene ncells+1 global point indices (from the last sort)
     const TileItem *tiles;
+    const TileItem *tile_list; // the same tiles in the order of the workgroups' work
     const TileRun *tile_runs; // tx entries per tile
     const TileWork *tile_work; // one per workgroup of a tile launch
     const int *n_tiles;       // device-side count of live tiles

@@ -62,3 +62,17 @@ def test_shape_by_rule_matches_oracle(nx, ny):
     assert c["tx"] * c["ty"] <= 16 * 32
     if n <= 4096:
         assert (c["tx"], c["ty"]) == (4, 8)
+
+
+# tiles of one to all of their points: 2, 4 and 8 tiles per workgroup (assigned
+# by weight, the last at the edge of that) and 16 and more (taken in turn)
+@pytest.mark.parametrize("shape", [(3, 5, 1), (3, 3, 0), (2, 2, 1), (1, 2, 1)])
+@pytest.mark.parametrize("nx,ny", [(200, 128), (230, 160)])
+def test_uneven_tiles_match_oracle(nx, ny, shape):
+    P, h, n = scenes.block_scene(nx=nx, ny=ny, grid=(nx + 40, ny + 24), n_grains=40)
+    r = np.random.default_rng(nx)
+    thin = 0.5 + 0.5 * np.sin(h[4, :n] * (7.0 / h[4, :n].max())) * np.cos(h[5, :n] * (9.0 / h[5, :n].max()))
+    keep = np.flatnonzero(r.random(n) < thin)
+    h[:, :keep.size] = h[:, keep]
+    c = step_and_compare(P, h, keep.size, shape)
+    assert (c["tx"], c["ty"], c["margin"]) == shape
