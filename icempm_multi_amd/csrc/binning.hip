@@ -415,28 +415,39 @@ __global__ void __launch_bounds__(kBlock) k_tile_split(const TileItem *tiles, co
     }
 }
 
-// Tiles that hold points under each of several shapes (blockIdx.y).
-__global__ void __launch_bounds__(kBlock) k_tile_census(StepArgs a, TileShapes shapes, int *counts)
+// Tiles that hold points under each of several shapes (blockIdx.y), counted by
+// their passes of kBlock points.
+__global__ void __launch_bounds__(kBlock) k_tile_census(StepArgs a, TileShapes shapes, TileCensus *out)
 {
-    const int tx = shapes.tx[blockIdx.y], ty = shapes.ty[blockIdx.y];
-    int live = 0;
+    __shared__ TileCensus here;
+    const int tx = shapes.tx[blockIdx.y], ty = shapes.ty[blockIdx.y], tid = threadIdx.x;
+    if (tid < TileCensus::kPasses) here.tiles[tid] = 0;
+    if (tid == 0) here.most = here.points = 0;
+    __syncthreads();
     for (int sc = 0; sc < a.nscenes; sc++) {
         const SceneDev &S = a.scenes[sc];
         const int ntx = (S.c.ncols + tx - 1) / tx, nty = (S.c.gridY + ty - 1) / ty;
         const long long n = (long long)ntx * nty;
-        for (long long t = (long long)blockIdx.x * kBlock + threadIdx.x; t < n; t += (long long)gridDim.x * kBlock) {
+        for (long long t = (long long)blockIdx.x * kBlock + tid; t < n; t += (long long)gridDim.x * kBlock) {
             const int col0 = (int)(t / nty) * tx, row0 = (int)(t % nty) * ty, rend = min(row0 + ty, S.c.gridY);
             int points = 0;
             for (int c = col0; c < min(col0 + tx, S.c.ncols); c++) {
                 const int *cs = a.cell_start + S.cell_off + (long long)c * S.c.gridY;
-                points |= cs[rend] - cs[row0];
+                points += cs[rend] - cs[row0];
             }
-            live += points != 0;
+            if (points == 0) continue;
+            const int passes = (points + kBlock - 1) / kBlock;
+            atomicAdd(&here.tiles[min(passes, TileCensus::kPasses) - 1], 1);
+            atomicMax(&here.most, passes);
+            atomicAdd(&here.points, points);
         }
     }
-#pragma unroll
-    for (int k = 32; k > 0; k >>= 1) live += __shfl_xor(live, k);
-    if ((threadIdx.x & 63) == 0 && live) atomicAdd(&counts[blockIdx.y], live);
+    __syncthreads();
+    if (tid < TileCensus::kPasses && here.tiles[tid]) atomicAdd(&out[blockIdx.y].tiles[tid], here.tiles[tid]);
+    if (tid == 0 && here.points) {
+        atomicMax(&out[blockIdx.y].most, here.most);
+        atomicAdd(&out[blockIdx.y].points, here.points);
+    }
 }
 
 inline unsigned nblk(long long n, int b) { return (unsigned)((n + b - 1) / b); }
@@ -486,13 +497,13 @@ hipError_t launch_sort(const StepArgs &a, const SceneDev *host_scenes, int nscen
     return hipGetLastError();
 }
 
-hipError_t launch_tile_census(const StepArgs &a, const TileShapes &shapes, long long n_cells, int *counts,
+hipError_t launch_tile_census(const StepArgs &a, const TileShapes &shapes, long long n_cells, TileCensus *out,
                               hipStream_t s)
 {
-    const hipError_t e = launch_fill_zero(counts, sizeof(int) * shapes.n, s);
+    const hipError_t e = launch_fill_zero(out, sizeof(TileCensus) * shapes.n, s);
     if (e != hipSuccess) return e;
     const unsigned g = (unsigned)std::min<long long>(std::max<long long>(n_cells / (32 * kBlock), 1), 256);
-    hipLaunchKernelGGL(k_tile_census, dim3(g, shapes.n), dim3(kBlock), 0, s, a, shapes, counts);
+    hipLaunchKernelGGL(k_tile_census, dim3(g, shapes.n), dim3(kBlock), 0, s, a, shapes, out);
     return hipGetLastError();
 }
 

@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <map>
 #include <string>
 #include <vector>
 
@@ -487,7 +488,8 @@ int Engine::alloc_bins()
 {
     if (bin_mem_) { hipFree(bin_mem_); bin_mem_ = nullptr; }
     const long long np = std::max<long long>(n_pts_space_, 1), nc = std::max<long long>(bins_.n_cells_total, 1);
-    const long long nscan = std::max(np, nc) / 1000 + 64;
+    // the scan's block sums, or the tile census
+    const long long nscan = std::max(np, nc) / 1000 + 64 + sizeof(TileCensus) / sizeof(int) * TileShapes::kMax;
     const long long n_int = 3 * np + 3 * nc + nscan + nscenes() + 16;
     HIPCHK(hipMalloc(&bin_mem_, sizeof(int) * n_int));
     int *p = (int *)bin_mem_;
@@ -601,17 +603,41 @@ int Engine::set_tile_shape(int tx, int ty, int margin)
     return ICEMPM_OK;
 }
 
+// Passes of the most loaded of n_work workgroups that take the tiles of a
+// census, the heavy ones first, each by the least loaded (as k_tile_split
+// assigns them); a tile's staging and flush count as a pass.
+static long long most_loaded(const TileCensus &t, long long n_work)
+{
+    std::map<long long, long long> groups{{0, n_work}};   // load -> workgroups
+    for (int k = TileCensus::kPasses; k > 0; k--) {
+        const long long cost = 1 + (k == TileCensus::kPasses ? t.most : k);
+        for (long long left = t.tiles[k - 1]; left > 0;) {
+            const auto least = groups.begin();
+            const long long m = std::min(left, least->second), load = least->first + cost;
+            if ((least->second -= m) == 0) groups.erase(least);
+            groups[load] += m;
+            left -= m;
+        }
+    }
+    return groups.rbegin()->first;
+}
+
 // The tile shape of a scene set whose caller pinned none, by the tiles its
-// points occupy after the first sort of an upload.  The smallest shape whose
-// tiles all run at once is the fastest where there is one: a launch then lasts
-// as long as one workgroup's chain of one tile, and a small tile's points need
-// one pass (FP64 substep of 25.6k points: 8.3 us with 4x8 cells, 12.4 with
-// 8x16, 15.9 with 8x32; 102k points: 12.4 with 4x16, 13.2 with 8x16, 18.3 with
-// 8x32).  Where none fits, larger tiles repeat fewer window nodes, but a
-// second round that is nearly empty costs more: 16x32 from two rounds on (4.0M
-// points, 2.9 rounds: 126 us, 137 with 8x32), else 8x32 (1.2M points of floes,
-// 1.3 rounds of 16x32: 79 us, 64 with 8x32).  Small shapes whose table over a
-// huge grid would take more memory than is set aside for it are left out.
+// points occupy after the first sort of an upload: the one with the least
+//     passes of the most loaded workgroup
+//     + work of a compute unit: 0.3 per 256 points, 0.2 per tile, 0.5 per 256
+//       window nodes (of the unit with most tiles, if all tiles run at once).
+// A launch is a chain of passes in one workgroup while the chip is not full
+// (FP64 substep of 25.6k points: 8.0 us with 4x8 cells, 12.0 with 8x16, 25.9
+// with 16x32) and bound by the units' throughput beyond, where larger tiles
+// repeat fewer window nodes (4.0M points: 127 us with 16x32, 134 with 8x32,
+// 160 with 8x16) unless they leave units idle (1.0M points, 525 tiles of 16x32:
+// 46.5 us, 37.5 with 8x32).  Fitted to 203 measured substeps of blocks, sheets,
+// floes and batches of 19k to 4M points in both forms; over these the shape
+// taken is at most 7% off the fastest of the five, on average 0.4%.
+//
+// Small shapes whose table over a huge grid would take more memory than is set
+// aside for it are left out.
 int Engine::choose_tile_shape()
 {
     static const int ladder[][2] = {{kMinTile[0], kMinTile[1]}, {4, 16}, {8, 16}, {8, 32}, {16, 32}};
@@ -623,11 +649,13 @@ int Engine::choose_tile_shape()
         shapes.ty[i] = ladder[i][1];
     }
     static_assert(n <= TileShapes::kMax, "shapes to count");
-    HIPCHK(launch_tile_census(args(), shapes, bins_.n_cells_total, bins_.scan_tmp, stream_));
-    int counts[n];
-    HIPCHK(hipMemcpyAsync(counts, bins_.scan_tmp, sizeof counts, hipMemcpyDeviceToHost, stream_));
+    TileCensus *const d_census = (TileCensus *)bins_.scan_tmp;
+    HIPCHK(launch_tile_census(args(), shapes, bins_.n_cells_total, d_census, stream_));
+    TileCensus census[n];
+    HIPCHK(hipMemcpyAsync(census, d_census, sizeof census, hipMemcpyDeviceToHost, stream_));
     HIPCHK(hipStreamSynchronize(stream_));
     int pick = n - 2;
+    double best = 1e300;
     for (int i = 0; i < n; i++) {
         StepArgs a = args();
         a.tx = shapes.tx[i];
@@ -636,11 +664,19 @@ int Engine::choose_tile_shape()
         a.win_h = a.ty + 2 + 2 * margin_;
         if (i < n - 2 && table_bytes(a.tx, a.ty, n_cus_ * 8) > std::max(tile_mem_bytes_, kTileMemStart)) continue;
         const int r = LAUNCH_PREC(tiles_resident_per_cu, a, kTileChain);
-        if (r > 0 && counts[i] <= (long long)n_cus_ * r) {
+        if (r <= 0) continue;
+        const TileCensus &t = census[i];
+        long long tiles = 0;
+        for (int k : t.tiles) tiles += k;
+        const long long n_work = (long long)n_cus_ * r;
+        // tiles of a compute unit
+        const double per_cu = tiles <= n_work ? (double)((tiles + n_cus_ - 1) / n_cus_) : (double)tiles / n_cus_;
+        const double tile = 0.2 + (0.3 * t.points / std::max(1LL, tiles) + 0.5 * a.win_w * a.win_h) / 256;
+        const double cost = (double)most_loaded(t, n_work) + per_cu * tile;
+        if (cost < best) {
+            best = cost;
             pick = i;
-            break;
         }
-        if (r > 0 && i == n - 1 && counts[i] >= 2LL * n_cus_ * r) pick = i;
     }
     if (shapes.tx[pick] == tx_ && shapes.ty[pick] == ty_) return ICEMPM_OK;
     tx_ = shapes.tx[pick];

@@ -80,7 +80,14 @@ struct TileShapes {
     int n = 0;
     int tx[kMax], ty[kMax];
 };
-hipError_t launch_tile_census(const StepArgs &a, const TileShapes &shapes, long long n_cells, int *counts,
+// The tiles of one shape: how many take k + 1 passes of a workgroup (the last
+// entry: that many and more), the most passes, the points of all.
+struct TileCensus {
+    static constexpr int kPasses = 64;
+    int tiles[kPasses];
+    int most, points;
+};
+hipError_t launch_tile_census(const StepArgs &a, const TileShapes &shapes, long long n_cells, TileCensus *out,
                               hipStream_t s);
 // The tile table of the binned kernels (mpm_common.h) and its builder's memory.
 struct TileTable {
