@@ -8,8 +8,8 @@
 //   * positions are fixed point, x/h = xq * 2^-frac_bits - origin, so the
 //     resolution is uniform over the grid (2^-19 cells at 4096 columns) and
 //     the B-spline offset fx is exact;
-//   * the 2x2 SVD and the yield-surface projection of crushed points, and
-//     the grid velocity division, run in FP64 (physics_fp64.h).
+//   * the yield-surface projection of crushed points and the grid velocity
+//     division run in FP64 (physics_fp64.h).
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -88,8 +88,8 @@ __device__ __forceinline__ unsigned stencil_error(const SceneConsts &c, int bxc,
 }
 
 // The constitutive branch of partition_kernel_g2p (kernels.cuh:378-391):
-// intact points in FP32; crushed points go through the 2x2 SVD and the
-// Drucker-Prager projection in FP64.
+// intact points in FP32; crushed points go through the Drucker-Prager
+// projection in FP64.
 // The stress terms of the updated D are left in st (st.valid false when the
 // projection changed D or the point is liquid).
 __device__ __forceinline__ void constitutive(const SceneConsts &c, const ConstsF &cf, float D[4], float &Jm1,
