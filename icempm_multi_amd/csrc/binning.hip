@@ -170,17 +170,16 @@ __global__ void __launch_bounds__(kBlock) k_gather(StepArgs a, BinWork w, const 
 constexpr int kTileLanes = 32;
 
 // Place of tile t of the table: its scene and first cell.
-__device__ __forceinline__ const SceneDev &tile_place(const StepArgs &a, const int *tile_off, int t, int &scene,
-                                                      int &col0, int &row0)
+__device__ __forceinline__ const SceneDev &tile_place(const StepArgs &a, int t, int &scene, int &col0, int &row0)
 {
     int lo = 0, hi = a.nscenes - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if (tile_off[mid] <= t) lo = mid;
+        if (a.scenes[mid].tile_off <= t) lo = mid;
         else hi = mid - 1;
     }
     const SceneDev &S = a.scenes[lo];
-    const int local = t - tile_off[lo];
+    const int local = t - S.tile_off;
     scene = lo;
     col0 = (local / S.n_tiles_y) * a.tx;
     row0 = (local % S.n_tiles_y) * a.ty;
@@ -195,13 +194,12 @@ __device__ __forceinline__ int half_wave_min(int v)
 }
 
 // 1 per tile that holds points.
-__global__ void __launch_bounds__(kBlock) k_tile_count(StepArgs a, const int *tile_off, int n_tiles_all,
-                                                       int *tile_flag)
+__global__ void __launch_bounds__(kBlock) k_tile_count(StepArgs a, int n_tiles_all, int *tile_flag)
 {
     const int t = (blockIdx.x * kBlock + threadIdx.x) / kTileLanes, k = threadIdx.x & (kTileLanes - 1);
     if (t >= n_tiles_all) return;
     int sc, col0, row0;
-    const SceneDev &S = tile_place(a, tile_off, t, sc, col0, row0);
+    const SceneDev &S = tile_place(a, t, sc, col0, row0);
     int empty = 1;
     if (k < a.tx && col0 + k < S.c.ncols) {
         const int *cs = a.cell_start + S.cell_off + (long long)(col0 + k) * S.c.gridY;
@@ -215,8 +213,8 @@ __global__ void __launch_bounds__(kBlock) k_tile_count(StepArgs a, const int *ti
 // columns.  Each lane bisects its column: cell_start is nondecreasing, so the
 // first and last occupied rows are found in log2(ty) steps (one thread per
 // tile, column after column, took 12 us for any scene).
-__global__ void __launch_bounds__(kBlock) k_tile_emit(StepArgs a, const int *tile_off, int n_tiles_all,
-                                                      const int *tile_flag, const int *tile_pos, TileItem *tiles,
+__global__ void __launch_bounds__(kBlock) k_tile_emit(StepArgs a, int n_tiles_all, const int *tile_flag,
+                                                      const int *tile_pos, TileItem *tiles,
                                                       TileRun *runs, int *weight, int tile_cost, int *n_tiles)
 {
     const int t = (blockIdx.x * kBlock + threadIdx.x) / kTileLanes, k = threadIdx.x & (kTileLanes - 1);
@@ -225,7 +223,7 @@ __global__ void __launch_bounds__(kBlock) k_tile_emit(StepArgs a, const int *til
     if (t == n_tiles_all - 1 && k == 0) *n_tiles = pos + live;
     if (!live) return;
     int sc, col0, row0;
-    const SceneDev &S = tile_place(a, tile_off, t, sc, col0, row0);
+    const SceneDev &S = tile_place(a, t, sc, col0, row0);
     const int rend = min(row0 + a.ty, S.c.gridY);
     int c_lo = kTileLanes, c_hi = 0, r_lo = a.ty, r_hi = 0, s0 = 0, n = 0;   // c_hi, r_hi: negated for the minimum
     if (k < a.tx && col0 + k < S.c.ncols) {
@@ -510,7 +508,7 @@ hipError_t launch_tile_census(const StepArgs &a, const TileShapes &shapes, long 
 // The parts of a tile table of at most max_tiles tiles in one allocation: the
 // workgroups' work, the items, their runs, the tile count, and the builder's
 // own ints (scene offsets, flags, positions or weight sums, weights, scan sums).
-size_t tile_table_layout(char *base, long long max_tiles, int tx, int nscenes, int n_work, TileTable &t)
+size_t tile_table_layout(char *base, long long max_tiles, int tx, int n_work, TileTable &t)
 {
     size_t at = 0;
     auto part = [&](size_t bytes) {
@@ -525,7 +523,6 @@ size_t tile_table_layout(char *base, long long max_tiles, int tx, int nscenes, i
     t.list = (TileItem *)part(sizeof(TileItem) * max_tiles);
     t.runs = (TileRun *)part(sizeof(TileRun) * tx * max_tiles);
     t.n_tiles = (int *)part(sizeof(int));
-    t.tile_off = (int *)part(sizeof(int) * (nscenes + 1));
     t.flag = (int *)part(sizeof(int) * max_tiles);
     t.pos = (int *)part(sizeof(int) * max_tiles);
     t.weight = (int *)part(sizeof(int) * max_tiles);
@@ -537,33 +534,24 @@ hipError_t launch_build_tiles(const StepArgs &a, const SceneDev *host_scenes, in
                               const TileTable &t, hipStream_t s)
 {
     long long total = 0;
-    std::vector<int> off(nscenes + 1);
-    for (int i = 0; i < nscenes; i++) {
-        off[i] = (int)total;
-        total += (long long)host_scenes[i].n_tiles_x * host_scenes[i].n_tiles_y;
-    }
-    off[nscenes] = (int)total;
+    for (int i = 0; i < nscenes; i++) total += (long long)host_scenes[i].n_tiles_x * host_scenes[i].n_tiles_y;
     if (total > t.max_tiles || total == 0 || a.tx > kTileLanes || t.n_work <= 0) return hipErrorInvalidValue;
     // a tile's staging and flush cost about as much as 250 points (the sums of
     // the weights stay below 2^31)
     const int tile_cost = (int)std::max<long long>(0, std::min<long long>(250, (0x7fffffff - n_points) / total - 1));
-    hipError_t e = hipMemcpyAsync(t.tile_off, off.data(), sizeof(int) * (nscenes + 1), hipMemcpyHostToDevice, s);
-    if (e != hipSuccess) return e;
+    hipError_t e;
     const unsigned g = nblk(total * kTileLanes, kBlock);
-    hipLaunchKernelGGL(k_tile_count, dim3(g), dim3(kBlock), 0, s, a, t.tile_off, (int)total, t.flag);
+    hipLaunchKernelGGL(k_tile_count, dim3(g), dim3(kBlock), 0, s, a, (int)total, t.flag);
     // positions of the non-empty tiles: exclusive scan of the 0/1 flags
     if ((e = scan_exclusive(t.flag, t.pos, total, t.scan_tmp, s)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_tile_emit, dim3(g), dim3(kBlock), 0, s, a, t.tile_off, (int)total, t.flag, t.pos, t.tiles,
+    hipLaunchKernelGGL(k_tile_emit, dim3(g), dim3(kBlock), 0, s, a, (int)total, t.flag, t.pos, t.tiles,
                        t.runs, t.weight, tile_cost, t.n_tiles);
     // (weights past the live tiles are not read from the sums)
     if ((e = scan_exclusive(t.weight, t.pos, total, t.scan_tmp, s)) != hipSuccess) return e;
     const int parts = t.n_work % 8 ? 1 : 8;
     hipLaunchKernelGGL(k_tile_split, dim3(parts), dim3(kBlock), 0, s, t.tiles, t.weight, t.pos, t.n_tiles, t.list,
                        t.flag, t.work, t.n_work, parts);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    // the host copy of off[] must stay alive until the copy ran
-    return hipStreamSynchronize(s);
+    return hipGetLastError();
 }
 
 }  // namespace icempm

@@ -130,6 +130,8 @@ private:
     const std::shared_ptr<TransferPool> &transfer_pool();
     int import_points(int scene, const double *hssoa, size_t capacity, long long offset, long long n);
     int export_points(int scene, double *hssoa, size_t capacity, long long offset, long long n);
+    // Device words to the host once the stream has reached this point.
+    int read_back(void *dst, const void *src, size_t bytes);
     int alloc_bins();
     int alloc_tiles();
     long long count_tiles(int tx, int ty) const;
@@ -174,6 +176,7 @@ private:
     long long grid_buf_bytes_ = 0; // bytes of one of the three grid buffers (all scenes)
     double *ind_force_mem_ = nullptr;
     SceneDev *d_scenes_ = nullptr;
+    bool scenes_pushed_ = false;   // d_scenes_ holds host_dev_
     SceneClock *d_clocks_ = nullptr;
     unsigned *d_err_ = nullptr;
     int *d_tile_queue_ = nullptr;

@@ -314,17 +314,27 @@ int Engine::build_scene_dev(int i, SceneDev &d) const
 
 int Engine::push_scenes()
 {
-    host_dev_.resize(nscenes());
+    std::vector<SceneDev> dev(nscenes());
     int n_ind = 0;
+    long long tiles = 0;
     for (int i = 0; i < nscenes(); i++) {
-        build_scene_dev(i, host_dev_[i]);
-        n_ind += host_dev_[i].c.ind_rsq > 0;
+        build_scene_dev(i, dev[i]);
+        n_ind += dev[i].c.ind_rsq > 0;
+        dev[i].tile_off = (int)tiles;
+        tiles += (long long)dev[i].n_tiles_x * dev[i].n_tiles_y;
     }
     // service workgroups of the substep launches: one per scene with an
     // indenter, at most 16 (each takes every n_service-th scene)
     n_service_ = std::min(n_ind, 16);
+    // most sorts change nothing in the table
+    if (scenes_pushed_ && host_dev_.size() == dev.size() &&
+        std::memcmp(host_dev_.data(), dev.data(), sizeof(SceneDev) * dev.size()) == 0)
+        return ICEMPM_OK;
+    host_dev_ = std::move(dev);
+    scenes_pushed_ = false;
     HIPCHK(hipMemcpyAsync(d_scenes_, host_dev_.data(), sizeof(SceneDev) * nscenes(), hipMemcpyHostToDevice, stream_));
     HIPCHK(hipStreamSynchronize(stream_));
+    scenes_pushed_ = true;
     return ICEMPM_OK;
 }
 
@@ -449,6 +459,7 @@ int Engine::commit()
     if (d_scenes_) hipFree(d_scenes_);
     if (d_clocks_) hipFree(d_clocks_);
     if (d_err_) hipFree(d_err_);
+    scenes_pushed_ = false;
     HIPCHK(hipMalloc(&d_scenes_, sizeof(SceneDev) * nscenes()));
     HIPCHK(hipMalloc(&d_clocks_, sizeof(SceneClock) * 2 * nscenes()));   // two slots
     clock_slot_ = 0;
@@ -518,7 +529,7 @@ long long Engine::count_tiles(int tx, int ty) const
 size_t Engine::table_bytes(int tx, int ty, int n_work) const
 {
     TileTable t;
-    return tile_table_layout(nullptr, count_tiles(tx, ty), tx, nscenes(), n_work, t);
+    return tile_table_layout(nullptr, count_tiles(tx, ty), tx, n_work, t);
 }
 
 // The tile table for the current shape.
@@ -535,7 +546,7 @@ int Engine::alloc_tiles()
     int r = LAUNCH_PREC(tiles_resident_per_cu, args(), kTileChain);
     if (r <= 0) r = 8;   // the runtime could not tell: several generations
     const int n_work = (int)std::min<long long>(std::max<long long>(mt, 1), (long long)n_cus_ * r);
-    const size_t tbytes = tile_table_layout(nullptr, mt, tx_, nscenes(), n_work, tiles_);
+    const size_t tbytes = tile_table_layout(nullptr, mt, tx_, n_work, tiles_);
     if (tbytes > tile_mem_bytes_) {
         // room for the smallest shape choose_tile_shape() may take, unless the
         // grids are huge: no second allocation when it does
@@ -546,7 +557,7 @@ int Engine::alloc_tiles()
         HIPCHK(hipMalloc(&tile_mem_, bytes));
         tile_mem_bytes_ = bytes;
     }
-    tile_table_layout((char *)tile_mem_, mt, tx_, nscenes(), n_work, tiles_);
+    tile_table_layout((char *)tile_mem_, mt, tx_, n_work, tiles_);
     HIPCHK(launch_fill_zero(tiles_.work, sizeof(TileWork) * n_work, stream_));   // no tiles until the next build
     return ICEMPM_OK;
 }
@@ -652,8 +663,7 @@ int Engine::choose_tile_shape()
     TileCensus *const d_census = (TileCensus *)bins_.scan_tmp;
     HIPCHK(launch_tile_census(args(), shapes, bins_.n_cells_total, d_census, stream_));
     TileCensus census[n];
-    HIPCHK(hipMemcpyAsync(census, d_census, sizeof census, hipMemcpyDeviceToHost, stream_));
-    HIPCHK(hipStreamSynchronize(stream_));
+    RC(read_back(census, d_census, sizeof census));
     int pick = n - 2;
     double best = 1e300;
     for (int i = 0; i < n; i++) {
@@ -918,17 +928,14 @@ int Engine::get_indenter_force(int scene, double *out, int n)
     RC(ensure_committed());
     const SceneHost &s = scenes_[scene];
     const int m = std::min(n, 2 * s.prms.n_indenter_subdivisions);
-    HIPCHK(hipMemcpyAsync(out, s.ind_force, sizeof(double) * m, hipMemcpyDeviceToHost, stream_));
-    HIPCHK(hipStreamSynchronize(stream_));
-    return ICEMPM_OK;
+    return read_back(out, s.ind_force, sizeof(double) * m);
 }
 
 int Engine::get_error_code(uint8_t *code)
 {
     RC(ensure_committed());
     std::vector<unsigned> e(nscenes());
-    HIPCHK(hipMemcpyAsync(e.data(), d_err_, sizeof(unsigned) * nscenes(), hipMemcpyDeviceToHost, stream_));
-    HIPCHK(hipStreamSynchronize(stream_));
+    RC(read_back(e.data(), d_err_, sizeof(unsigned) * nscenes()));
     unsigned m = 0;
     for (unsigned v : e) m = std::max(m, v);
     *code = (uint8_t)m;
@@ -969,7 +976,7 @@ int Engine::build_tiles()
     const StepArgs a = args();
     HIPCHK(launch_build_tiles(a, host_dev_.data(), nscenes(), total_points(), tiles_, stream_));
     int nt = 0;
-    HIPCHK(hipMemcpy(&nt, tiles_.n_tiles, sizeof(int), hipMemcpyDeviceToHost));
+    RC(read_back(&nt, tiles_.n_tiles, sizeof(int)));
     if (nt < 0 || nt > tiles_.max_tiles) {
         bins_valid_ = false;
         return fail(ICEMPM_ERR_STATE, "build_tiles: tile count out of range");
@@ -990,8 +997,7 @@ int Engine::sort()
     std::swap(pts_[0], pts_[1]);
     pts_flip_ ^= 1;
     std::vector<int> cnt(nscenes());
-    HIPCHK(hipMemcpyAsync(cnt.data(), bins_.scene_count, sizeof(int) * nscenes(), hipMemcpyDeviceToHost, stream_));
-    HIPCHK(hipStreamSynchronize(stream_));
+    RC(read_back(cnt.data(), bins_.scene_count, sizeof(int) * nscenes()));
     bool counts_changed = false;
     for (int i = 0; i < nscenes(); i++) {
         const int m = scenes_[i].n_pts > 0 ? cnt[i] : 0;

@@ -98,10 +98,10 @@ struct TileTable {
     TileItem *list = nullptr;     // by workgroup
     TileRun *runs = nullptr;
     int *n_tiles = nullptr;
-    int *tile_off = nullptr, *flag = nullptr, *pos = nullptr, *weight = nullptr, *scan_tmp = nullptr;
+    int *flag = nullptr, *pos = nullptr, *weight = nullptr, *scan_tmp = nullptr;
 };
 // Lays the table out from base (null: only counts); returns its bytes.
-size_t tile_table_layout(char *base, long long max_tiles, int tx, int nscenes, int n_work, TileTable &t);
+size_t tile_table_layout(char *base, long long max_tiles, int tx, int n_work, TileTable &t);
 hipError_t launch_build_tiles(const StepArgs &a, const SceneDev *host_scenes, int nscenes, long long n_points,
                               const TileTable &t, hipStream_t s);
 

@@ -92,7 +92,7 @@ struct SceneDev {
     long long cell_off;     // first entry of the scene in the cell_start array
     int ncells;             // ncols*gridY
     int n_tiles_x, n_tiles_y;
-    int pad0;
+    int tile_off;           // tiles of the scenes before this one
     long long force_off;    // first of 2*n_ind_sub doubles in StepArgs::force_mem
     long long seg_off;      // first segment flag of the scene in each half of StepArgs::dirty
     // grain-dependent terms of the FP64 failure surface (scene_fail_table)
