@@ -219,7 +219,8 @@ private:
     bool capturing_ = false;                 // a graph capture is in progress
     static constexpr int kTimingSample = 32;  // ICEMPM_STEP_SAMPLED: one substep in 32 is timed
 
-    // Graphs of chunks of 1, 2, 4, ..., kMaxChunk units, keyed by (unit kind,
+    // Graphs of chunks of kMinChunk, ..., kMaxChunk units (of 1, 2, 4, ... where
+    // the launches are timed), keyed by (unit kind,
     // units, grid buffer, clock slot, point buffer parity, timing mode, first
     // unit timed).  A timed graph owns the hipEvents its capture recorded
     // (event record nodes); they are read after each replay.
@@ -231,6 +232,7 @@ private:
     };
     typedef std::array<int, 7> GraphKey;
     static constexpr int kMaxChunk = 64;      // units per graph: at most 192 kernel nodes (3 per unfused unit)
+    static constexpr int kMinChunk = 16;      // fewer are launched one by one
     static constexpr size_t kMaxGraphs = 256; // the cache is cleared between calls beyond this
     // Graphs one call can add: head and tail 1 each; the chain's 64-unit
     // chunks start from each of the 3 grid buffers, and its shorter chunks

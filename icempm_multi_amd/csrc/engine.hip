@@ -1128,7 +1128,7 @@ static void advance_units(int kind, int n, int &b, int &cs)
 }
 
 // The graph of n units of a kind from (b, cs), captured on first use.  The
-// cache holds chunks of 1, 2, 4, ..., kMaxChunk units, so its size is bounded
+// cache holds chunks of powers of two up to kMaxChunk units, so its size is bounded
 // whatever substep counts the callers use; a captured chunk refers to device
 // buffers that only commit(), set_tile_shape() and upload() replace (they
 // clear the cache), and to the point buffer pair member that the sort swaps
@@ -1209,6 +1209,14 @@ int Engine::run_units(int kind, int n, int &b, int &cs, bool use_graph, int tmod
         // units then starts at a multiple of 32 within the segment
         int len = kMaxChunk;
         while (len > n) len >>= 1;
+        if (!tmode && len < kMinChunk) {
+            // Too few for a graph: its launch takes the stream about as long as
+            // 10 units' launches take the host (10 substeps of 1.6k points as
+            // graphs of 8, 1 and 1 units 115 us, as launches 84).
+            RC(emit_units(kind, n, b, cs, false, sample, k, false));
+            advance_units(kind, n, b, cs);
+            return ICEMPM_OK;
+        }
         const bool first_timed = tmode == 2 ? (k % kTimingSample) == 0 : tmode != 0;
         GraphExec *gx = nullptr;
         RC(chunk_graph(kind, len, b, cs, tmode, first_timed, gx));

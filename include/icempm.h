@@ -284,8 +284,9 @@ int icempm_partition_autotune(icempm_partition *p, int n_trials, float *out_ms, 
 int icempm_partition_get_tile_config(icempm_partition *p, int *tx, int *ty, int *margin, int *lane_spread);
 /* hipGraph cache of the stepping calls (no reference counterpart): graphs
  * captured since creation and graphs held now.  A call of n substeps with
- * ICEMPM_STEP_GRAPH replays graphs of 1, 2, 4, ..., 64 substeps, captured on
- * first use and kept across calls and re-sorts. */
+ * ICEMPM_STEP_GRAPH replays graphs of 16, 32 and 64 substeps, captured on first
+ * use and kept across calls and re-sorts, and launches what is left directly
+ * (with ICEMPM_STEP_TIMINGS as graphs of 1, 2, 4 and 8). */
 int icempm_partition_get_graph_stats(icempm_partition *p, long long *captures, int *cached);
 
 /* ------------------------------------------------------------------------- */
