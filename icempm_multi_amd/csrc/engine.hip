@@ -568,6 +568,23 @@ int Engine::ensure_committed()
     return commit();
 }
 
+// LDS of the fused launch per window node, and its limit.
+constexpr size_t kWindowBytes = 64 * 1024;
+static size_t node_bytes(int precision) { return precision == ICEMPM_PRECISION_MIXED ? 56 : 64; }
+
+// The LDS window of a tile shape.  Heights a little below one that the tile
+// kernels are compiled for take its column stride.
+static void set_window(StepArgs &a, int tx, int ty, int margin, int precision)
+{
+    a.win_w = tx + 2 + 2 * margin;
+    a.win_h = ty + 2 + 2 * margin;
+    for (int h : {12, 18, 20, 34, 36, 66, 68})
+        if (h >= a.win_h && h <= a.win_h + 2 && (size_t)a.win_w * h * node_bytes(precision) <= kWindowBytes) {
+            a.win_h = h;
+            break;
+        }
+}
+
 StepArgs Engine::args() const
 {
     StepArgs a{};
@@ -592,8 +609,7 @@ StepArgs Engine::args() const
     a.tx = tx_;
     a.ty = ty_;
     a.margin = margin_;
-    a.win_w = tx_ + 2 + 2 * margin_;
-    a.win_h = ty_ + 2 + 2 * margin_;
+    set_window(a, tx_, ty_, margin_, precision_);
     a.lane_spread = lane_spread_;
     a.dyn_tiles = dyn_tiles_;
     a.tile_queue = d_tile_queue_;
@@ -644,14 +660,22 @@ static long long most_loaded(const TileCensus &t, long long n_work)
 // repeat fewer window nodes (4.0M points: 127 us with 16x32, 134 with 8x32,
 // 160 with 8x16) unless they leave units idle (1.0M points, 525 tiles of 16x32:
 // 46.5 us, 37.5 with 8x32).  Fitted to 203 measured substeps of blocks, sheets,
-// floes and batches of 19k to 4M points in both forms; over these the shape
-// taken is at most 7% off the fastest of the five, on average 0.4%.
+// floes and batches of 19k to 4M points in both forms.
+//
+// Ice is seeded with four points per cell, so a full tile of 16 or 32 rows holds
+// a few more points than whole passes take, or a few less: its last pass is
+// nearly empty for every other tile.  Tiles of 14 and 30 rows avoid that where
+// one workgroup's chain decides (FP64 substep of 102k points 11.9 -> 10.2 us
+// with 4x14 for 4x16 cells, 410k points 24.1 -> 20.8 with 8x14 for 8x32; 250k
+// points in the mixed form 18.1 -> 17.0 with 8x14 for 8x16).  Over 28 scenes the
+// shape taken is at most 10% off the fastest of twelve, on average 2%.
 //
 // Small shapes whose table over a huge grid would take more memory than is set
 // aside for it are left out.
 int Engine::choose_tile_shape()
 {
-    static const int ladder[][2] = {{kMinTile[0], kMinTile[1]}, {4, 16}, {8, 16}, {8, 32}, {16, 32}};
+    static const int ladder[][2] = {{kMinTile[0], kMinTile[1]}, {4, 14}, {8, 14}, {8, 16},
+                                    {8, 30}, {8, 32}, {16, 32}};
     constexpr int n = sizeof(ladder) / sizeof(ladder[0]);
     TileShapes shapes;
     shapes.n = n;
@@ -670,8 +694,7 @@ int Engine::choose_tile_shape()
         StepArgs a = args();
         a.tx = shapes.tx[i];
         a.ty = shapes.ty[i];
-        a.win_w = a.tx + 2 + 2 * margin_;
-        a.win_h = a.ty + 2 + 2 * margin_;
+        set_window(a, a.tx, a.ty, margin_, precision_);
         if (i < n - 2 && table_bytes(a.tx, a.ty, n_cus_ * 8) > std::max(tile_mem_bytes_, kTileMemStart)) continue;
         const int r = LAUNCH_PREC(tiles_resident_per_cu, a, kTileChain);
         if (r <= 0) continue;
@@ -701,9 +724,8 @@ int Engine::apply_tile_shape(int tx, int ty, int margin)
         return fail(ICEMPM_ERR_ARGUMENT, "tile shape out of range");
     // LDS of the fused launch per window node: (vx, vy) and two FP64 (m, px, py)
     // accumulators, 64 B in FP64 and 56 B in the mixed form (FP32 velocities)
-    const size_t per_node = precision_ == ICEMPM_PRECISION_MIXED ? 56 : 64;
-    const size_t lds = (size_t)(tx + 2 + 2 * margin) * (ty + 2 + 2 * margin) * per_node;
-    if (lds > 64 * 1024) return fail(ICEMPM_ERR_ARGUMENT, "tile window exceeds the LDS budget");
+    const size_t lds = (size_t)(tx + 2 + 2 * margin) * (ty + 2 + 2 * margin) * node_bytes(precision_);
+    if (lds > kWindowBytes) return fail(ICEMPM_ERR_ARGUMENT, "tile window exceeds the LDS budget");
     if (tx == tx_ && ty == ty_ && margin == margin_) return ICEMPM_OK;
     tx_ = tx;
     ty_ = ty;

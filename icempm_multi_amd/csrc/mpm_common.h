@@ -198,7 +198,8 @@ struct StepArgs {
     int nscenes;
     unsigned *err;            // per-scene error byte (max over points)
     int tx, ty, margin;       // tile shape and drift margin of the LDS windows
-    int win_w, win_h;         // tx+2+2*margin, ty+2+2*margin: the largest tile window (LDS size)
+    int win_w, win_h;         // the largest tile window in LDS: tx+2+2*margin columns, their stride
+                              // (at least ty+2+2*margin)
     int lane_spread;          // lane-to-point map of the tile kernels: 0 identity, 1 over 16 cells, 2 over 32 cells
     int dyn_tiles;            // 1: tiles pulled from per-XCD atomic queues, 0: static round robin
     int *tile_queue;          // 8 queue counters + 1 finished-block counter, zero between launches
