@@ -158,6 +158,9 @@ private:
     int record(int cls, bool timed, hipError_t (*)(void *), void *);
     void timed_begin(bool timed);
     void timed_end(bool timed, int cls, int launches = 1);
+    int phase_begin(StepArgs &a, int n_blocks);
+    void phase_end(const StepArgs &a, int cls);
+    int sum_stamps();
     int collect_timings();
     void record(hipEvent_t e);
     void invalidate_graphs();
@@ -212,6 +215,11 @@ private:
     std::vector<int> ev_cls_;
     std::vector<int> ev_w_;     // launches each event pair spans
     size_t ev_used_ = 0;
+    // phase calls: stamps of the launches not summed yet, then the sums by class
+    unsigned long long *stamps_ = nullptr;
+    StampClasses stamp_cls_;
+    bool ticks_pending_ = false;
+    int ticks_per_ms_ = 0;
     double cls_ms_[kNumCls] = {0};
     long long cls_cnt_[kNumCls] = {0};
     float last_step_ms_ = 0;

@@ -89,6 +89,15 @@ struct TileCensus {
 };
 hipError_t launch_tile_census(const StepArgs &a, const TileShapes &shapes, long long n_cells, TileCensus *out,
                               hipStream_t s);
+// Phase calls' times: stamps of launches (StepArgs::stamp, kStampStride words
+// each), summed by class into ticks.
+constexpr int kStampSlots = 32, kStampStride = 2 + kStampBlocks;
+struct StampClasses {
+    int n = 0;
+    unsigned char cls[kStampSlots];
+};
+hipError_t launch_sum_stamps(const unsigned long long *stamps, const StampClasses &classes, unsigned long long *ticks,
+                             hipStream_t s);
 // The tile table of the binned kernels (mpm_common.h) and its builder's memory.
 struct TileTable {
     long long max_tiles = 0;

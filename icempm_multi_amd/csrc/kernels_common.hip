@@ -15,7 +15,30 @@ __global__ void k_fill_zero(uint4 *p, size_t n16, unsigned char *tail, size_t nt
     if (i < ntail) tail[i] = 0;
 }
 
+// One workgroup per stamped launch: the time from its start to its last workgroup's end.
+__global__ void __launch_bounds__(256) k_sum_stamps(const unsigned long long *stamps, StampClasses classes,
+                                                    unsigned long long *ticks)
+{
+    __shared__ unsigned long long last;
+    const unsigned long long *const st = stamps + (long long)blockIdx.x * kStampStride;
+    if (threadIdx.x == 0) last = 0;
+    __syncthreads();
+    unsigned long long mine = 0;
+    for (unsigned b = threadIdx.x; b < st[1] && b < kStampBlocks; b += 256) mine = max(mine, st[2 + b]);
+    atomicMax(&last, mine);
+    __syncthreads();
+    if (threadIdx.x == 0 && last > st[0]) atomicAdd(&ticks[classes.cls[blockIdx.x]], last - st[0]);
+}
+
 }  // namespace
+
+hipError_t launch_sum_stamps(const unsigned long long *stamps, const StampClasses &classes, unsigned long long *ticks,
+                             hipStream_t s)
+{
+    if (classes.n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_sum_stamps, dim3(classes.n), dim3(256), 0, s, stamps, classes, ticks);
+    return hipGetLastError();
+}
 
 // Zero-fills `bytes` bytes with a kernel (graph-safe, unlike a memset node).
 // ptr must be 16-byte aligned.

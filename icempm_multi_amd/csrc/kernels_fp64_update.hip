@@ -30,6 +30,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))
     // lane) and their flags reset; flagged segments of this buffer are
     // updated, 8 at a time with their loads in flight together.
     constexpr int kU = 8;
+    stamp_begin(a);
     const int lane = threadIdx.x & 63;
     const int wave = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6), n_waves = gridDim.x * (kBlock / 64);
     for (int r = wave; r < a.n_chunks; r += n_waves) {
@@ -92,6 +93,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))
     if (advance_clock && blockIdx.x == 0)
         for (int sc = threadIdx.x; sc < a.nscenes; sc += kBlock)
             a.clocks_next[sc] = next_clock(a.scenes[sc].c, a.clocks[sc]);
+    stamp_end(a);
 }
 
 hipError_t launch_update(const StepArgs &a, int buf, int zero_other, int advance_clock, int n_blocks, hipStream_t s)
@@ -118,7 +120,9 @@ hipError_t launch_update_at(StepArgs a, int buf, const SceneClock &clock, SceneC
 __global__ void __launch_bounds__(kBlock) k_clear(StepArgs a, int buf)
 {
     constexpr int per = kBlock / 64;
+    stamp_begin(a);
     clear_flagged(a, buf, blockIdx.x * per + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), gridDim.x * per);
+    stamp_end(a);
 }
 
 hipError_t launch_clear(const StepArgs &a, int buf, int n_blocks, hipStream_t s)

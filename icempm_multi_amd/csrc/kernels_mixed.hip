@@ -88,6 +88,7 @@ k_tiles(StepArgs a, int rbuf, int wbuf, int zbuf, int record_mode)
     const int tid = threadIdx.x;
     const PtRef R{(unsigned *)a.pts, a.pitch};
     int block = blockIdx.x;
+    if (!FROM_M) stamp_begin(a);
     if (FROM_M && side_work(a, rbuf, zbuf, block)) return;
     const int n_blocks = a.n_work;
     TileWork work = scalar_load(a.tile_work + xcd_block(block, n_blocks));
@@ -380,6 +381,8 @@ k_tiles(StepArgs a, int rbuf, int wbuf, int zbuf, int record_mode)
             aside = a.defer_next[pt];
             deferred_point(a, DO_P2G, rbuf, wbuf, pt);
         }
+    } else {
+        stamp_end(a);
     }
 }
 

@@ -212,7 +212,25 @@ struct StepArgs {
     // point of the point space; -1 ends a list), and the points' scenes.
     int *defer_next;
     int *defer_scene;
+    // Phase calls: where the launch leaves its times (null: nowhere), see stamp_begin.
+    unsigned long long *stamp;
 };
+
+// A launch's times in ticks of the device's wall clock: [0] is when its first
+// workgroup started, [1] the number of its workgroups, [2 + b] when the first
+// wave of workgroup b was done.
+constexpr int kStampBlocks = 2048;   // a stamped launch has no more workgroups
+__device__ __forceinline__ void stamp_begin(const StepArgs &a)
+{
+    if (a.stamp && blockIdx.x == 0 && threadIdx.x == 0) {
+        a.stamp[0] = wall_clock64();
+        a.stamp[1] = gridDim.x;
+    }
+}
+__device__ __forceinline__ void stamp_end(const StepArgs &a)
+{
+    if (a.stamp && threadIdx.x == 0) a.stamp[2 + blockIdx.x] = wall_clock64();
+}
 
 // The clock of the next substep (model.cpp:39-41): t += dt by repeated
 // addition, indenter_x = x0 + t*V, each operation rounded on its own so that
