@@ -24,15 +24,14 @@ namespace icempm {
 
 // Tile candidates of the autotuner: {tx, ty, lane spread, dynamic queues}.
 // The widths between the powers of two let the tile count of a scene come
-// close to a whole number of rounds of the resident workgroups: a launch
-// whose last round holds a few tiles runs that round with most of the GPU
-// idle (on the 4M-point sheet, 8x64 tiles make 2.6 rounds, and the launch
-// costs 12% more per point than at a tile count of 2.0 rounds).
+// close to a whole number of tiles per resident workgroup.  The last one is for
+// scenes of a few tiles (25.6k points: 8.0 us per substep, 9.9 with 4x16 cells).
 const int kTileCandidates[][4] = {{4, 16, 1, 0},  {8, 8, 1, 0},   {4, 32, 1, 0},  {4, 64, 1, 0},  {8, 16, 1, 0},
                                   {8, 32, 1, 0},  {16, 16, 1, 0}, {4, 32, 0, 0},  {8, 32, 0, 0},  {4, 32, 2, 0},
                                   {8, 32, 2, 0},  {16, 32, 1, 0}, {8, 64, 1, 0},  {32, 16, 1, 0}, {5, 64, 1, 0},
                                   {6, 64, 1, 0},  {7, 64, 1, 0},  {10, 64, 1, 0}, {6, 32, 1, 0},  {10, 32, 1, 0},
-                                  {12, 32, 1, 0}, {14, 32, 1, 0}, {20, 32, 1, 0}, {24, 32, 1, 0}, {24, 16, 1, 0}};
+                                  {12, 32, 1, 0}, {14, 32, 1, 0}, {20, 32, 1, 0}, {24, 32, 1, 0}, {24, 16, 1, 0},
+                                  {4, 8, 1, 0}};
 const int kNumTileCandidates = (int)(sizeof(kTileCandidates) / sizeof(kTileCandidates[0]));
 
 namespace {
