@@ -314,15 +314,16 @@ __device__ __forceinline__ unsigned wave_min(unsigned v)
 // Past that, and where there is at most one tile each, the workgroups take the
 // range's tiles in turn: the loads then differ by little, and the assignment,
 // which is serial, would take longer than it saves.  pre: exclusive prefix sums
-// of the weights; place: one int per tile.
+// of the weights.
 constexpr int kPackTiles = 8, kPackBins = 256, kPackLane = kPackBins / 64;
 
 __global__ void __launch_bounds__(kBlock) k_tile_split(const TileItem *tiles, const int *weight, const int *pre,
-                                                       const int *n_tiles, TileItem *list, int *place, TileWork *work,
-                                                       int n_work, int parts)
+                                                       const int *n_tiles, TileItem *list, TileWork *work, int n_work,
+                                                       int parts)
 {
     static_assert(kPackBins == kBlock, "one workgroup's tile count per thread");
     __shared__ int base[kPackBins + 1];
+    __shared__ int wt[kPackTiles * kPackBins], place[kPackTiles * kPackBins];   // of the range's tiles
     const int tid = threadIdx.x, n = *n_tiles, per = n_work / parts, part = blockIdx.x;
     // first tile of range k: the first whose middle (doubled) reaches k parts of the weight
     auto start = [&](int k) {
@@ -338,6 +339,9 @@ __global__ void __launch_bounds__(kBlock) k_tile_split(const TileItem *tiles, co
     };
     const int t0 = start(part), t1 = start(part + 1);
     const bool pack = n > n_work && per <= kPackBins && t1 - t0 <= kPackTiles * per;
+    if (pack)
+        for (int t = t0 + tid; t < t1; t += kBlock) wt[t - t0] = weight[t];
+    __syncthreads();
     if (pack && tid < 64) {
         // workgroup b of the range is kept by lane b / J
         const int J = (per + 63) / 64;
@@ -349,14 +353,14 @@ __global__ void __launch_bounds__(kBlock) k_tile_split(const TileItem *tiles, co
             count[j] = 0;
         }
         unsigned most = 1;
-        for (int t = t0 + tid; t < t1; t += 64) most = max(most, (unsigned)weight[t]);
+        for (int t = tid; t < t1 - t0; t += 64) most = max(most, (unsigned)wt[t]);
         most = ~wave_min(~most);
         for (int c = 7; c >= 0; c--) {
-            for (int first = t0; first < t1; first += 64) {
+            for (int first = 0; first < t1 - t0; first += 64) {
                 const int t = first + tid;
-                const int w = t < t1 ? weight[t] : 0;
+                const int w = t < t1 - t0 ? wt[t] : 0;
                 const int cls = min(7, (int)(8.0f * (float)w / (float)most));
-                for (unsigned long long m = __ballot(t < t1 && cls == c); m; m &= m - 1) {
+                for (unsigned long long m = __ballot(t < t1 - t0 && cls == c); m; m &= m - 1) {
                     const int i = __builtin_ctzll(m);
                     // (the full tiles count alike: theirs go in turn)
                     const unsigned wi = c == 7 ? most : (unsigned)__builtin_amdgcn_readlane(w, i);
@@ -401,7 +405,10 @@ __global__ void __launch_bounds__(kBlock) k_tile_split(const TileItem *tiles, co
         if (tid + 1 >= o) base[tid + 1] += v;
         __syncthreads();
     }
-    for (int t = t0 + tid; t < t1; t += kBlock) list[t0 + base[place[t] >> 16] + (place[t] & 0xffff)] = tiles[t];
+    for (int t = t0 + tid; t < t1; t += kBlock) {
+        const int p = place[t - t0];
+        list[t0 + base[p >> 16] + (p & 0xffff)] = tiles[t];
+    }
     __syncthreads();
     if (tid < per) {
         TileWork out{};
@@ -550,7 +557,7 @@ hipError_t launch_build_tiles(const StepArgs &a, const SceneDev *host_scenes, in
     if ((e = scan_exclusive(t.weight, t.pos, total, t.scan_tmp, s)) != hipSuccess) return e;
     const int parts = t.n_work % 8 ? 1 : 8;
     hipLaunchKernelGGL(k_tile_split, dim3(parts), dim3(kBlock), 0, s, t.tiles, t.weight, t.pos, t.n_tiles, t.list,
-                       t.flag, t.work, t.n_work, parts);
+                       t.work, t.n_work, parts);
     return hipGetLastError();
 }
 
