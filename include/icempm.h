@@ -213,7 +213,9 @@ int icempm_partition_get_timings(icempm_partition *p, float *out, int n);
 
 /* Device time per kernel class since the last reset_indenter_force_accumulator,
  * recorded with hipEvents around each launch when ICEMPM_STEP_TIMINGS is set
- * (around each run of back-to-back fused launches with ICEMPM_STEP_SPAN):
+ * (around each run of back-to-back fused launches with ICEMPM_STEP_SPAN); the
+ * single-phase calls are always timed, by stamps of their launch after a sort
+ * (start of its first workgroup to end of its last) and by hipEvents before:
  * class 0 clock, 1 zero-fill, 2 P2G, 3 fused G2P+P2G (the grid update folded
  * in), 4 G2P (the last of a binned call also folds the grid update in), 5 grid
  * update (unbinned and unfused stepping, and the phase calls), 6 sort.
@@ -255,7 +257,8 @@ int icempm_partition_get_position_map(icempm_partition *p, int *frac_bits, int *
 
 /* Tile shape of the binned kernels: tx x ty cells per workgroup tile, LDS
  * windows widened by `margin` cells for points that drifted since the last
- * sort.  The autotuner sets it; callers may pin it. */
+ * sort.  By default it follows from the tiles that the points occupy at the
+ * first sort after an upload; the autotuner or this call pins it. */
 int icempm_partition_set_tile_shape(icempm_partition *p, int tx, int ty, int margin);
 /* Lane-to-point map of the binned kernels (the autotuner sets it with the tile
  * shape): 0 = lane l of a wave takes point l of its group, 1 = points of 16
@@ -274,7 +277,8 @@ int icempm_tile_candidates(int *tx, int *ty, int *lane_spread, int n);
 /* Project-written autotuner: times the substep launch of every candidate
  * tile shape, each with a window drift margin of 0 and of 1, on the current
  * point set after half a frame of substeps (the state drifts from its sort as
- * it does mid-frame), keeps the fastest and restores the state.  Results (ms
+ * it does mid-frame), keeps the fastest (no margin only if that is 3% faster)
+ * and restores the state.  Results (ms
  * per substep launch; -1 for a shape that does not fit) go to out_ms if
  * non-null: the K candidates at margin 0, then at margin 1 (2K values).
  * *chosen = margin * K + candidate, the shape kept; the shape itself is read
@@ -349,7 +353,7 @@ int icempm_poisson_disk(double r, double x0, double y0, double x1, double y1, ui
  * memory (code under hipGraph capture, serving loops, harnesses that forbid
  * hipMalloc): n_substeps substeps of one scene on points the caller holds in
  * device memory, FP64, in the HostSideSOA layout (16 lines of `pitch`
- * doubles, parameters_sim.h:27-35), with the unbinned P2G and G2P of
+ * doubles, parameters_sim.h:27-35), in the points' own order, as
  * icempm_partition_step(..., ICEMPM_STEP_DIRECT_P2G).  The clock starts at
  * prms->SimulationTime / SimulationStep and the indenter at
  * prms->indenter_x / indenter_y.  Every other buffer (grid, node flags,
