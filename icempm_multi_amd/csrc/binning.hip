@@ -319,12 +319,14 @@ constexpr int kPackTiles = 8, kPackBins = 256, kPackLane = kPackBins / 64;
 
 __global__ void __launch_bounds__(kBlock) k_tile_split(const TileItem *tiles, const int *weight, const int *pre,
                                                        const int *n_tiles, TileItem *list, TileWork *work, int n_work,
-                                                       int parts)
+                                                       int n_few, int parts)
 {
     static_assert(kPackBins == kBlock, "one workgroup's tile count per thread");
     __shared__ int base[kPackBins + 1];
     __shared__ int wt[kPackTiles * kPackBins], place[kPackTiles * kPackBins];   // of the range's tiles
-    const int tid = threadIdx.x, n = *n_tiles, per = n_work / parts, part = blockIdx.x;
+    const int tid = threadIdx.x, n = *n_tiles, part = blockIdx.x;
+    if (n <= n_few) n_work = n_few;
+    const int per = n_work / parts;
     // first tile of range k: the first whose middle (doubled) reaches k parts of the weight
     auto start = [&](int k) {
         if (n <= n_work) return (int)((long long)n * k / parts);
@@ -557,7 +559,7 @@ hipError_t launch_build_tiles(const StepArgs &a, const SceneDev *host_scenes, in
     if ((e = scan_exclusive(t.weight, t.pos, total, t.scan_tmp, s)) != hipSuccess) return e;
     const int parts = t.n_work % 8 ? 1 : 8;
     hipLaunchKernelGGL(k_tile_split, dim3(parts), dim3(kBlock), 0, s, t.tiles, t.weight, t.pos, t.n_tiles, t.list,
-                       t.work, t.n_work, parts);
+                       t.work, t.n_work, t.n_few, parts);
     return hipGetLastError();
 }
 

@@ -208,6 +208,7 @@ private:
     bool tiles_pinned_ = false;    // the caller (or the autotuner) chose the shape
     int lane_spread_ = 1;
     int dyn_tiles_ = 0;
+    bool few_ = false;        // StepArgs::few, from the tile count of the last build
     std::vector<SceneDev> host_dev_;
 
     // timings
@@ -230,7 +231,7 @@ private:
     // Graphs of chunks of kMinChunk, ..., kMaxChunk units (of 1, 2, 4, ... where
     // the launches are timed), keyed by (unit kind,
     // units, grid buffer, clock slot, point buffer parity, timing mode, first
-    // unit timed).  A timed graph owns the hipEvents its capture recorded
+    // unit timed, few_).  A timed graph owns the hipEvents its capture recorded
     // (event record nodes); they are read after each replay.
     struct GraphExec {
         hipGraphExec_t exec = nullptr;
@@ -238,7 +239,7 @@ private:
         std::vector<int> cls;
         std::vector<int> w;
     };
-    typedef std::array<int, 7> GraphKey;
+    typedef std::array<int, 8> GraphKey;
     static constexpr int kMaxChunk = 64;      // units per graph: at most 192 kernel nodes (3 per unfused unit)
     static constexpr int kMinChunk = 16;      // fewer are launched one by one
     static constexpr size_t kMaxGraphs = 256; // the cache is cleared between calls beyond this

@@ -550,9 +550,15 @@ int Engine::alloc_tiles()
     // 139.7 us with 8 workgroups per CU, 133.5 us with 2, its residency; mixed
     // 106.0 us with 8, 103.6 us with 4, its residency, 133 us with 2).  The
     // other launches take the substep launch's count: the tiles are split for it.
+    few_ = false;   // until the next build
     int r = LAUNCH_PREC(tiles_resident_per_cu, args(), kTileChain);
     if (r <= 0) r = 8;   // the runtime could not tell: several generations
     const int n_work = (int)std::min<long long>(std::max<long long>(mt, 1), (long long)n_cus_ * r);
+    StepArgs f = args();
+    f.few = 1;
+    const int r_few = LAUNCH_PREC(tiles_resident_per_cu, f, kTileChain);
+    int n_few = (int)std::min<long long>(n_work, (long long)n_cus_ * std::max(r_few, 0));
+    if (n_work % 8 == 0 && n_few % 8) n_few = 0;   // one share per XCD
     const size_t tbytes = tile_table_layout(nullptr, mt, tx_, n_work, tiles_);
     if (tbytes > tile_mem_bytes_) {
         // room for the smallest shape choose_tile_shape() may take, unless the
@@ -565,6 +571,7 @@ int Engine::alloc_tiles()
         tile_mem_bytes_ = bytes;
     }
     tile_table_layout((char *)tile_mem_, mt, tx_, n_work, tiles_);
+    tiles_.n_few = n_few;
     HIPCHK(launch_fill_zero(tiles_.work, sizeof(TileWork) * n_work, stream_));   // no tiles until the next build
     return ICEMPM_OK;
 }
@@ -621,7 +628,8 @@ StepArgs Engine::args() const
     a.dyn_tiles = dyn_tiles_;
     a.tile_queue = d_tile_queue_;
     a.dirty = d_dirty_;
-    a.n_work = tiles_.n_work;
+    a.n_work = few_ ? tiles_.n_few : tiles_.n_work;
+    a.few = few_;
     a.n_service = n_service_;
     a.n_clear = std::max(1, std::min((n_chunks_ + 3) / 4, n_cus_ * 8));
     a.defer_next = d_defer_;
@@ -699,6 +707,7 @@ int Engine::choose_tile_shape()
     double best = 1e300;
     for (int i = 0; i < n; i++) {
         StepArgs a = args();
+        a.few = 0;
         a.tx = shapes.tx[i];
         a.ty = shapes.ty[i];
         set_window(a, a.tx, a.ty, margin_, precision_);
@@ -1054,6 +1063,11 @@ int Engine::build_tiles()
         bins_valid_ = false;
         return fail(ICEMPM_ERR_STATE, "build_tiles: tile count out of range");
     }
+    // Where all tiles run at once in the kernel built for two waves per SIMD, the
+    // substep launch uses that one: nothing of it is spilled, and places for more
+    // waves would stay empty.  25.6k points FP64 8.0 -> 7.2 us, 102k 10.2 -> 9.6;
+    // mixed 102k 9.5 -> 8.9, 250k 16.5 -> 15.9.
+    few_ = nt <= tiles_.n_few;
     return ICEMPM_OK;
 }
 
@@ -1209,7 +1223,7 @@ static void advance_units(int kind, int n, int &b, int &cs)
 int Engine::chunk_graph(int kind, int n, int b, int cs, int tmode, bool first_timed, GraphExec *&out)
 {
     const int sample = tmode == 2 ? kTimingSample : 1;
-    const GraphKey key{kind, n, b, cs, pts_flip_, tmode, first_timed ? 1 : 0};
+    const GraphKey key{kind, n, b, cs, pts_flip_, tmode, first_timed ? 1 : 0, few_ ? 1 : 0};
     auto it = graphs_.find(key);
     if (it == graphs_.end()) {
         // step() makes room before a call's first launch: clearing the cache

@@ -60,12 +60,17 @@ __device__ __forceinline__ void deferred_point(const StepArgs &a, bool p2g, int 
     });
 }
 
-// 4 waves per SIMD (<= 128 VGPRs).  WHC: the LDS row stride (the largest
+// Waves per SIMD the tile kernel is built for; the second for launches whose
+// tiles all run at once with its 154 VGPRs, three per SIMD (StepArgs::few): 102k
+// points 8.9 us per substep, 9.5 with four.
+constexpr int kWaves = 4, kWavesFew = 2;
+
+// 4 waves per SIMD (<= 128 VGPRs), or fewer (see above).  WHC: the LDS row stride (the largest
 // window's height) when fixed at compile time (0: read from the arguments),
 // as in the FP64 form; so are the tile windows and the folded grid update of
 // kTileFromMomenta.
-template <int MODE, int WHC>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
+template <int MODE, int WHC, int WAVES>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES)))
 k_tiles(StepArgs a, int rbuf, int wbuf, int zbuf, int record_mode)
 {
     constexpr bool DO_G2P = (MODE & kTileG2P) != 0;
@@ -396,19 +401,22 @@ size_t tile_lds_bytes(const StepArgs &a, int mode)
 }
 
 // window heights compiled in: ty = 16, 32, 64 with a drift margin of 1 or 0, and 8 with 1
-template <int MODE>
+template <int MODE, int WAVES>
 static hipError_t launch_tiles_wh(const StepArgs &a, int rbuf, int wbuf, int zbuf, int record_mode, size_t lds,
                                   hipStream_t s)
 {
+    auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(tile_grid(a, MODE)), dim3(kBlock), lds, s, a, rbuf, wbuf, zbuf, record_mode);
+    };
     switch (a.win_h) {
-    case 12: hipLaunchKernelGGL((k_tiles<MODE, 12>), dim3(tile_grid(a, MODE)), dim3(kBlock), lds, s, a, rbuf, wbuf, zbuf, record_mode); break;
-    case 20: hipLaunchKernelGGL((k_tiles<MODE, 20>), dim3(tile_grid(a, MODE)), dim3(kBlock), lds, s, a, rbuf, wbuf, zbuf, record_mode); break;
-    case 36: hipLaunchKernelGGL((k_tiles<MODE, 36>), dim3(tile_grid(a, MODE)), dim3(kBlock), lds, s, a, rbuf, wbuf, zbuf, record_mode); break;
-    case 68: hipLaunchKernelGGL((k_tiles<MODE, 68>), dim3(tile_grid(a, MODE)), dim3(kBlock), lds, s, a, rbuf, wbuf, zbuf, record_mode); break;
-    case 18: hipLaunchKernelGGL((k_tiles<MODE, 18>), dim3(tile_grid(a, MODE)), dim3(kBlock), lds, s, a, rbuf, wbuf, zbuf, record_mode); break;
-    case 34: hipLaunchKernelGGL((k_tiles<MODE, 34>), dim3(tile_grid(a, MODE)), dim3(kBlock), lds, s, a, rbuf, wbuf, zbuf, record_mode); break;
-    case 66: hipLaunchKernelGGL((k_tiles<MODE, 66>), dim3(tile_grid(a, MODE)), dim3(kBlock), lds, s, a, rbuf, wbuf, zbuf, record_mode); break;
-    default: hipLaunchKernelGGL((k_tiles<MODE, 0>), dim3(tile_grid(a, MODE)), dim3(kBlock), lds, s, a, rbuf, wbuf, zbuf, record_mode); break;
+    case 12: run(k_tiles<MODE, 12, WAVES>); break;
+    case 18: run(k_tiles<MODE, 18, WAVES>); break;
+    case 20: run(k_tiles<MODE, 20, WAVES>); break;
+    case 34: run(k_tiles<MODE, 34, WAVES>); break;
+    case 36: run(k_tiles<MODE, 36, WAVES>); break;
+    case 66: run(k_tiles<MODE, 66, WAVES>); break;
+    case 68: run(k_tiles<MODE, 68, WAVES>); break;
+    default: run(k_tiles<MODE, 0, WAVES>); break;
     }
     return hipGetLastError();
 }
@@ -418,40 +426,44 @@ hipError_t launch_tiles(const StepArgs &a, int mode, int rbuf, int wbuf, int zbu
     if (a.tx > kMaxTX || a.n_work <= 0) return hipErrorInvalidValue;
     const size_t lds = tile_lds_bytes(a, mode);
     switch (mode) {
-    case kTileG2P: return launch_tiles_wh<kTileG2P>(a, rbuf, wbuf, zbuf, record_mode, lds, s);
-    case kTileP2G: return launch_tiles_wh<kTileP2G>(a, rbuf, wbuf, zbuf, record_mode, lds, s);
-    case kTileTail: return launch_tiles_wh<kTileTail>(a, rbuf, wbuf, zbuf, record_mode, lds, s);
-    case kTileChain: return launch_tiles_wh<kTileChain>(a, rbuf, wbuf, zbuf, record_mode, lds, s);
+    case kTileG2P: return launch_tiles_wh<kTileG2P, kWaves>(a, rbuf, wbuf, zbuf, record_mode, lds, s);
+    case kTileP2G: return launch_tiles_wh<kTileP2G, kWaves>(a, rbuf, wbuf, zbuf, record_mode, lds, s);
+    case kTileTail: return launch_tiles_wh<kTileTail, kWaves>(a, rbuf, wbuf, zbuf, record_mode, lds, s);
+    case kTileChain:
+        return a.few ? launch_tiles_wh<kTileChain, kWavesFew>(a, rbuf, wbuf, zbuf, record_mode, lds, s)
+                     : launch_tiles_wh<kTileChain, kWaves>(a, rbuf, wbuf, zbuf, record_mode, lds, s);
     default: return hipErrorInvalidValue;
     }
 }
 
-template <int MODE>
+template <int MODE, int WAVES>
 static int resident_wh(const StepArgs &a, size_t lds)
 {
-    int n = 0;
-    hipError_t e;
+    auto ask = [&](auto kernel) {
+        int n = 0;
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kBlock, lds) == hipSuccess ? n : 0;
+    };
     switch (a.win_h) {
-    case 12: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_tiles<MODE, 12>, kBlock, lds); break;
-    case 20: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_tiles<MODE, 20>, kBlock, lds); break;
-    case 36: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_tiles<MODE, 36>, kBlock, lds); break;
-    case 68: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_tiles<MODE, 68>, kBlock, lds); break;
-    case 18: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_tiles<MODE, 18>, kBlock, lds); break;
-    case 34: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_tiles<MODE, 34>, kBlock, lds); break;
-    case 66: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_tiles<MODE, 66>, kBlock, lds); break;
-    default: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_tiles<MODE, 0>, kBlock, lds); break;
+    case 12: return ask(k_tiles<MODE, 12, WAVES>);
+    case 18: return ask(k_tiles<MODE, 18, WAVES>);
+    case 20: return ask(k_tiles<MODE, 20, WAVES>);
+    case 34: return ask(k_tiles<MODE, 34, WAVES>);
+    case 36: return ask(k_tiles<MODE, 36, WAVES>);
+    case 66: return ask(k_tiles<MODE, 66, WAVES>);
+    case 68: return ask(k_tiles<MODE, 68, WAVES>);
+    default: return ask(k_tiles<MODE, 0, WAVES>);
     }
-    return e == hipSuccess ? n : 0;
 }
 
 int tiles_resident_per_cu(const StepArgs &a, int mode)
 {
     const size_t lds = tile_lds_bytes(a, mode);
     switch (mode) {
-    case kTileG2P: return resident_wh<kTileG2P>(a, lds);
-    case kTileP2G: return resident_wh<kTileP2G>(a, lds);
-    case kTileTail: return resident_wh<kTileTail>(a, lds);
-    case kTileChain: return resident_wh<kTileChain>(a, lds);
+    case kTileG2P: return resident_wh<kTileG2P, kWaves>(a, lds);
+    case kTileP2G: return resident_wh<kTileP2G, kWaves>(a, lds);
+    case kTileTail: return resident_wh<kTileTail, kWaves>(a, lds);
+    case kTileChain:
+        return a.few ? resident_wh<kTileChain, kWavesFew>(a, lds) : resident_wh<kTileChain, kWaves>(a, lds);
     default: return 0;
     }
 }

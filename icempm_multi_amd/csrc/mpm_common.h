@@ -206,6 +206,7 @@ struct StepArgs {
     int *dirty;               // segment flags: [buffer 0 of all scenes][buffer 1 ...][buffer 2 ...]
     long long dirty_stride;   // segments per buffer (all scenes)
     int n_work;               // tile workgroups of a tile launch
+    int few;                  // 1: all tiles run at once in the kernel built for fewer waves per SIMD
     int n_service, n_clear;   // workgroups before and after them in a kTileFromMomenta launch (side_work)
     // Points that a thread of a kTileFromMomenta launch sets aside for the end
     // of its work: a list per thread, linked through defer_next (one slot per
