@@ -206,7 +206,6 @@ struct StepArgs {
     int *dirty;               // segment flags: [buffer 0 of all scenes][buffer 1 ...][buffer 2 ...]
     long long dirty_stride;   // segments per buffer (all scenes)
     int n_work;               // tile workgroups of a tile launch
-    int few;                  // 1: all tiles run at once in the kernel built for fewer waves per SIMD
     int n_service, n_clear;   // workgroups before and after them in a kTileFromMomenta launch (side_work)
     // Points that a thread of a kTileFromMomenta launch sets aside for the end
     // of its work: a list per thread, linked through defer_next (one slot per
@@ -215,6 +214,10 @@ struct StepArgs {
     int *defer_scene;
     // Phase calls: where the launch leaves its times (null: nowhere), see stamp_begin.
     unsigned long long *stamp;
+    // 1: all tiles run at once in the kernel built for fewer waves per SIMD.  (Only
+    // the host reads it.  Kept behind the rest: between n_work and n_service it
+    // moved the kernel's argument loads, and 2.8M points took 89 us for 84.)
+    int few;
 };
 
 // A launch's times in ticks of the device's wall clock: [0] is when its first
