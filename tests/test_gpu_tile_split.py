@@ -76,3 +76,33 @@ def test_uneven_tiles_match_oracle(nx, ny, shape):
     h[:, :keep.size] = h[:, keep]
     c = step_and_compare(P, h, keep.size, shape)
     assert (c["tx"], c["ty"], c["margin"]) == shape
+
+
+# 400 to 1600 tiles: on both sides of the counts from which on the launch uses
+# the kernel built for more waves per SIMD, changed between graph replays
+@pytest.mark.parametrize("shapes", [[(4, 8, 1), (1, 2, 1), (4, 8, 1)], [(1, 3, 0), (2, 2, 1), (1, 4, 1), (1, 3, 0)]])
+def test_few_and_many_tiles_in_turn_match_oracle(shapes):
+    P, h, n = scenes.block_scene(nx=80, ny=20, grid=(128, 64), n_grains=40)
+    h[6, :n] = 0.3 * np.sin(3 * h[4, :n])
+    h[7, :n] = -0.2 * np.cos(2 * h[5, :n])
+    part = im.Partition(0, 0, im.PRECISION_FP64)
+    part.allocate(h.shape[1], P.GridXTotal)
+    part.update_constants(P)
+    part.transfer_points_from_soa_to_device(h, 0, n)
+    ref = h.copy()
+    t, step = 0.0, 0
+    for shape in shapes:
+        print(f"{n} points, tile {shape}", flush=True)
+        part.set_tile_shape(*shape)
+        part.step(20, im.STEP_GRAPH | im.STEP_RESORT)
+        O.sort(P, ref, n)
+        t, step, _, err = O.substeps(P, ref, n, 20, t, step)
+        assert err == 0
+    out = np.zeros_like(h)
+    part.transfer_from_device(out, 0)
+    assert part.error_code == 0
+    part.close()
+    for name, (a, b) in FIELDS.items():
+        scale = np.abs(ref[a:b, :n]).max()
+        assert np.abs(out[a:b, :n] - ref[a:b, :n]).max() <= 1e-9 * scale, name
+    assert np.array_equal(out[0, :n].view(np.int64), ref[0, :n].view(np.int64))
