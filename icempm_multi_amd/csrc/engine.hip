@@ -1065,7 +1065,7 @@ int Engine::build_tiles()
     }
     // Where all tiles run at once in the kernel built for two waves per SIMD, the
     // substep launch uses that one: nothing of it is spilled, and places for more
-    // waves would stay empty.  25.6k points FP64 8.0 -> 7.2 us, 102k 10.2 -> 9.6;
+    // waves would stay empty.  25.6k points FP64 8.0 -> 7.1 us, 102k 10.2 -> 9.6;
     // mixed 102k 9.5 -> 8.9, 250k 16.5 -> 15.9.
     few_ = nt <= tiles_.n_few;
     return ICEMPM_OK;

@@ -75,7 +75,7 @@ __device__ __forceinline__ void deferred_point(const StepArgs &a, bool p2g, int 
 }
 
 // Waves per SIMD the tile kernel is built for; the second for launches whose
-// tiles all run at once at two (StepArgs::few): 25.6k points 7.2 us per substep,
+// tiles all run at once at two (StepArgs::few): 25.6k points 7.1 us per substep,
 // 8.0 with three; the 4M-point sheet 140 with two, 127 with three.
 constexpr int kWaves = 3, kWavesFew = 2;
 
