@@ -325,7 +325,7 @@ __global__ void __launch_bounds__(kBlock) k_tile_split(const TileItem *tiles, co
     __shared__ int base[kPackBins + 1];
     __shared__ int wt[kPackTiles * kPackBins], place[kPackTiles * kPackBins];   // of the range's tiles
     const int tid = threadIdx.x, n = *n_tiles, part = blockIdx.x;
-    if (n <= n_few) n_work = n_few;
+    if (n_few > 0 && n <= n_few) n_work = n_few;
     const int per = n_work / parts;
     // first tile of range k: the first whose middle (doubled) reaches k parts of the weight
     auto start = [&](int k) {

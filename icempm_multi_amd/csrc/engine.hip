@@ -1067,7 +1067,8 @@ int Engine::build_tiles()
     // substep launch uses that one: nothing of it is spilled, and places for more
     // waves would stay empty.  25.6k points FP64 8.0 -> 7.1 us, 102k 10.2 -> 9.6;
     // mixed 102k 9.5 -> 8.9, 250k 16.5 -> 15.9.
-    few_ = nt <= tiles_.n_few;
+    // (Without a count for that kernel, an empty table too takes the other one.)
+    few_ = tiles_.n_few > 0 && nt <= tiles_.n_few;
     return ICEMPM_OK;
 }
 

@@ -102,7 +102,7 @@ hipError_t launch_sum_stamps(const unsigned long long *stamps, const StampClasse
 struct TileTable {
     long long max_tiles = 0;
     int n_work = 0;               // workgroups of a tile launch
-    int n_few = 0;                // workgroups where no more tiles than these are found
+    int n_few = 0;                // workgroups where no more tiles than these are found (0: always n_work)
     TileWork *work = nullptr;
     TileItem *tiles = nullptr;    // in spatial order
     TileItem *list = nullptr;     // by workgroup

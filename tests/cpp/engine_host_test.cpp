@@ -1,0 +1,90 @@
+// Host side of the engine on the runtime of fake_hip.cpp: one check per name.
+#include "fake_hip.h"
+
+#include <cstdio>
+#include <cstring>
+#include <functional>
+#include <vector>
+
+#include "../../include/icempm.h"
+
+namespace {
+
+int g_failed = 0;
+
+#define EXPECT(cond)                                                                        \
+    do {                                                                                    \
+        if (!(cond)) {                                                                      \
+            std::printf("%s:%d: %s (last error: %s)\n", __FILE__, __LINE__, #cond, icempm_last_error()); \
+            g_failed++;                                                                     \
+        }                                                                                   \
+    } while (0)
+
+icempm_simparams params(int gx, int gy)
+{
+    icempm_simparams P;
+    icempm_params_reset(&P);
+    P.GridXTotal = gx;
+    P.GridY = gy;
+    P.GridHaloSize = 8;
+    P.GridXDimension = 0.1 * gx;
+    P.nPtsTotal = 100;
+    P.ParticleVolume = 1e-3;
+    icempm_params_derive(&P);
+    return P;
+}
+
+icempm_partition *partition(const icempm_simparams &P, int capacity, int precision = ICEMPM_PRECISION_FP64, int device = 0)
+{
+    icempm_partition *p = nullptr;
+    EXPECT(icempm_partition_create(device, 0, precision, &p) == ICEMPM_OK);
+    EXPECT(icempm_partition_allocate(p, capacity, P.GridXTotal) == ICEMPM_OK);
+    EXPECT(icempm_partition_update_constants(p, &P, sizeof P) == ICEMPM_OK);
+    return p;
+}
+
+int launched(const char *name)
+{
+    int n = 0;
+    for (auto &l : fake::state().launches) n += l.name.find(name) != std::string::npos;
+    return n;
+}
+
+// A scene without points steps, also where the runtime cannot tell how many
+// workgroups a compute unit holds: its tile table has no tiles.
+void empty_scene()
+{
+    for (int occupancy : {2, 0}) {
+        fake::state().occupancy = occupancy;
+        const icempm_simparams P = params(64, 32);
+        icempm_partition *p = partition(P, 100);
+        std::vector<double> soa(16 * 100);
+        EXPECT(icempm_partition_transfer_points_from_soa_to_device(p, soa.data(), 100, 0, 0) == ICEMPM_OK);
+        EXPECT(icempm_partition_sort_points(p) == ICEMPM_OK);
+        EXPECT(icempm_partition_step(p, 3, 0) == ICEMPM_OK);
+        EXPECT(launched("k_tiles") > 0);
+        for (auto &l : fake::state().launches) EXPECT(l.grid.x > 0);
+        icempm_partition_destroy(p);
+    }
+}
+
+const struct {
+    const char *name;
+    void (*check)();
+} checks[] = {
+    {"empty_scene", empty_scene},
+};
+
+}  // namespace
+
+int main(int argc, char **argv)
+{
+    for (auto &c : checks)
+        if (argc == 2 && std::strcmp(argv[1], c.name) == 0) {
+            c.check();
+            std::printf("%s: %s\n", c.name, g_failed ? "failed" : "ok");
+            return g_failed != 0;
+        }
+    for (auto &c : checks) std::printf("%s\n", c.name);
+    return argc == 1 ? 0 : 2;
+}
