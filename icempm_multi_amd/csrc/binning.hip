@@ -166,8 +166,11 @@ __global__ void __launch_bounds__(kBlock) k_gather(StepArgs a, BinWork w, const 
     sorted_keys[j] = (col - S.c.halo + S.c.xoff) * S.c.gridY + row;
 }
 
-// Tile builder: half a wave per tile, a lane per column (tx <= 32).
-constexpr int kTileLanes = 32;
+// Tile builder: half a wave per tile, a lane per column (tx <= 32).  Its
+// launches have at most kBuildBlocks workgroups, which take the tiles in turn:
+// a launch of 2^32 threads (2^27 tiles) and more is refused, and small pinned
+// shapes on huge grids have up to 2^31 tiles.
+constexpr int kTileLanes = 32, kBuildBlocks = 65536;
 
 // Place of tile t of the table: its scene and first cell.
 __device__ __forceinline__ const SceneDev &tile_place(const StepArgs &a, int t, int &scene, int &col0, int &row0)
@@ -193,32 +196,41 @@ __device__ __forceinline__ int half_wave_min(int v)
     return v;
 }
 
+// f(t, k) for every tile t of the table, by its lanes k.
+template <class F>
+__device__ __forceinline__ void for_each_tile(int n_tiles_all, F &&f)
+{
+    const int k = threadIdx.x & (kTileLanes - 1);
+    constexpr int per = kBlock / kTileLanes;
+    for (long long t = (long long)blockIdx.x * per + threadIdx.x / kTileLanes; t < n_tiles_all;
+         t += (long long)gridDim.x * per)
+        f((int)t, k);
+}
+
 // 1 per tile that holds points.
 __global__ void __launch_bounds__(kBlock) k_tile_count(StepArgs a, int n_tiles_all, int *tile_flag)
 {
-    const int t = (blockIdx.x * kBlock + threadIdx.x) / kTileLanes, k = threadIdx.x & (kTileLanes - 1);
-    if (t >= n_tiles_all) return;
-    int sc, col0, row0;
-    const SceneDev &S = tile_place(a, t, sc, col0, row0);
-    int empty = 1;
-    if (k < a.tx && col0 + k < S.c.ncols) {
-        const int *cs = a.cell_start + S.cell_off + (long long)(col0 + k) * S.c.gridY;
-        empty = cs[min(row0 + a.ty, S.c.gridY)] == cs[row0];
-    }
-    empty = half_wave_min(empty);
-    if (k == 0) tile_flag[t] = !empty;
+    for_each_tile(n_tiles_all, [&](int t, int k) {
+        int sc, col0, row0;
+        const SceneDev &S = tile_place(a, t, sc, col0, row0);
+        int empty = 1;
+        if (k < a.tx && col0 + k < S.c.ncols) {
+            const int *cs = a.cell_start + S.cell_off + (long long)(col0 + k) * S.c.gridY;
+            empty = cs[min(row0 + a.ty, S.c.gridY)] == cs[row0];
+        }
+        empty = half_wave_min(empty);
+        if (k == 0) tile_flag[t] = !empty;
+    });
 }
 
 // The box of a tile's cells that hold points, and the runs of the box's
 // columns.  Each lane bisects its column: cell_start is nondecreasing, so the
 // first and last occupied rows are found in log2(ty) steps (one thread per
 // tile, column after column, took 12 us for any scene).
-__global__ void __launch_bounds__(kBlock) k_tile_emit(StepArgs a, int n_tiles_all, const int *tile_flag,
-                                                      const int *tile_pos, TileItem *tiles,
-                                                      TileRun *runs, int *weight, int tile_cost, int *n_tiles)
+__device__ __forceinline__ void emit_tile(const StepArgs &a, int t, int k, int n_tiles_all, const int *tile_flag,
+                                          const int *tile_pos, TileItem *tiles, TileRun *runs, int *weight,
+                                          int tile_cost, int *n_tiles)
 {
-    const int t = (blockIdx.x * kBlock + threadIdx.x) / kTileLanes, k = threadIdx.x & (kTileLanes - 1);
-    if (t >= n_tiles_all) return;
     const int live = tile_flag[t], pos = tile_pos[t];
     if (t == n_tiles_all - 1 && k == 0) *n_tiles = pos + live;
     if (!live) return;
@@ -280,6 +292,15 @@ __global__ void __launch_bounds__(kBlock) k_tile_emit(StepArgs a, int n_tiles_al
         tiles[pos] = it;
         weight[pos] = total + tile_cost;
     }
+}
+
+__global__ void __launch_bounds__(kBlock) k_tile_emit(StepArgs a, int n_tiles_all, const int *tile_flag,
+                                                      const int *tile_pos, TileItem *tiles,
+                                                      TileRun *runs, int *weight, int tile_cost, int *n_tiles)
+{
+    for_each_tile(n_tiles_all, [&](int t, int k) {
+        emit_tile(a, t, k, n_tiles_all, tile_flag, tile_pos, tiles, runs, weight, tile_cost, n_tiles);
+    });
 }
 
 // Smallest of the wave's values, in every lane.
@@ -549,7 +570,7 @@ hipError_t launch_build_tiles(const StepArgs &a, const SceneDev *host_scenes, in
     // the weights stay below 2^31)
     const int tile_cost = (int)std::max<long long>(0, std::min<long long>(250, (0x7fffffff - n_points) / total - 1));
     hipError_t e;
-    const unsigned g = nblk(total * kTileLanes, kBlock);
+    const unsigned g = std::min(nblk(total * kTileLanes, kBlock), (unsigned)kBuildBlocks);
     hipLaunchKernelGGL(k_tile_count, dim3(g), dim3(kBlock), 0, s, a, (int)total, t.flag);
     // positions of the non-empty tiles: exclusive scan of the 0/1 flags
     if ((e = scan_exclusive(t.flag, t.pos, total, t.scan_tmp, s)) != hipSuccess) return e;

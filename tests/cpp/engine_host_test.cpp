@@ -68,11 +68,25 @@ void empty_scene()
     }
 }
 
+// A table of more than 2^27 tiles (the smallest shape on a grid of 135M cells):
+// no launch of 2^32 threads or more, which the runtime refuses.
+void huge_tile_table()
+{
+    const icempm_simparams P = params(16400, 8200);
+    icempm_partition *p = partition(P, 100);
+    EXPECT(icempm_partition_set_tile_shape(p, 1, 1, 1) == ICEMPM_OK);
+    EXPECT(icempm_partition_sort_points(p) == ICEMPM_OK);
+    EXPECT(launched("k_tile_count") == 1 && launched("k_tile_emit") == 1);
+    for (auto &l : fake::state().launches) EXPECT((unsigned long long)l.grid.x * l.block.x < 1ull << 32);
+    icempm_partition_destroy(p);
+}
+
 const struct {
     const char *name;
     void (*check)();
 } checks[] = {
     {"empty_scene", empty_scene},
+    {"huge_tile_table", huge_tile_table},
 };
 
 }  // namespace

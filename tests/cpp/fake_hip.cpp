@@ -41,6 +41,12 @@ void *map(size_t bytes)
     return p == MAP_FAILED ? nullptr : p;
 }
 
+// The largest parts of memory are fresh where a test clears them, and zero.
+void clear(void *p, size_t n)
+{
+    if (n < (size_t(1) << 28)) std::memset(p, 0, n);
+}
+
 std::map<const void *, std::string> &kernel_names()
 {
     static std::map<const void *, std::string> m;
@@ -94,7 +100,7 @@ hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args, si
         void *p = *(void **)args[0];
         const size_t n16 = *(size_t *)args[1], tail = *(size_t *)args[3];
         l.pointer = p;
-        std::memset(p, 0, n16 * 16 + tail);
+        clear(p, n16 * 16 + tail);
     } else if (name.find("k_read") != std::string::npos) {
         std::memcpy(*(void **)args[1], *(void **)args[0], *(int *)args[2] * sizeof(unsigned));
     }
@@ -148,7 +154,8 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipSt
 }
 hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t)
 {
-    if (v != 0 || n < (size_t(1) << 28)) std::memset(p, v, n);   // the largest are fresh, and zero
+    if (v == 0) clear(p, n);
+    else std::memset(p, v, n);
     return hipSuccess;
 }
 

@@ -106,3 +106,12 @@ def test_few_and_many_tiles_in_turn_match_oracle(shapes):
         scale = np.abs(ref[a:b, :n]).max()
         assert np.abs(out[a:b, :n] - ref[a:b, :n]).max() <= 1e-9 * scale, name
     assert np.array_equal(out[0, :n].view(np.int64), ref[0, :n].view(np.int64))
+
+
+# a table of 1.1M tiles, of which the builder's workgroups take 524,288 at once;
+# the points' columns lie around the end of the first of these sweeps
+def test_table_beyond_one_sweep_of_the_builder_matches_oracle():
+    P, h, n = scenes.block_scene(nx=80, ny=20, grid=(1100, 1000), n_grains=40)
+    c = step_and_compare(P, h, n, (1, 1, 1))
+    first, last = (int(t(h[4, :n]) / P.cellsize) + P.GridHaloSize for t in (np.min, np.max))
+    assert first * P.GridY < 524288 < last * P.GridY and (c["tx"], c["ty"]) == (1, 1)
