@@ -81,6 +81,7 @@ int Engine::fail(int code, const std::string &msg)
 int Engine::hipfail(hipError_t e, const char *what)
 {
     set_last_error(std::string(what) + ": " + hipGetErrorString(e));
+    hipGetLastError();   // reported: not to be taken for the error of a later launch
     return ICEMPM_ERR_HIP;
 }
 
@@ -567,7 +568,12 @@ int Engine::alloc_tiles()
             std::max(tbytes, std::min(table_bytes(kMinTile[0], kMinTile[1], n_cus_ * 8), kTileMemStart));
         if (tile_mem_) { hipFree(tile_mem_); tile_mem_ = nullptr; }
         tile_mem_bytes_ = 0;
-        HIPCHK(hipMalloc(&tile_mem_, bytes));
+        const hipError_t e = hipMalloc(&tile_mem_, bytes);
+        if (e != hipSuccess) {
+            tile_mem_ = nullptr;
+            bins_valid_ = false;   // no table: nothing binned may be launched
+            return hipfail(e, "tile table");
+        }
         tile_mem_bytes_ = bytes;
     }
     tile_table_layout((char *)tile_mem_, mt, tx_, n_work, tiles_);
@@ -743,16 +749,25 @@ int Engine::apply_tile_shape(int tx, int ty, int margin)
     const size_t lds = (size_t)(tx + 2 + 2 * margin) * (ty + 2 + 2 * margin) * node_bytes(precision_);
     if (lds > kWindowBytes) return fail(ICEMPM_ERR_ARGUMENT, "tile window exceeds the LDS budget");
     if (tx == tx_ && ty == ty_ && margin == margin_) return ICEMPM_OK;
+    const int tx0 = tx_, ty0 = ty_, margin0 = margin_;
+    const bool bins = bins_valid_;
     tx_ = tx;
     ty_ = ty;
     margin_ = margin;
     invalidate_graphs();
     if (!committed_) return ICEMPM_OK;
     // the tile table depends on the shape; cell_start does not
-    RC(alloc_tiles());
+    const int rc = alloc_tiles();
+    if (rc != ICEMPM_OK) {   // no memory for this table: the shape stays what it was
+        tx_ = tx0;
+        ty_ = ty0;
+        margin_ = margin0;
+        if (alloc_tiles() != ICEMPM_OK) return rc;
+        bins_valid_ = bins;
+    }
     RC(push_scenes());
     if (bins_valid_) RC(build_tiles());
-    return ICEMPM_OK;
+    return rc;
 }
 
 // ---------------------------------------------------------------------------
@@ -1055,6 +1070,7 @@ int Engine::get_grid(int scene, int buf, double *out, long long n_nodes)
 // ---------------------------------------------------------------------------
 int Engine::build_tiles()
 {
+    if (!tile_mem_) RC(alloc_tiles());   // there was no memory for it
     const StepArgs a = args();
     HIPCHK(launch_build_tiles(a, host_dev_.data(), nscenes(), total_points(), tiles_, stream_));
     int nt = 0;

@@ -81,12 +81,41 @@ void huge_tile_table()
     icempm_partition_destroy(p);
 }
 
+// A tile shape whose table gets no memory is refused, and the calls after it
+// go on with the shape before it; without memory for any table the points are
+// stepped in their own order, and sorted again once there is memory.
+void no_memory_for_tiles()
+{
+    const icempm_simparams P = params(600, 400);
+    icempm_partition *p = partition(P, 100);
+    std::vector<double> soa(16 * 100);
+    EXPECT(icempm_partition_transfer_points_from_soa_to_device(p, soa.data(), 100, 0, 100) == ICEMPM_OK);
+    EXPECT(icempm_partition_set_tile_shape(p, 16, 16, 1) == ICEMPM_OK);
+    EXPECT(icempm_partition_sort_points(p) == ICEMPM_OK);
+    fake::state().malloc_limit = 8u << 20;   // a table of 1x1 cells takes 20 MB
+    EXPECT(icempm_partition_set_tile_shape(p, 1, 1, 0) == ICEMPM_ERR_HIP);
+    int tx = 0, ty = 0, margin = 0, spread = 0;
+    EXPECT(icempm_partition_get_tile_config(p, &tx, &ty, &margin, &spread) == ICEMPM_OK);
+    EXPECT(tx == 16 && ty == 16 && margin == 1);
+    EXPECT(icempm_partition_step(p, 3, 0) == ICEMPM_OK && launched("k_tiles") == 4);
+    fake::state().malloc_limit = 1;
+    EXPECT(icempm_partition_set_tile_shape(p, 1, 1, 0) == ICEMPM_ERR_HIP);
+    EXPECT(icempm_partition_step(p, 3, 0) == ICEMPM_OK && launched("k_tiles") == 4);
+    EXPECT(icempm_partition_sort_points(p) == ICEMPM_ERR_HIP);
+    EXPECT(icempm_partition_step(p, 3, 0) == ICEMPM_OK && launched("k_tiles") == 4);
+    fake::state().malloc_limit = ~size_t(0);
+    EXPECT(icempm_partition_sort_points(p) == ICEMPM_OK);
+    EXPECT(icempm_partition_step(p, 3, 0) == ICEMPM_OK && launched("k_tiles") == 8);
+    icempm_partition_destroy(p);
+}
+
 const struct {
     const char *name;
     void (*check)();
 } checks[] = {
     {"empty_scene", empty_scene},
     {"huge_tile_table", huge_tile_table},
+    {"no_memory_for_tiles", no_memory_for_tiles},
 };
 
 }  // namespace
