@@ -509,17 +509,27 @@ int Engine::alloc_bins()
     const long long np = std::max<long long>(n_pts_space_, 1), nc = std::max<long long>(bins_.n_cells_total, 1);
     // the scan's block sums, or the tile census
     const long long nscan = std::max(np, nc) / 1000 + 64 + sizeof(TileCensus) / sizeof(int) * TileShapes::kMax;
-    const long long n_int = 3 * np + 3 * nc + nscan + nscenes() + 16;
+    long long n_int = 0;
+    // each part 64-byte aligned: launch_fill_zero clears some of them
+    auto part = [&](long long n) {
+        int *p = (int *)bin_mem_ + n_int;
+        n_int += round_up(n, 16);
+        return p;
+    };
+    auto layout = [&] {
+        n_int = 0;
+        bins_.keys = part(np);
+        bins_.perm = part(np);
+        bins_.sorted_keys = part(np);
+        bins_.cell_count = part(nc);
+        bins_.cell_fill = part(nc);
+        bins_.cell_start = part(nc);
+        bins_.scan_tmp = part(nscan);
+        bins_.scene_count = part(nscenes());
+    };
+    layout();   // the size
     HIPCHK(hipMalloc(&bin_mem_, sizeof(int) * n_int));
-    int *p = (int *)bin_mem_;
-    bins_.keys = p; p += np;
-    bins_.perm = p; p += np;
-    bins_.sorted_keys = p; p += np;
-    bins_.cell_count = p; p += nc;
-    bins_.cell_fill = p; p += nc;
-    bins_.cell_start = p; p += nc;
-    bins_.scan_tmp = p; p += nscan;
-    bins_.scene_count = p;
+    layout();
     HIPCHK(hipMemsetAsync(bin_mem_, 0, sizeof(int) * n_int, stream_));
     return alloc_tiles();
 }

@@ -109,6 +109,26 @@ void no_memory_for_tiles()
     icempm_partition_destroy(p);
 }
 
+// The zero-fill kernel stores 16 bytes at a time: everything it clears is
+// aligned to that, also behind tables of odd length (cells + 1 of each scene).
+void fill_alignment()
+{
+    for (int gy : {32, 33}) {
+        for (int gx : {64, 65, 67}) {
+            const icempm_simparams P = params(gx, gy);
+            icempm_partition *p = partition(P, 100);
+            std::vector<double> soa(16 * 100);
+            EXPECT(icempm_partition_transfer_points_from_soa_to_device(p, soa.data(), 100, 0, 100) == ICEMPM_OK);
+            EXPECT(icempm_partition_sort_points(p) == ICEMPM_OK);
+            EXPECT(icempm_partition_step(p, 2, ICEMPM_STEP_DIRECT_P2G) == ICEMPM_OK);
+            EXPECT(icempm_partition_reset_indenter_force_accumulator(p) == ICEMPM_OK);
+            icempm_partition_destroy(p);
+        }
+    }
+    EXPECT(launched("k_fill_zero") > 0);
+    for (auto &l : fake::state().launches) EXPECT((size_t)l.pointer % 16 == 0);
+}
+
 const struct {
     const char *name;
     void (*check)();
@@ -116,6 +136,7 @@ const struct {
     {"empty_scene", empty_scene},
     {"huge_tile_table", huge_tile_table},
     {"no_memory_for_tiles", no_memory_for_tiles},
+    {"fill_alignment", fill_alignment},
 };
 
 }  // namespace
