@@ -122,7 +122,11 @@ __global__ void __launch_bounds__(kBlock) k_read(const unsigned *src, unsigned *
 }  // namespace
 
 // Pinned memory for the chunks in flight of one transfer, and an event per
-// chunk, of one device.
+// chunk, of one device.  The host reads a chunk after its event alone, and the
+// next kernel reads what the host wrote, so the memory is coherent: without
+// that flag it need not be, and an event need not make a kernel's stores
+// visible to the host.  (It costs nothing: 4.0M points 12.24 ms up and 9.87
+// down with it, 12.25 and 9.87 without.)
 struct Staging {
     int device = 0;
     double *mem = nullptr;
@@ -221,7 +225,9 @@ public:
         }
         std::unique_ptr<Staging> st(new Staging);
         st->device = device;
-        if ((e = hipHostMalloc((void **)&st->mem, bytes, hipHostMallocPortable)) != hipSuccess) return nullptr;
+        if ((e = hipHostMalloc((void **)&st->mem, bytes, hipHostMallocPortable | hipHostMallocCoherent)) !=
+            hipSuccess)
+            return nullptr;
         st->bytes = bytes;
         for (hipEvent_t &ev : st->ev)
             if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return nullptr;

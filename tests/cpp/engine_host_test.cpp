@@ -129,6 +129,20 @@ void fill_alignment()
     for (auto &l : fake::state().launches) EXPECT((size_t)l.pointer % 16 == 0);
 }
 
+// The staging memory of the transfers is coherent by its own flags: the host
+// reads a chunk that a kernel wrote after the chunk's event.
+void coherent_staging()
+{
+    const icempm_simparams P = params(64, 32);
+    icempm_partition *p = partition(P, 100);
+    std::vector<double> soa(16 * 100);
+    EXPECT(icempm_partition_transfer_points_from_soa_to_device(p, soa.data(), 100, 0, 100) == ICEMPM_OK);
+    EXPECT(icempm_partition_transfer_from_device(p, soa.data(), 100, 0) == ICEMPM_OK);
+    EXPECT(!fake::state().host_flags.empty());
+    for (unsigned f : fake::state().host_flags) EXPECT(f & hipHostMallocCoherent);
+    icempm_partition_destroy(p);
+}
+
 const struct {
     const char *name;
     void (*check)();
@@ -137,6 +151,7 @@ const struct {
     {"huge_tile_table", huge_tile_table},
     {"no_memory_for_tiles", no_memory_for_tiles},
     {"fill_alignment", fill_alignment},
+    {"coherent_staging", coherent_staging},
 };
 
 }  // namespace
