@@ -59,6 +59,21 @@ struct SceneHost {
 
 class TransferPool;   // transfer.hip
 
+// Makes a device current for a scope: memory and events belong to the device
+// current at their creation, which need not be the engine's where one thread
+// drives several.
+struct OnDevice {
+    int before = -1;
+    explicit OnDevice(int device)
+    {
+        int d = device;
+        if (hipGetDevice(&d) == hipSuccess && d != device && hipSetDevice(device) == hipSuccess) before = d;
+    }
+    ~OnDevice() { if (before >= 0) hipSetDevice(before); }
+    OnDevice(const OnDevice &) = delete;
+    OnDevice &operator=(const OnDevice &) = delete;
+};
+
 class Engine {
 public:
     // Units of a substep call (see emit_units in engine.hip).

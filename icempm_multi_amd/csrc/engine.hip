@@ -578,6 +578,7 @@ int Engine::alloc_tiles()
             std::max(tbytes, std::min(table_bytes(kMinTile[0], kMinTile[1], n_cus_ * 8), kTileMemStart));
         if (tile_mem_) { hipFree(tile_mem_); tile_mem_ = nullptr; }
         tile_mem_bytes_ = 0;
+        const OnDevice here(device_);
         const hipError_t e = hipMalloc(&tile_mem_, bytes);
         if (e != hipSuccess) {
             tile_mem_ = nullptr;
@@ -828,6 +829,7 @@ void Engine::timed_begin(bool timed)
     // while a graph is being captured)
     if (ev_used_ >= 4096 && !capturing_) collect_timings();
     if (ev_used_ == ev_pool_.size()) {
+        const OnDevice here(device_);
         hipEvent_t a, b;
         hipEventCreateWithFlags(&a, hipEventDisableSystemFence);
         hipEventCreateWithFlags(&b, hipEventDisableSystemFence);

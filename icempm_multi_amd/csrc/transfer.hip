@@ -211,7 +211,7 @@ public:
         cv_.notify_all();
         for (auto &t : threads_) t.join();
     }
-    // Staging of at least `bytes` on the current device; null and e set if there is none to be had.
+    // Staging of at least `bytes` for a device; null and e set if there is none to be had.
     std::unique_ptr<Staging> take(int device, size_t bytes, hipError_t &e)
     {
         {
@@ -229,6 +229,7 @@ public:
             hipSuccess)
             return nullptr;
         st->bytes = bytes;
+        const OnDevice here(device);
         for (hipEvent_t &ev : st->ev)
             if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return nullptr;
         return st;

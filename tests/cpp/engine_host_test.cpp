@@ -143,6 +143,26 @@ void coherent_staging()
     icempm_partition_destroy(p);
 }
 
+// One thread drives a partition on each of two devices: transfers of either
+// work whichever device is current, and leave it as it is.
+void two_devices()
+{
+    fake::state().n_devices = 2;
+    const icempm_simparams P = params(64, 32);
+    icempm_partition *a = partition(P, 100, ICEMPM_PRECISION_FP64, 0), *b = partition(P, 100, ICEMPM_PRECISION_FP64, 1);
+    std::vector<double> soa(16 * 100);
+    for (int current : {0, 1}) {
+        for (icempm_partition *p : {a, b}) {
+            fake::state().device = current;
+            EXPECT(icempm_partition_transfer_points_from_soa_to_device(p, soa.data(), 100, 0, 100) == ICEMPM_OK);
+            EXPECT(icempm_partition_transfer_from_device(p, soa.data(), 100, 0) == ICEMPM_OK);
+            EXPECT(fake::state().device == current);
+        }
+    }
+    icempm_partition_destroy(a);
+    icempm_partition_destroy(b);
+}
+
 const struct {
     const char *name;
     void (*check)();
@@ -152,6 +172,7 @@ const struct {
     {"no_memory_for_tiles", no_memory_for_tiles},
     {"fill_alignment", fill_alignment},
     {"coherent_staging", coherent_staging},
+    {"two_devices", two_devices},
 };
 
 }  // namespace
