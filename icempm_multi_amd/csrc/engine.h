@@ -145,6 +145,7 @@ private:
     const std::shared_ptr<TransferPool> &transfer_pool();
     int import_points(int scene, const double *hssoa, size_t capacity, long long offset, long long n);
     int export_points(int scene, double *hssoa, size_t capacity, long long offset, long long n);
+    int copy_points(int scene, double *host, size_t capacity, long long n, bool to_host);
     // Device words to the host once the stream has reached this point.
     int read_back(void *dst, const void *src, size_t bytes);
     int alloc_bins();

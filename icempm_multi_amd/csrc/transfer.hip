@@ -46,31 +46,38 @@ struct PosMap {
     int origin[2];
 };
 
+template <class To, class From>
+__host__ __device__ __forceinline__ To bits_as(From v)
+{
+    static_assert(sizeof(To) == sizeof(From), "the same bits");
+    return __builtin_bit_cast(To, v);
+}
+
 // One element of a line from the mixed form to FP64 bits.
-__device__ __forceinline__ unsigned long long widen(int line, unsigned v, const PosMap &m)
+__host__ __device__ __forceinline__ unsigned long long widen(int line, unsigned v, const PosMap &m)
 {
     if (line == kLineUtility) return v;
     double d;
     if (line == kLinePosX || line == kLinePosX + 1) {
         d = ((double)v * m.inv - m.origin[line - kLinePosX]) * m.h;
     } else {
-        d = (double)__uint_as_float(v);
+        d = (double)bits_as<float>(v);
         if (line == kLineJp || line == kLineFe00 || line == kLineFe00 + 3) d += 1.0;   // stored as the difference from 1
     }
-    return (unsigned long long)__double_as_longlong(d);
+    return bits_as<unsigned long long>(d);
 }
 
 // And back.
-__device__ __forceinline__ unsigned narrow(int line, unsigned long long v, const PosMap &m)
+__host__ __device__ __forceinline__ unsigned narrow(int line, unsigned long long v, const PosMap &m)
 {
     if (line == kLineUtility) return (unsigned)v;
-    double d = __longlong_as_double((long long)v);
+    double d = bits_as<double>(v);
     if (line == kLinePosX || line == kLinePosX + 1) {
         const double q = rint((d * m.hinv + m.origin[line - kLinePosX]) * m.scale);
         return q > 0 ? (unsigned)fmin(q, 4294967295.0) : 0u;   // clamped to the fixed-point range (NaN: 0)
     }
     if (line == kLineJp || line == kLineFe00 || line == kLineFe00 + 3) d -= 1.0;
-    return __float_as_uint((float)d);
+    return bits_as<unsigned>((float)d);
 }
 
 // Points [first, first + m) of the device lines to staging, line l at
@@ -211,8 +218,8 @@ public:
         cv_.notify_all();
         for (auto &t : threads_) t.join();
     }
-    // Staging of at least `bytes` for a device; null and e set if there is none to be had.
-    std::unique_ptr<Staging> take(int device, size_t bytes, hipError_t &e)
+    // Staging of at least `bytes` for a device; null if there is none to be had.
+    std::unique_ptr<Staging> take(int device, size_t bytes)
     {
         {
             std::lock_guard<std::mutex> lock(m_);
@@ -225,14 +232,15 @@ public:
         }
         std::unique_ptr<Staging> st(new Staging);
         st->device = device;
-        if ((e = hipHostMalloc((void **)&st->mem, bytes, hipHostMallocPortable | hipHostMallocCoherent)) !=
-            hipSuccess)
-            return nullptr;
+        hipError_t e = hipHostMalloc((void **)&st->mem, bytes, hipHostMallocPortable | hipHostMallocCoherent);
+        if (e != hipSuccess) st->mem = nullptr;
         st->bytes = bytes;
         const OnDevice here(device);
         for (hipEvent_t &ev : st->ev)
-            if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return nullptr;
-        return st;
+            if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+        if (e == hipSuccess) return st;
+        hipGetLastError();   // the caller does without: not the error of its next launch
+        return nullptr;
     }
     void give_back(std::unique_ptr<Staging> st)
     {
@@ -352,6 +360,30 @@ static PosMap position_map(const SceneConsts &c)
     return m;
 }
 
+// A transfer without staging, where there is no pinned memory to be had: line
+// by line from or to the caller's memory, the mixed form's elements converted
+// by this thread.  Many times slower.
+int Engine::copy_points(int scene, double *host, size_t capacity, long long n, bool to_host)
+{
+    const PosMap map = position_map(host_dev_[scene].c);
+    const size_t eb = elem_bytes();
+    std::vector<unsigned> words(eb == 4 ? n : 0);
+    for (int line = 0; line < kNumPtsLines; line++) {
+        char *const dev = (char *)pts_[0] + (line * pitch_ + scenes_[scene].pt_off) * eb;
+        double *const h = host + line * capacity;
+        void *const mem = eb == 4 ? (void *)words.data() : (void *)h;
+        for (long long i = 0; i < (long long)words.size() && !to_host; i++)
+            words[i] = narrow(line, bits_as<unsigned long long>(h[i]), map);
+        hipError_t e = to_host ? hipMemcpyAsync(mem, dev, eb * n, hipMemcpyDeviceToHost, stream_)
+                               : hipMemcpyAsync(dev, mem, eb * n, hipMemcpyHostToDevice, stream_);
+        if (e == hipSuccess) e = hipStreamSynchronize(stream_);
+        if (e != hipSuccess) return hipfail(e, "point transfer");
+        for (long long i = 0; i < (long long)words.size() && to_host; i++)
+            h[i] = bits_as<double>(widen(line, words[i], map));
+    }
+    return ICEMPM_OK;
+}
+
 int Engine::import_points(int scene, const double *hssoa, size_t capacity, long long offset, long long n)
 {
     if (n <= 0) return ICEMPM_OK;
@@ -365,8 +397,8 @@ int Engine::import_points(int scene, const double *hssoa, size_t capacity, long 
     job.to_host = false;
     const long long chunk = job.chunk, n_chunks = (n + chunk - 1) / chunk, first = scenes_[scene].pt_off;
     const int depth = job.depth = (int)std::min<long long>(kStageDepth, n_chunks);
-    t.st = t.pool->take(device_, (size_t)chunk * depth * kNumPtsLines * sizeof(double), e);
-    if (!t.st) return hipfail(e, "transfer staging");
+    t.st = t.pool->take(device_, (size_t)chunk * depth * kNumPtsLines * sizeof(double));
+    if (!t.st) return copy_points(scene, job.host, capacity, n, job.to_host);
     job.stage = t.st->mem;
     const PosMap map = position_map(host_dev_[scene].c);
     t.begin();
@@ -400,8 +432,8 @@ int Engine::export_points(int scene, double *hssoa, size_t capacity, long long o
     job.to_host = true;
     const long long chunk = job.chunk, n_chunks = (n + chunk - 1) / chunk, first = scenes_[scene].pt_off;
     const int depth = job.depth = (int)std::min<long long>(kStageDepth, n_chunks);
-    t.st = t.pool->take(device_, (size_t)chunk * depth * kNumPtsLines * sizeof(double), e);
-    if (!t.st) return hipfail(e, "transfer staging");
+    t.st = t.pool->take(device_, (size_t)chunk * depth * kNumPtsLines * sizeof(double));
+    if (!t.st) return copy_points(scene, job.host, capacity, n, job.to_host);
     job.stage = t.st->mem;
     const PosMap map = position_map(host_dev_[scene].c);
     auto launch = [&](long long k) {
@@ -430,7 +462,7 @@ int Engine::read_back(void *dst, const void *src, size_t bytes)
     constexpr size_t kMost = 64 * 1024;
     hipError_t e = hipSuccess;
     Transfer t(transfer_pool(), stream_);
-    if (bytes <= kMost && bytes % sizeof(unsigned) == 0) t.st = t.pool->take(device_, kMost, e);
+    if (bytes <= kMost && bytes % sizeof(unsigned) == 0) t.st = t.pool->take(device_, kMost);
     if (!t.st) {
         e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream_);
         if (e == hipSuccess) e = hipStreamSynchronize(stream_);

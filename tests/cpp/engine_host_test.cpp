@@ -1,6 +1,7 @@
 // Host side of the engine on the runtime of fake_hip.cpp: one check per name.
 #include "fake_hip.h"
 
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <functional>
@@ -163,6 +164,49 @@ void two_devices()
     icempm_partition_destroy(b);
 }
 
+// Without pinned memory the transfers and the queries still work, with the
+// same values: FP64 bits as they were, the mixed form's elements in FP32 (Jp
+// and the diagonal of F as differences from 1) and positions to its fixed point.
+void no_pinned_memory()
+{
+    fake::state().host_malloc_fails = true;
+    constexpr int n = 700, capacity = 900, offset = 13;
+    const icempm_simparams P = params(64, 32);
+    std::vector<double> soa(16 * capacity), out(16 * capacity, -1.0);
+    for (int line = 0; line < 16; line++)
+        for (int i = 0; i < n; i++) {
+            double v = 0.25 + 1e-3 * i + 0.1 * line;
+            if (line == 0) {
+                const long long ud = 1000 + i;
+                std::memcpy(&v, &ud, 8);
+            }
+            soa[line * capacity + offset + i] = v;
+        }
+    for (int precision : {ICEMPM_PRECISION_FP64, ICEMPM_PRECISION_MIXED}) {
+        icempm_partition *p = partition(P, n, precision);
+        EXPECT(icempm_partition_transfer_points_from_soa_to_device(p, soa.data(), capacity, offset, n) == ICEMPM_OK);
+        uint8_t code = 1;
+        EXPECT(icempm_partition_get_error_code(p, &code) == ICEMPM_OK && code == 0);
+        EXPECT(icempm_partition_transfer_from_device(p, out.data(), capacity, offset) == ICEMPM_OK);
+        for (int line = 0; line < 16; line++)
+            for (int i = 0; i < n; i++) {
+                const double want = soa[line * capacity + offset + i], got = out[line * capacity + offset + i];
+                const bool one = line == 3 || line == 8 || line == 11, pos = line == 4 || line == 5;
+                if (precision == ICEMPM_PRECISION_FP64 || line == 0)
+                    EXPECT(std::memcmp(&want, &got, 8) == 0);
+                else if (pos)
+                    EXPECT(std::abs(got - want) <= P.cellsize / (1 << 22));
+                else
+                    EXPECT(got == (one ? 1.0 + (double)(float)(want - 1.0) : (double)(float)want));
+            }
+        EXPECT(out[offset - 1] == -1.0 && out[16 * capacity - 1] == -1.0);
+        EXPECT(icempm_partition_step(p, 2, 0) == ICEMPM_OK);
+        EXPECT(icempm_partition_sort_points(p) == ICEMPM_OK);
+        EXPECT(icempm_partition_step(p, 2, 0) == ICEMPM_OK);
+        icempm_partition_destroy(p);
+    }
+}
+
 const struct {
     const char *name;
     void (*check)();
@@ -173,6 +217,7 @@ const struct {
     {"fill_alignment", fill_alignment},
     {"coherent_staging", coherent_staging},
     {"two_devices", two_devices},
+    {"no_pinned_memory", no_pinned_memory},
 };
 
 }  // namespace
