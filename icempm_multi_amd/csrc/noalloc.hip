@@ -202,6 +202,7 @@ int icempm_substeps_noalloc(int device, const icempm_simparams *prms, size_t prm
     d.ncells = (int)nodes;
     d.force_off = 0;
     d.seg_off = 0;
+    d.ind_scene = d.c.ind_rsq > 0 ? 0 : -1;
     SceneClock ck{};
     ck.t = P.SimulationTime;
     ck.ind_x = P.indenter_x;

@@ -156,7 +156,11 @@ __device__ __forceinline__ bool side_work(const StepArgs &a, int rb, int zb, int
 {
     block = blockIdx.x - a.n_service;
     if (block < 0) {
-        for (int sc = blockIdx.x; sc < a.nscenes; sc += a.n_service) indenter_force_nodes(a, sc, rb);
+        for (int k = blockIdx.x; k < a.nscenes; k += a.n_service) {
+            const int sc = a.scenes[k].ind_scene;
+            if (sc < 0) break;
+            indenter_force_nodes(a, sc, rb);
+        }
         return true;
     }
     if (block < a.n_work) return false;

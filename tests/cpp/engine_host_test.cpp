@@ -207,6 +207,35 @@ void no_pinned_memory()
     }
 }
 
+// The substep launches of a batch have a workgroup for each scene with an
+// indenter, as many as there are compute units, and none for the others.
+void indenter_workgroups()
+{
+    unsigned grid[4];
+    const int n_scenes = 300, with_indenter[4] = {0, 1, 200, 300};
+    for (int c = 0; c < 4; c++) {
+        icempm_batch *b = nullptr;
+        EXPECT(icempm_batch_create(0, ICEMPM_PRECISION_FP64, &b) == ICEMPM_OK);
+        std::vector<double> soa(16);
+        for (int i = 0; i < n_scenes; i++) {
+            icempm_simparams P = params(64, 32);
+            P.IndRSq = i >= n_scenes - with_indenter[c] ? 1.0 : 0.0;
+            int id;
+            EXPECT(icempm_batch_add_scene(b, &P, sizeof P, soa.data(), 1, 1, &id) == ICEMPM_OK);
+        }
+        EXPECT(icempm_batch_commit(b) == ICEMPM_OK);
+        fake::state().launches.clear();
+        EXPECT(icempm_batch_step(b, 2, ICEMPM_STEP_RESORT) == ICEMPM_OK);
+        grid[c] = 0;
+        for (auto &l : fake::state().launches)
+            if (l.name.find("k_tiles") != std::string::npos) grid[c] = l.grid.x;   // of the last, with the indenter
+        icempm_batch_destroy(b);
+    }
+    EXPECT(grid[1] - grid[0] == 1);
+    EXPECT(grid[2] - grid[0] == 200);
+    EXPECT(grid[3] - grid[0] == 256);
+}
+
 const struct {
     const char *name;
     void (*check)();
@@ -218,6 +247,7 @@ const struct {
     {"coherent_staging", coherent_staging},
     {"two_devices", two_devices},
     {"no_pinned_memory", no_pinned_memory},
+    {"indenter_workgroups", indenter_workgroups},
 };
 
 }  // namespace

@@ -149,3 +149,33 @@ def test_floe_fields_batched_mixed_and_fp64():
             assert d <= 1e-9 * s, f"floes {i} {name}: {d:.3e} vs {s:.3e}"
         rel = np.linalg.norm(outs_m[i][4:6, :n] - ref[4:6, :n]) / np.linalg.norm(ref[4:6, :n])
         assert rel <= 1e-4, (i, rel)
+
+
+# more scenes with an indenter than compute units, with scenes without one among them
+@pytest.mark.parametrize("precision", [im.PRECISION_FP64, im.PRECISION_MIXED])
+def test_indenter_forces_of_many_scenes(precision):
+    bag = []
+    for i in range(340):
+        P, h, n = scenes.sheet_scene(seed=0x1CE0C00 + i, nx=12 + i % 5, ny=6 + i % 3, grid=(48, 24), h=0.05,
+                                     ind_diameter=0.2, ind_depth=0.04, n_grains=5, sampler="jittered")
+        if i % 5 == 2:
+            P.IndRSq = 0.0
+        h[6, :n] = 0.3 * np.sin(h[4, :n] + i)
+        h[7, :n] = 0.4
+        bag.append((P, h, n))
+    assert sum(P.IndRSq > 0 for P, _, _ in bag) == 272
+    b, _, forces = run_batch(bag, precision, 0)
+    assert b.error_code == 0
+    tol = 1e-8 if precision == im.PRECISION_FP64 else 2e-3
+    touched = 0
+    for i, (P, h, n) in enumerate(bag):
+        ref = h.copy()
+        O.sort(P, ref, n)
+        _, _, fref, err = O.substeps(P, ref, n, 20, 0.0, 0)
+        assert err == 0
+        f, r = forces[i].reshape(-1, 2).sum(0), fref.reshape(-1, 2).sum(0)
+        touched += np.abs(r).max() > 0
+        assert np.abs(f - r).max() <= tol * np.abs(r).max(), i
+        if i % 5 == 2:
+            assert not forces[i].any()
+    assert touched > 256
