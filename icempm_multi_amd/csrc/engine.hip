@@ -722,7 +722,7 @@ int Engine::choose_tile_shape()
     }
     static_assert(n <= TileShapes::kMax, "shapes to count");
     TileCensus *const d_census = (TileCensus *)bins_.scan_tmp;
-    HIPCHK(launch_tile_census(args(), shapes, bins_.n_cells_total, d_census, stream_));
+    HIPCHK(launch_tile_census(args(), shapes, bins_, d_census, stream_));
     TileCensus census[n];
     RC(read_back(census, d_census, sizeof census));
     int pick = n - 2;

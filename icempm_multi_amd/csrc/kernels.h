@@ -74,7 +74,7 @@ struct BinWork {
 hipError_t launch_sort(const StepArgs &a, const SceneDev *host_scenes, int nscenes, BinWork &w, int elem_bytes,
                        void *pts_src, void *pts_dst, hipStream_t s);
 // Tile shapes to count the tiles of (launch_tile_census: counts[i] = tiles of
-// shape i that hold points, by the current cell_start).
+// shape i that hold points, by the points as last sorted).
 struct TileShapes {
     static constexpr int kMax = 8;
     int n = 0;
@@ -87,7 +87,7 @@ struct TileCensus {
     int tiles[kPasses];
     int most, points;
 };
-hipError_t launch_tile_census(const StepArgs &a, const TileShapes &shapes, long long n_cells, TileCensus *out,
+hipError_t launch_tile_census(const StepArgs &a, const TileShapes &shapes, const BinWork &w, TileCensus *out,
                               hipStream_t s);
 // Phase calls' times: stamps of launches (StepArgs::stamp, kStampStride words
 // each), summed by class into ticks.

@@ -236,6 +236,21 @@ void indenter_workgroups()
     EXPECT(grid[3] - grid[0] == 256);
 }
 
+// The count of the tiles that decides a scene's tile shape is made by the
+// points: few of them on a huge grid take a small launch.
+void census_by_points()
+{
+    const icempm_simparams P = params(8000, 8000);
+    icempm_partition *p = partition(P, 1000);
+    std::vector<double> soa(16 * 1000);
+    EXPECT(icempm_partition_transfer_points_from_soa_to_device(p, soa.data(), 1000, 0, 1000) == ICEMPM_OK);
+    EXPECT(icempm_partition_sort_points(p) == ICEMPM_OK);
+    EXPECT(launched("k_tile_census") == 1);
+    for (auto &l : fake::state().launches)
+        if (l.name.find("k_tile_census") != std::string::npos) EXPECT(l.grid.x * l.grid.y <= 4);
+    icempm_partition_destroy(p);
+}
+
 const struct {
     const char *name;
     void (*check)();
@@ -248,6 +263,7 @@ const struct {
     {"two_devices", two_devices},
     {"no_pinned_memory", no_pinned_memory},
     {"indenter_workgroups", indenter_workgroups},
+    {"census_by_points", census_by_points},
 };
 
 }  // namespace

@@ -9,7 +9,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIBDIR = os.path.join(ROOT, "icempm_multi_amd")
 CHECKS = ["empty_scene", "huge_tile_table", "no_memory_for_tiles", "fill_alignment", "coherent_staging",
-          "two_devices", "no_pinned_memory", "indenter_workgroups"]
+          "two_devices", "no_pinned_memory", "indenter_workgroups", "census_by_points"]
 
 
 @pytest.fixture(scope="module")
