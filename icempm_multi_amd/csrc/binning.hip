@@ -556,10 +556,12 @@ hipError_t launch_tile_census(const StepArgs &a, const TileShapes &shapes, const
     return hipGetLastError();
 }
 
-// The parts of a tile table of at most max_tiles tiles in one allocation: the
+// The parts of a tile table of max_tiles places in one allocation, no more of
+// which than there are points can hold any (a small shape on a huge grid has
+// many times more places): the
 // workgroups' work, the items, their runs, the tile count, and the builder's
 // own ints (scene offsets, flags, positions or weight sums, weights, scan sums).
-size_t tile_table_layout(char *base, long long max_tiles, int tx, int n_work, TileTable &t)
+size_t tile_table_layout(char *base, long long max_tiles, long long max_points, int tx, int n_work, TileTable &t)
 {
     size_t at = 0;
     auto part = [&](size_t bytes) {
@@ -567,16 +569,18 @@ size_t tile_table_layout(char *base, long long max_tiles, int tx, int n_work, Ti
         at = (at + bytes + 63) / 64 * 64;
         return p;
     };
+    const long long live = std::min(max_tiles, max_points);
     t.max_tiles = max_tiles;
+    t.max_live = live;
     t.n_work = n_work;
     t.work = (TileWork *)part(sizeof(TileWork) * n_work);
-    t.tiles = (TileItem *)part(sizeof(TileItem) * max_tiles);
-    t.list = (TileItem *)part(sizeof(TileItem) * max_tiles);
-    t.runs = (TileRun *)part(sizeof(TileRun) * tx * max_tiles);
+    t.tiles = (TileItem *)part(sizeof(TileItem) * live);
+    t.list = (TileItem *)part(sizeof(TileItem) * live);
+    t.runs = (TileRun *)part(sizeof(TileRun) * tx * live);
     t.n_tiles = (int *)part(sizeof(int));
     t.flag = (int *)part(sizeof(int) * max_tiles);
     t.pos = (int *)part(sizeof(int) * max_tiles);
-    t.weight = (int *)part(sizeof(int) * max_tiles);
+    t.weight = (int *)part(sizeof(int) * live);
     t.scan_tmp = (int *)part(sizeof(int) * (max_tiles / 1000 + 64));
     return at;
 }
@@ -598,7 +602,7 @@ hipError_t launch_build_tiles(const StepArgs &a, const SceneDev *host_scenes, in
     hipLaunchKernelGGL(k_tile_emit, dim3(g), dim3(kBlock), 0, s, a, (int)total, t.flag, t.pos, t.tiles,
                        t.runs, t.weight, tile_cost, t.n_tiles);
     // (weights past the live tiles are not read from the sums)
-    if ((e = scan_exclusive(t.weight, t.pos, total, t.scan_tmp, s)) != hipSuccess) return e;
+    if ((e = scan_exclusive(t.weight, t.pos, std::min(total, t.max_live), t.scan_tmp, s)) != hipSuccess) return e;
     const int parts = t.n_work % 8 ? 1 : 8;
     hipLaunchKernelGGL(k_tile_split, dim3(parts), dim3(kBlock), 0, s, t.tiles, t.weight, t.pos, t.n_tiles, t.list,
                        t.work, t.n_work, t.n_few, parts);

@@ -151,7 +151,7 @@ private:
     int alloc_bins();
     int alloc_tiles();
     long long count_tiles(int tx, int ty) const;
-    size_t table_bytes(int tx, int ty, int n_work) const;
+    size_t table_bytes(int tx, int ty, int n_work) const;   // with points everywhere
     int apply_tile_shape(int tx, int ty, int margin);
     int choose_tile_shape();
     StepArgs args() const;

@@ -552,7 +552,8 @@ long long Engine::count_tiles(int tx, int ty) const
 size_t Engine::table_bytes(int tx, int ty, int n_work) const
 {
     TileTable t;
-    return tile_table_layout(nullptr, count_tiles(tx, ty), tx, n_work, t);
+    const long long places = count_tiles(tx, ty);
+    return tile_table_layout(nullptr, places, places, tx, n_work, t);
 }
 
 // The tile table for the current shape.
@@ -575,7 +576,7 @@ int Engine::alloc_tiles()
     const int r_few = LAUNCH_PREC(tiles_resident_per_cu, f, kTileChain);
     int n_few = (int)std::min<long long>(n_work, (long long)n_cus_ * std::max(r_few, 0));
     if (n_work % 8 == 0 && n_few % 8) n_few = 0;   // one share per XCD
-    const size_t tbytes = tile_table_layout(nullptr, mt, tx_, n_work, tiles_);
+    const size_t tbytes = tile_table_layout(nullptr, mt, n_pts_space_, tx_, n_work, tiles_);
     if (tbytes > tile_mem_bytes_) {
         // room for the smallest shape choose_tile_shape() may take, unless the
         // grids are huge: no second allocation when it does
@@ -592,7 +593,7 @@ int Engine::alloc_tiles()
         }
         tile_mem_bytes_ = bytes;
     }
-    tile_table_layout((char *)tile_mem_, mt, tx_, n_work, tiles_);
+    tile_table_layout((char *)tile_mem_, mt, n_pts_space_, tx_, n_work, tiles_);
     tiles_.n_few = n_few;
     HIPCHK(launch_fill_zero(tiles_.work, sizeof(TileWork) * n_work, stream_));   // no tiles until the next build
     return ICEMPM_OK;
@@ -727,13 +728,14 @@ int Engine::choose_tile_shape()
     RC(read_back(census, d_census, sizeof census));
     int pick = n - 2;
     double best = 1e300;
+    const size_t most = std::max(table_bytes(ladder[pick][0], ladder[pick][1], n_cus_ * 8), kTileMemStart);
     for (int i = 0; i < n; i++) {
         StepArgs a = args();
         a.few = 0;
         a.tx = shapes.tx[i];
         a.ty = shapes.ty[i];
         set_window(a, a.tx, a.ty, margin_, precision_);
-        if (i < n - 2 && table_bytes(a.tx, a.ty, n_cus_ * 8) > std::max(tile_mem_bytes_, kTileMemStart)) continue;
+        if (i < n - 2 && table_bytes(a.tx, a.ty, n_cus_ * 8) > most) continue;
         const int r = LAUNCH_PREC(tiles_resident_per_cu, a, kTileChain);
         if (r <= 0) continue;
         const TileCensus &t = census[i];
@@ -1092,7 +1094,7 @@ int Engine::build_tiles()
     HIPCHK(launch_build_tiles(a, host_dev_.data(), nscenes(), total_points(), tiles_, stream_));
     int nt = 0;
     RC(read_back(&nt, tiles_.n_tiles, sizeof(int)));
-    if (nt < 0 || nt > tiles_.max_tiles) {
+    if (nt < 0 || nt > tiles_.max_live) {
         bins_valid_ = false;
         return fail(ICEMPM_ERR_STATE, "build_tiles: tile count out of range");
     }

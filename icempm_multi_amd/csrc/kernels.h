@@ -100,7 +100,8 @@ hipError_t launch_sum_stamps(const unsigned long long *stamps, const StampClasse
                              hipStream_t s);
 // The tile table of the binned kernels (mpm_common.h) and its builder's memory.
 struct TileTable {
-    long long max_tiles = 0;
+    long long max_tiles = 0;      // places of tiles
+    long long max_live = 0;       // tiles that can hold points
     int n_work = 0;               // workgroups of a tile launch
     int n_few = 0;                // workgroups where no more tiles than these are found (0: always n_work)
     TileWork *work = nullptr;
@@ -111,7 +112,7 @@ struct TileTable {
     int *flag = nullptr, *pos = nullptr, *weight = nullptr, *scan_tmp = nullptr;
 };
 // Lays the table out from base (null: only counts); returns its bytes.
-size_t tile_table_layout(char *base, long long max_tiles, int tx, int n_work, TileTable &t);
+size_t tile_table_layout(char *base, long long max_tiles, long long max_points, int tx, int n_work, TileTable &t);
 hipError_t launch_build_tiles(const StepArgs &a, const SceneDev *host_scenes, int nscenes, long long n_points,
                               const TileTable &t, hipStream_t s);
 

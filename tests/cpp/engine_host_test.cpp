@@ -70,12 +70,16 @@ void empty_scene()
 }
 
 // A table of more than 2^27 tiles (the smallest shape on a grid of 135M cells):
-// no launch of 2^32 threads or more, which the runtime refuses.
+// no launch of 2^32 threads or more, which the runtime refuses, and of the
+// table no more than flags and positions (8 bytes) for the places that cannot
+// all hold one of the few points.
 void huge_tile_table()
 {
     const icempm_simparams P = params(16400, 8200);
     icempm_partition *p = partition(P, 100);
+    fake::state().allocated.clear();
     EXPECT(icempm_partition_set_tile_shape(p, 1, 1, 1) == ICEMPM_OK);
+    for (size_t bytes : fake::state().allocated) EXPECT(bytes < (9ull << 27));
     EXPECT(icempm_partition_sort_points(p) == ICEMPM_OK);
     EXPECT(launched("k_tile_count") == 1 && launched("k_tile_emit") == 1);
     for (auto &l : fake::state().launches) EXPECT((unsigned long long)l.grid.x * l.block.x < 1ull << 32);
@@ -87,13 +91,13 @@ void huge_tile_table()
 // stepped in their own order, and sorted again once there is memory.
 void no_memory_for_tiles()
 {
-    const icempm_simparams P = params(600, 400);
+    const icempm_simparams P = params(2000, 2000);
     icempm_partition *p = partition(P, 100);
     std::vector<double> soa(16 * 100);
     EXPECT(icempm_partition_transfer_points_from_soa_to_device(p, soa.data(), 100, 0, 100) == ICEMPM_OK);
     EXPECT(icempm_partition_set_tile_shape(p, 16, 16, 1) == ICEMPM_OK);
     EXPECT(icempm_partition_sort_points(p) == ICEMPM_OK);
-    fake::state().malloc_limit = 8u << 20;   // a table of 1x1 cells takes 20 MB
+    fake::state().malloc_limit = 24u << 20;   // a table of 1x1 cells takes 32 MB
     EXPECT(icempm_partition_set_tile_shape(p, 1, 1, 0) == ICEMPM_ERR_HIP);
     int tx = 0, ty = 0, margin = 0, spread = 0;
     EXPECT(icempm_partition_get_tile_config(p, &tx, &ty, &margin, &spread) == ICEMPM_OK);
