@@ -282,7 +282,7 @@ class Partition:
     def autotune(self, n_trials=5):
         """Returns (chosen index, ms per substep launch of the candidates of
         tile_candidates() at margin 0 then margin 1); tile_config() gives the
-        shape kept."""
+        shape kept.  An index past the list: the shape in force at the call."""
         k = 2 * len(tile_candidates())
         out = (C.c_float * k)()
         chosen = C.c_int(-1)

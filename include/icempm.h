@@ -281,8 +281,9 @@ int icempm_tile_candidates(int *tx, int *ty, int *lane_spread, int n);
  * and restores the state.  Results (ms
  * per substep launch; -1 for a shape that does not fit) go to out_ms if
  * non-null: the K candidates at margin 0, then at margin 1 (2K values).
- * *chosen = margin * K + candidate, the shape kept; the shape itself is read
- * with icempm_partition_get_tile_config. */
+ * *chosen = margin * K + candidate, the shape kept, or 2K for the shape in force
+ * at the call, which is timed too if it is none of them; the shape itself is
+ * read with icempm_partition_get_tile_config. */
 int icempm_partition_autotune(icempm_partition *p, int n_trials, float *out_ms, int n_out, int *chosen);
 /* The tile shape, window drift margin and lane map in use (no reference counterpart). */
 int icempm_partition_get_tile_config(icempm_partition *p, int *tx, int *ty, int *margin, int *lane_spread);

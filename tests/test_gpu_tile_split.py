@@ -115,3 +115,29 @@ def test_table_beyond_one_sweep_of_the_builder_matches_oracle():
     c = step_and_compare(P, h, n, (1, 1, 1))
     first, last = (int(t(h[4, :n]) / P.cellsize) + P.GridHaloSize for t in (np.min, np.max))
     assert first * P.GridY < 524288 < last * P.GridY and (c["tx"], c["ty"]) == (1, 1)
+
+
+# 102k points: the built-in rule takes 4x14 cells, which are no candidate of the
+# autotuner and 14% faster than the best of them
+def test_autotuner_keeps_a_faster_shape_in_force():
+    P, h, n = scenes.block_scene(nx=320, ny=80, grid=(384, 112), h=0.1, n_grains=20)
+    out = []
+    for tune in (True, False):
+        part = im.Partition(0, 0, im.PRECISION_FP64)
+        part.allocate(h.shape[1], P.GridXTotal)
+        part.update_constants(P)
+        part.transfer_points_from_soa_to_device(h, 0, n)
+        part.sort_points()
+        before = part.tile_config()
+        if tune:
+            chosen, ms = part.autotune(20)
+            assert chosen == len(ms) == 2 * len(im.capi.tile_candidates())
+        assert part.tile_config() == before and (before["tx"], before["ty"]) == (4, 14)
+        part.step(20, im.STEP_GRAPH | im.STEP_RESORT)
+        out.append(np.zeros_like(h))
+        part.transfer_from_device(out[-1], 0)
+        assert part.error_code == 0
+        part.close()
+    for name, (a, b) in FIELDS.items():
+        scale = np.abs(out[1][a:b, :n]).max()
+        assert np.abs(out[0][a:b, :n] - out[1][a:b, :n]).max() <= 1e-9 * scale, name
