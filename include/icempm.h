@@ -215,7 +215,8 @@ int icempm_partition_get_timings(icempm_partition *p, float *out, int n);
  * recorded with hipEvents around each launch when ICEMPM_STEP_TIMINGS is set
  * (around each run of back-to-back fused launches with ICEMPM_STEP_SPAN); the
  * single-phase calls are always timed, by stamps of their launch after a sort
- * (start of its first workgroup to end of its last) and by hipEvents before:
+ * (start of its first workgroup to end of its last) and by hipEvents before,
+ * whose times include the launch (about 8 us more for each):
  * class 0 clock, 1 zero-fill, 2 P2G, 3 fused G2P+P2G (the grid update folded
  * in), 4 G2P (the last of a binned call also folds the grid update in), 5 grid
  * update (unbinned and unfused stepping, and the phase calls), 6 sort.

@@ -4,6 +4,7 @@ to no more than the host's, and time in which the host does nothing between two
 calls belongs to neither."""
 import time
 
+import numpy as np
 import pytest
 
 import icempm_multi_amd as im
@@ -47,3 +48,32 @@ def test_phase_times(precision, binned, pause):
         assert total <= wall - 4 * 50 + 20    # the pauses, less 5 ms of scheduling each
     assert part.error_code == 0
     part.close()
+
+
+def test_phase_time_lasts_to_the_last_wave():
+    """A launch's time ends with its last wave, not with the first of each workgroup: a
+    grid update whose workgroups have one wave without nodes (it takes every fourth grid
+    column, a run of 64 segments) takes as long whichever wave that is."""
+    P, _, _ = scenes.block_scene(nx=20, ny=8, grid=(2100, 4096), n_grains=5)
+    ms = []
+    for first in (2, 3):        # columns of points, which touch the one before and the one after
+        x, y = np.meshgrid((np.arange(100, 500) * 4 + first) * P.cellsize, (np.arange(2, 126) * 32) * P.cellsize)
+        n = x.size
+        h = np.zeros((16, n))
+        h[3], h[4], h[5], h[8], h[11] = 1, x.ravel(), y.ravel(), 1, 1
+        part = im.Partition(0, 0, im.PRECISION_FP64)
+        part.allocate(n, P.GridXTotal)
+        part.update_constants(P)
+        part.transfer_points_from_soa_to_device(h, 0, n)
+        for i in range(13):
+            if i == 3:
+                part.reset_indenter_force_accumulator()   # and the times
+            part.reset_grid()
+            part.p2g()
+            part.update_nodes(0.0, P.indenter_x, P.indenter_y)
+        st = part.kernel_stats()
+        assert st["update"][1] == 10 and part.error_code == 0
+        ms.append(st["update"][0] / 10)
+        part.close()
+    print(ms, flush=True)
+    assert ms[0] >= 0.75 * ms[1]
