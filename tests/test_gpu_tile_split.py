@@ -141,3 +141,51 @@ def test_autotuner_keeps_a_faster_shape_in_force():
     for name, (a, b) in FIELDS.items():
         scale = np.abs(out[1][a:b, :n]).max()
         assert np.abs(out[0][a:b, :n] - out[1][a:b, :n]).max() <= 1e-9 * scale, name
+
+
+# Pairs of points 0.6 cells apart, far from each other, fly a cell and a half: with
+# tiles of one cell each pair fills one tile, then two, then one again, on both sides
+# of the count from which on the launch uses the kernel built for more waves per SIMD
+# (512 tiles in FP64, 768 in the mixed form).  The shape stays, so the captured graphs
+# do: the frames with two tiles per pair capture graphs of their own, and those of the
+# first kind serve again.
+@pytest.mark.parametrize("precision,side", [(im.PRECISION_FP64, 20), (im.PRECISION_MIXED, 25)])
+def test_few_and_many_tiles_by_motion_match_oracle(precision, side):
+    gap, frames, substeps = 8, 49, 20
+    grid = side * gap + 40
+    P, _, _ = scenes.block_scene(nx=20, ny=8, grid=(grid, grid), n_grains=5)
+    P.IndRSq = 0.0
+    i, j = (a.ravel() for a in np.meshgrid(np.arange(side), np.arange(side)))
+    x = np.concatenate([20 + gap * i + 0.52, 20 + gap * i + 1.12])      # 0.02 and 0.62 into cell 21 + 8 i
+    n = x.size
+    h = np.zeros((16, n))
+    h[3], h[8], h[11] = 1, 1, 1
+    h[4] = x * P.cellsize
+    h[5] = np.tile(20 + gap * j + 0.1, 2) * P.cellsize
+    h[6] = P.cellsize / (35 * substeps * P.InitialTimeStep)             # a cell in 35 frames
+    part = im.Partition(0, 0, precision)
+    part.allocate(n, P.GridXTotal)
+    part.update_constants(P)
+    part.set_tile_shape(1, 1, 1)
+    part.transfer_points_from_soa_to_device(h, 0, n)
+    ref = h.copy()
+    t, step, captures = 0.0, 0, []
+    print(precision, n, flush=True)
+    for k in range(frames):
+        part.step(substeps, im.STEP_GRAPH | im.STEP_RESORT)
+        captures.append(part.graph_stats()[0])
+        O.sort(P, ref, n)
+        t, step, _, err = O.substeps(P, ref, n, substeps, t, step)
+        assert err == 0
+    out = np.zeros_like(h)
+    part.transfer_from_device(out, 0)
+    assert part.error_code == 0
+    part.close()
+    # frames 0 to 13 and 35 to 48: one tile per pair; 14 to 34: two
+    assert captures[13] == captures[6] and captures[34] == 2 * captures[13] and captures[48] == captures[34]
+    tol = dict(x=1e-9, v=1e-9, F=1e-9, C=1e-9, Jp=1e-9) if precision == im.PRECISION_FP64 else dict(x=1e-6, v=1e-4)
+    for name, rtol in tol.items():
+        a, b = FIELDS[name]
+        scale = max(np.abs(ref[a:b]).max(), 1e-3 if name == "C" else 0)
+        assert np.abs(out[a:b] - ref[a:b]).max() <= rtol * scale, name
+    assert np.array_equal(out[0].view(np.int64), ref[0].view(np.int64))
