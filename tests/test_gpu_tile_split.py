@@ -189,3 +189,32 @@ def test_few_and_many_tiles_by_motion_match_oracle(precision, side):
         scale = max(np.abs(ref[a:b]).max(), 1e-3 if name == "C" else 0)
         assert np.abs(out[a:b] - ref[a:b]).max() <= rtol * scale, name
     assert np.array_equal(out[0].view(np.int64), ref[0].view(np.int64))
+
+
+# The tiles behind the built-in shape are counted by the cells on the first grid and by
+# the points on the second, which has the same cells in its first columns and rows and
+# more than 10 cells per point: the same counts, the same shape.
+@pytest.mark.parametrize("precision", [im.PRECISION_FP64, im.PRECISION_MIXED])
+@pytest.mark.parametrize("nx,ny,thin", [(16, 4, False), (61, 33, True), (320, 80, False), (375, 167, False),
+                                        (300, 260, True), (633, 158, False), (633, 158, True)])
+def test_shape_by_cells_and_by_points(nx, ny, thin, precision):
+    P, h, n = scenes.block_scene(nx=nx, ny=ny, grid=(nx + 32, ny + 20), n_grains=40)
+    r = np.random.default_rng(nx)
+    if thin:
+        keep = np.flatnonzero(r.random(n) < 0.5 + 0.5 * np.sin(0.9 * h[4, :n]) * np.cos(0.7 * h[5, :n]))
+        n = keep.size
+        h[:, :n] = h[:, keep]
+    h[0, :n].view(np.int64)[r.random(n) < 0.05] |= 0x20000              # disabled: dropped by the sort
+    side = int(np.sqrt(12.0 * h.shape[1])) + nx + ny
+    Q, _, _ = scenes.block_scene(nx=16, ny=4, grid=(side, side), n_grains=4)
+    assert Q.cellsize == P.cellsize
+    got = []
+    for prms in (P, Q):
+        part = im.Partition(0, 0, precision)
+        part.allocate(h.shape[1], prms.GridXTotal)
+        part.update_constants(prms)
+        part.transfer_points_from_soa_to_device(h, 0, n)
+        part.sort_points()
+        got.append((part.tile_config(), part.nPts_partition))
+        part.close()
+    assert got[0] == got[1] and got[0][1] < n
