@@ -323,7 +323,7 @@ int Engine::push_scenes()
         dev[i].tile_off = (int)tiles;
         tiles += (long long)dev[i].n_tiles_x * dev[i].n_tiles_y;
     }
-    for (int k = n_ind; k < nscenes(); k++) dev[k].ind_scene = -1;
+    dev[0].n_ind = n_ind;
     // Workgroups of the substep launches for the indenter forces: one per scene
     // with an indenter (in contact or not: most of a scene's part is the load of
     // its constants), as many as there are compute units.  With fewer each walks

@@ -97,10 +97,10 @@ struct SceneDev {
     long long seg_off;      // first segment flag of the scene in each half of StepArgs::dirty
     // grain-dependent terms of the FP64 failure surface (scene_fail_table)
     double fail_tab[kFailTab];
-    // Entry k of the table also names the k-th scene with an indenter (-1: there
-    // are no more), for the workgroups that sum the indenter forces.
+    // For the workgroups that sum the indenter forces: entry k of the table also
+    // names the k-th scene with an indenter, and entry 0 says how many there are.
     int ind_scene;
-    int pad;
+    int n_ind;
 };
 
 // Device clock of a scene, advanced on the device once per substep so that a

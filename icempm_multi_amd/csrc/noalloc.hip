@@ -48,7 +48,7 @@ constexpr size_t kScratchBytes = kOffForce + align256(2 * (size_t)kMaxIndenterSu
 }  // namespace
 
 // The scratch memory of icempm_substeps_noalloc, one copy per GPU, held until
-// the process ends (about 24.2 MiB).  In host code `scratch` names a host-side
+// the process ends (about 24.6 MiB).  In host code `scratch` names a host-side
 // stand-in: only the address hipGetSymbolAddress returns for a device is used.
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
@@ -202,7 +202,8 @@ int icempm_substeps_noalloc(int device, const icempm_simparams *prms, size_t prm
     d.ncells = (int)nodes;
     d.force_off = 0;
     d.seg_off = 0;
-    d.ind_scene = d.c.ind_rsq > 0 ? 0 : -1;
+    d.ind_scene = 0;
+    d.n_ind = d.c.ind_rsq > 0 ? 1 : 0;
     SceneClock ck{};
     ck.t = P.SimulationTime;
     ck.ind_x = P.indenter_x;
