@@ -156,8 +156,6 @@ private:
     int choose_tile_shape();
     StepArgs args() const;
     StepArgs scene_runs(int scene, int &n_runs) const;
-    // timed: record hipEvents around the launches of every sample-th substep
-    int launch_substeps(int nsub, int start_buf, bool fused, bool direct, bool timed, int sample = 1);
     struct GraphExec;
     // n units of one kind from grid buffer b and clock slot cs; unit j is timed
     // when timed and (k0 + j) % sample == 0.  With span, the n units of a chain
@@ -171,7 +169,6 @@ private:
     int zero_grid(int scene, int buf);
     int start_buffer(bool fused, bool direct, int &b);
     void mark_buffers(bool fused, bool direct, int b, int nsub);
-    int record(int cls, bool timed, hipError_t (*)(void *), void *);
     void timed_begin(bool timed);
     void timed_end(bool timed, int cls, int launches = 1);
     int phase_begin(StepArgs &a, int n_blocks);

@@ -561,12 +561,13 @@ int Engine::alloc_tiles()
 {
     const long long mt = count_tiles(tx_, ty_);
     // The kernels loop over their workgroup's tiles, and a launch of exactly
-    // the workgroups the GPU holds at once (one generation) is the fastest:
-    // with more, the later generations start behind the first and the launch
-    // ends on a tail of partly busy CUs (4M-point sheet, substep launch: FP64
-    // 139.7 us with 8 workgroups per CU, 133.5 us with 2, its residency; mixed
-    // 106.0 us with 8, 103.6 us with 4, its residency, 133 us with 2).  The
-    // other launches take the substep launch's count: the tiles are split for it.
+    // the workgroups the GPU holds at once (one generation) leaves no later
+    // generation to start behind the first and end on a tail of partly busy
+    // CUs (4.0M points, substep launch at 16x32 cells: FP64 120.7 us with 3
+    // workgroups per CU, its residency, 132.0 with 4, 123.4 with 8, 137 with 2;
+    // mixed 88.0 us with 4, its residency, 93.8 with 3, 118 with 2; 85.9 with 8).
+    // The other launches take the substep launch's count: the tiles are split
+    // for it (in FP64 all have the same residency).
     few_ = false;   // until the next build
     int r = LAUNCH_PREC(tiles_resident_per_cu, args(), kTileChain);
     if (r <= 0) r = 8;   // the runtime could not tell: several generations
@@ -1401,25 +1402,6 @@ void Engine::mark_buffers(bool fused, bool direct, int b, int nsub)
             for (int k = 0; k < kGridBuffers; k++) s.clean[k] = k != last;
         }
     }
-}
-
-// The units of a call of nsub substeps (see emit_units), without graphs.
-int Engine::launch_substeps(int nsub, int start_buf, bool fused, bool direct, bool timed, int sample)
-{
-    std::vector<GraphExec *> none;
-    const int tmode = timed ? (sample > 1 ? 2 : 1) : 0;
-    int b = start_buf, cs = clock_slot_;
-    if (direct) {
-        RC(run_units(kUnitDirect, nsub, b, cs, false, tmode, 0, none));
-    } else if (!fused) {
-        RC(run_units(kUnitUnfused, nsub, b, cs, false, tmode, 0, none));
-    } else {
-        RC(run_units(kUnitHead, 1, b, cs, false, tmode, 0, none));
-        RC(run_units(kUnitChain, nsub - 1, b, cs, false, tmode, 0, none));
-        RC(run_units(kUnitTail, 1, b, cs, false, tmode, nsub - 1, none));
-    }
-    clock_slot_ = cs;
-    return ICEMPM_OK;
 }
 
 int Engine::step(int nsub, int flags)
