@@ -82,7 +82,7 @@ constexpr int kWaves = 3, kWavesFew = 2;
 // ---------------------------------------------------------------------------
 // Binned tile kernel: G2P from grid[rbuf] and/or P2G into grid[wbuf].
 // 3 waves per SIMD (up to 168 VGPRs; the fused kernel spills 7 outside the
-// point loop), or 2 (182 VGPRs, none) for launches of few workgroups.
+// point loop), or 2 (181 VGPRs, none) for launches of few workgroups.
 // What keeps it there: the scene invariants of the point loop (4/h, kappa/2,
 // sqrt(2) mu, the failure-surface and tension-branch terms) come from the host
 // in scalar registers, and the water stress uses J^-5 = 1/(J^2 J^2 J) rather

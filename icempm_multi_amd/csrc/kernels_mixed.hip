@@ -61,7 +61,7 @@ __device__ __forceinline__ void deferred_point(const StepArgs &a, bool p2g, int 
 }
 
 // Waves per SIMD the tile kernel is built for; the second for launches whose
-// tiles all run at once with its 154 VGPRs, three per SIMD (StepArgs::few): 102k
+// tiles all run at once with its 158 VGPRs, three per SIMD (StepArgs::few): 102k
 // points 8.9 us per substep, 9.5 with four.
 constexpr int kWaves = 4, kWavesFew = 2;
 
